@@ -2,13 +2,20 @@
 // for all canonical basis functions at once, written directly in the
 // pair-block layout.
 //
+// Two nodes are opposite corners of a box of grid nodes; the box's four diagonals
+// share midpoint and distance, hence the sphere and its integrals S_l, the costly
+// part.  Every box is integrated once, for its main diagonal (the pair whose xi has
+// the lower coordinate in every dimension), and serves its up to four pairs.
+//
 // Pipeline (cp = ordered cell pair X <= Y in the reference's cell order):
 //   1. k_count   : per cp, pairs (xi in X, xi1 in Y, xi < xi1) passing the
-//                  prefilter of lines 493-530                          -> cnt[cp]
-//   2. host scan -> offsets; k_list writes the flat list of (cp, p, q)
-//   3. k_integrate: one thread per pair, the D values of A (dgv_agen_math.h),
-//                  min_sens test, weights and |g|/8                      -> pairs
-//   4. k_keep_scan + k_compact: drop pairs whose D values are all zero and
+//                  prefilter of lines 493-530, and main diagonals among them
+//   2. host scan -> offsets; k_list writes the list of main diagonals, the pairs'
+//                  (p, q) and each cp's table (p, q) -> pair
+//   3. k_integrate: one thread per main diagonal, S_l (dgv_agen_math.h), then for
+//                  each pair of the box the D values of A: min_sens test, weights
+//                  and |g|/8                                             -> pairs
+//   4. k_kept + host scan + k_compact: drop pairs whose D values are all zero and
 //                  emit per-cp segment tables (the block headers)
 #include <algorithm>
 #include <array>
@@ -91,130 +98,220 @@ static int pair_raw_host(const AgenConsts& C, const double x[3], const double y[
 struct NodeGeo {
   const double *u, *v, *w, *gwts;
 };
+struct CellDims {
+  int Mv, Mw;
+  int64_t nc;
+};
 
-__device__ __forceinline__ bool prefilter_dev(const AgenConsts& C, const double* x, const double* y) {
-  const double d0 = x[0] - y[0], d1 = x[1] - y[1], d2 = x[2] - y[2];
-  const double dsph = sqrt(d0 * d0 + d1 * d1 + d2 * d2);
-  const double s0 = x[0] + y[0] - C.u0 - C.u1, s1 = x[1] + y[1] - C.v0 - C.v1, s2 = x[2] + y[2] - C.w0 - C.w1;
-  const double dist2 = sqrt(s0 * s0 + s1 * s1 + s2 * s2);
-  const double e0 = C.u1 - C.u0, e1 = C.v1 - C.v0, e2 = C.w1 - C.w0;
-  const double dphi = sqrt(e0 * e0 + e1 * e1 + e2 * e2);
-  return !((dist2 > dsph + dphi) || (dist2 + dphi < dsph) || (dsph > C.Trad));
-}
-
-template <int D>
-__global__ void k_count(AgenConsts C, int64_t ncp, const int2* __restrict__ cps, NodeGeo G,
-                        uint32_t* __restrict__ cnt) {
-  const int64_t cp = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (cp >= ncp) return;
-  const int2 XY = cps[cp];
-  uint32_t n = 0;
-  for (int p = 0; p < D; ++p) {
-    const int64_t i = (int64_t)XY.x * D + p;
-    const double x[3] = {G.u[i], G.v[i], G.w[i]};
-    for (int q = (XY.x == XY.y ? p + 1 : 0); q < D; ++q) {
-      const int64_t j = (int64_t)XY.y * D + q;
-      const double y[3] = {G.u[j], G.v[j], G.w[j]};
-      n += prefilter_dev(C, x, y) ? 1u : 0u;
-    }
-  }
-  cnt[cp] = n;
-}
-
-template <int D>
-__global__ void k_list(AgenConsts C, int64_t ncp, const int2* __restrict__ cps, NodeGeo G,
-                       const int64_t* __restrict__ off, uint64_t* __restrict__ list) {
-  const int64_t cp = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (cp >= ncp) return;
-  const int2 XY = cps[cp];
-  int64_t o = off[cp];
-  for (int p = 0; p < D; ++p) {
-    const int64_t i = (int64_t)XY.x * D + p;
-    const double x[3] = {G.u[i], G.v[i], G.w[i]};
-    for (int q = (XY.x == XY.y ? p + 1 : 0); q < D; ++q) {
-      const int64_t j = (int64_t)XY.y * D + q;
-      const double y[3] = {G.u[j], G.v[j], G.w[j]};
-      if (prefilter_dev(C, x, y)) list[o++] = ((uint64_t)cp << 16) | ((uint64_t)p << 8) | (uint64_t)q;
-    }
-  }
-}
-
+// (xi, xi1) = nodes (X, p), (Y, q): whether xi has the lower coordinate, or the same,
+// in every dimension
 template <int SU, int SV, int SW>
-__global__ __launch_bounds__(128) void k_integrate(AgenConsts C, int64_t npairs, const int2* __restrict__ cps,
-                                                   NodeGeo G, const uint64_t* __restrict__ list, double min_sens,
-                                                   double* __restrict__ pairs, uint8_t* __restrict__ keep) {
+__device__ __forceinline__ bool main_diagonal(const CellDims& d, int2 XY, int p, int q) {
+  const int xc[3] = {XY.x / (d.Mv * d.Mw), XY.x / d.Mw % d.Mv, XY.x % d.Mw};
+  const int yc[3] = {XY.y / (d.Mv * d.Mw), XY.y / d.Mw % d.Mv, XY.y % d.Mw};
+  const int xl[3] = {p / (SV * SW), p / SW % SV, p % SW}, yl[3] = {q / (SV * SW), q / SW % SV, q % SW};
+  bool ok = true;
+  for (int k = 0; k < 3; ++k) ok = ok && (xc[k] < yc[k] || (xc[k] == yc[k] && xl[k] <= yl[k]));
+  return ok;
+}
+
+// Candidate c of a cell pair: the nodes p = c / D, q = c % D
+template <int D>
+__device__ __forceinline__ bool candidate(const AgenConsts& C, int2 XY, int c, const NodeGeo& G) {
+  const int p = c / D, q = c - p * D;
+  if (c >= D * D || (XY.x == XY.y && q <= p)) return false;
+  const int64_t i = (int64_t)XY.x * D + p, j = (int64_t)XY.y * D + q;
+  const double x[3] = {G.u[i], G.v[i], G.w[i]}, y[3] = {G.u[j], G.v[j], G.w[j]};
+  return pair_distance(C, x, y) >= 0.0;
+}
+
+// One wave per cp: cnt = its pairs and its main diagonals
+template <int SU, int SV, int SW>
+__global__ __launch_bounds__(64) void k_count(AgenConsts C, CellDims dims, const int2* __restrict__ cps, NodeGeo G,
+                                              uint2* __restrict__ cnt) {
+  constexpr int D = SU * SV * SW;
+  const int64_t cp = blockIdx.x;
+  const int2 XY = cps[cp];
+  uint32_t n = 0, m = 0;
+  for (int c0 = 0; c0 < D * D; c0 += 64) {
+    const int c = c0 + (int)threadIdx.x;
+    const bool ok = candidate<D>(C, XY, c, G);
+    const bool main = ok && main_diagonal<SU, SV, SW>(dims, XY, c / D, c % D);
+    n += __popcll(__ballot(ok));
+    m += __popcll(__ballot(main));
+  }
+  if (threadIdx.x == 0) cnt[cp] = make_uint2(n, m);
+}
+
+// ... the pairs' codes p << 8 | q in (p, q) order, each candidate's rank among them
+// (-1: no pair) and the main diagonals
+template <int SU, int SV, int SW>
+__global__ __launch_bounds__(64) void k_list(AgenConsts C, CellDims dims, const int2* __restrict__ cps, NodeGeo G,
+                                             const int64_t* __restrict__ off, const int64_t* __restrict__ moff,
+                                             uint16_t* __restrict__ code, int16_t* __restrict__ rank,
+                                             uint64_t* __restrict__ mains) {
+  constexpr int D = SU * SV * SW;
+  const int64_t cp = blockIdx.x;
+  const int2 XY = cps[cp];
+  const int lane = threadIdx.x;
+  const uint64_t below = ((uint64_t)1 << lane) - 1;
+  int n = 0;
+  int64_t m = moff[cp];
+  const int64_t o = off[cp];
+  for (int c0 = 0; c0 < D * D; c0 += 64) {
+    const int c = c0 + lane;
+    const bool ok = candidate<D>(C, XY, c, G);
+    const bool main = ok && main_diagonal<SU, SV, SW>(dims, XY, c / D, c % D);
+    const uint64_t bo = __ballot(ok), bm = __ballot(main);
+    const int r = n + __popcll(bo & below);
+    if (c < D * D) rank[cp * (D * D) + c] = ok ? (int16_t)r : (int16_t)-1;
+    if (ok) code[o + r] = (uint16_t)((c / D) << 8 | c % D);
+    if (main) mains[m + __popcll(bm & below)] = ((uint64_t)cp << 16) | ((uint64_t)(c / D) << 8) | (uint64_t)(c % D);
+    n += __popcll(bo);
+    m += __popcll(bm);
+  }
+}
+
+// One thread per main diagonal.  FP64 transcendental arithmetic bounds it (up to 19
+// smooth pieces of 24 points, each with up to eight arc ends): 85 ms at 15^3 nodes
+// (3.2 M pairs) with one integration per pair, 26 ms with one per box.
+template <int SU, int SV, int SW>
+__global__ __launch_bounds__(128) void k_integrate(AgenConsts C, CellDims dims, int64_t nmain,
+                                                   const int2* __restrict__ cps, NodeGeo G,
+                                                   const uint64_t* __restrict__ mains,
+                                                   const int64_t* __restrict__ off, const int16_t* __restrict__ rank,
+                                                   double min_sens, double* __restrict__ pairs,
+                                                   uint8_t* __restrict__ keep) {
   constexpr int D = SU * SV * SW;
   const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= npairs) return;
-  const uint64_t e = list[k];
-  const int64_t cp = (int64_t)(e >> 16);
+  if (k >= nmain) return;
+  const uint64_t e = mains[k];
   const int p = (int)((e >> 8) & 255), q = (int)(e & 255);
-  const int2 XY = cps[cp];
-  const int64_t i = (int64_t)XY.x * D + p, j = (int64_t)XY.y * D + q;
-  const double x[3] = {G.u[i], G.v[i], G.w[i]};
-  const double y[3] = {G.u[j], G.v[j], G.w[j]};
-  double raw[D];
-  double dsph;
-  pair_raw<SU, SV, SW>(C, x, y, raw, &dsph);
-  const double wi = G.gwts[i], wj = G.gwts[j];
-  double* out = pairs + k * (D + 1);
-  bool any = false;
-  for (int l = 0; l < D; ++l) {
-    double a = 0.0;
-    if (fabs(raw[l]) > min_sens) {  // line 641, then lines 654-659
-      a = raw[l] * wj;
-      a = a * wi;
-      a = a * (dsph / 8.0);
-      any = true;
+  const int2 XY = cps[e >> 16];
+  const int64_t i0 = (int64_t)XY.x * D + p, j0 = (int64_t)XY.y * D + q;
+  const double lo[3] = {G.u[i0], G.v[i0], G.w[i0]}, hi[3] = {G.u[j0], G.v[j0], G.w[j0]};
+  const double dsph = pair_distance(C, lo, hi);
+  double S[D];
+  if (C.moment_mode == 0) {
+    const double cen[3] = {0.5 * (lo[0] + hi[0]), 0.5 * (lo[1] + hi[1]), 0.5 * (lo[2] + hi[2])};
+    sphere_integrals<SU, SV, SW>(C, cen, 0.5 * dsph, S);
+  }
+  // the box's corners: cell and local coordinates of the low and the high one
+  const int lc[3] = {XY.x / (dims.Mv * dims.Mw), XY.x / dims.Mw % dims.Mv, XY.x % dims.Mw};
+  const int hc[3] = {XY.y / (dims.Mv * dims.Mw), XY.y / dims.Mw % dims.Mv, XY.y % dims.Mw};
+  const int ll[3] = {p / (SV * SW), p / SW % SV, p % SW}, hl[3] = {q / (SV * SW), q / SW % SV, q % SW};
+  int differ = 0;
+  for (int d = 0; d < 3; ++d) differ |= (lc[d] != hc[d] || ll[d] != hl[d]) << d;
+  const int flips = differ & (differ - 1);   // the first dimension that differs stays: each diagonal once
+  for (int z = 0; z < 8; ++z) {
+    if (z & ~flips) continue;
+    int ac[3], al[3], bc[3], bl[3];   // the diagonal's ends: `a` takes the high corner where bit d of z is set
+    for (int d = 0; d < 3; ++d) {
+      const bool f = (z >> d) & 1;
+      ac[d] = f ? hc[d] : lc[d]; al[d] = f ? hl[d] : ll[d];
+      bc[d] = f ? lc[d] : hc[d]; bl[d] = f ? ll[d] : hl[d];
     }
-    out[l] = a;
+    int X = (ac[0] * dims.Mv + ac[1]) * dims.Mw + ac[2], Y = (bc[0] * dims.Mv + bc[1]) * dims.Mw + bc[2];
+    int P = (al[0] * SV + al[1]) * SW + al[2], Q = (bl[0] * SV + bl[1]) * SW + bl[2];
+    if (X > Y || (X == Y && P > Q)) {   // xi < xi1 in node order
+      const int t = X, u = P;
+      X = Y; Y = t;
+      P = Q; Q = u;
+    }
+    const int64_t cp = (int64_t)X * dims.nc - (int64_t)X * (X - 1) / 2 + (Y - X);
+    const int64_t at = off[cp] + rank[cp * (D * D) + P * D + Q];
+    const int64_t i = (int64_t)X * D + P, j = (int64_t)Y * D + Q;
+    const double x[3] = {G.u[i], G.v[i], G.w[i]}, y[3] = {G.u[j], G.v[j], G.w[j]};
+    double raw[D];
+    if (C.moment_mode == 0) {
+      raw_from_sphere<SU, SV, SW>(C, x, y, S, raw);
+    } else {
+      const double v = raw_moment(C.moment_mode, x, y, 0.5 * dsph);
+      for (int l = 0; l < D; ++l) raw[l] = v;
+    }
+    const double wi = G.gwts[i], wj = G.gwts[j];
+    double* out = pairs + at * (D + 1);
+    bool any = false;
+    for (int l = 0; l < D; ++l) {
+      double a = 0.0;
+      if (fabs(raw[l]) > min_sens) {  // line 641, then lines 654-659
+        a = raw[l] * wj;
+        a = a * wi;
+        a = a * (dsph / 8.0);
+        any = true;
+      }
+      out[l] = a;
+    }
+    out[D] = __longlong_as_double((long long)pair_code_bits(P, Q));
+    keep[at] = any ? 1 : 0;
   }
-  out[D] = __longlong_as_double((long long)pair_code_bits(p, q));
-  keep[k] = any ? 1 : 0;
 }
 
-// Per cp: number of kept pairs and, for each p, the first kept pair with local
-// index of xi >= p.
+// One wave per cp: its kept pairs and, for each p, the first kept pair with local
+// index of xi >= p
 template <int D>
-__global__ void k_segments(int64_t ncp, const int64_t* __restrict__ off, const uint64_t* __restrict__ list,
-                           const uint8_t* __restrict__ keep, int32_t* __restrict__ kcnt, uint16_t* __restrict__ seg) {
-  const int64_t cp = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (cp >= ncp) return;
-  uint16_t* s = seg + cp * (D + 1);
-  int n = 0, p_next = 0;
-  for (int64_t k = off[cp]; k < off[cp + 1]; ++k) {
-    if (!keep[k]) continue;
-    const int p = (int)((list[k] >> 8) & 255);
-    while (p_next <= p) s[p_next++] = (uint16_t)n;
-    ++n;
-  }
-  while (p_next <= D) s[p_next++] = (uint16_t)n;
-  kcnt[cp] = n;
-}
-
-template <int D>
-__global__ void k_compact(int64_t npairs, const uint8_t* __restrict__ keep, const int64_t* __restrict__ dst,
-                          const double* __restrict__ src, double* __restrict__ out) {
-  const int64_t step = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < npairs; k += step) {
-    if (!keep[k]) continue;
-    const double* a = src + k * (D + 1);
-    double* b = out + dst[k] * (D + 1);
-    for (int l = 0; l <= D; ++l) b[l] = a[l];
-  }
-}
-
-// per-basis record counts (integer atomics: exact and order independent)
-template <int D>
-__global__ void k_count_basis(int64_t npairs, const double* __restrict__ pairs, unsigned long long* __restrict__ cnt) {
-  __shared__ unsigned long long loc[D];
-  for (int l = threadIdx.x; l < D; l += blockDim.x) loc[l] = 0;
+__global__ __launch_bounds__(64) void k_kept(const int64_t* __restrict__ off, const uint16_t* __restrict__ code,
+                                             const uint8_t* __restrict__ keep, int32_t* __restrict__ kcnt,
+                                             uint16_t* __restrict__ seg) {
+  __shared__ int per[D];
+  const int64_t cp = blockIdx.x;
+  if (threadIdx.x < D) per[threadIdx.x] = 0;
   __syncthreads();
-  for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < npairs; k += (int64_t)gridDim.x * blockDim.x)
-    for (int l = 0; l < D; ++l)
-      if (pairs[k * (D + 1) + l] != 0.0) atomicAdd(&loc[l], 1ull);
+  for (int64_t k = off[cp] + threadIdx.x; k < off[cp + 1]; k += 64)
+    if (keep[k]) atomicAdd(&per[code[k] >> 8], 1);
   __syncthreads();
-  for (int l = threadIdx.x; l < D; l += blockDim.x) atomicAdd(&cnt[l], loc[l]);
+  if (threadIdx.x == 0) {
+    uint16_t* s = seg + cp * (D + 1);
+    int n = 0;
+    for (int p = 0; p < D; ++p) {
+      s[p] = (uint16_t)n;
+      n += per[p];
+    }
+    s[D] = (uint16_t)n;
+    kcnt[cp] = n;
+  }
+}
+
+// The kept pairs of each cp to their place, a workgroup per cp in turn, and the
+// records per basis function (integer sums: exact whatever the order)
+template <int D>
+__global__ __launch_bounds__(256) void k_compact(int64_t ncp, const int64_t* __restrict__ off,
+                                                 const int64_t* __restrict__ koff, const uint8_t* __restrict__ keep,
+                                                 const double* __restrict__ src, double* __restrict__ out,
+                                                 unsigned long long* __restrict__ cnt) {
+  __shared__ int16_t from[D * D];
+  __shared__ uint32_t nz[D];
+  __shared__ int base[5];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (threadIdx.x < D) nz[threadIdx.x] = 0;
+  for (int64_t cp = blockIdx.x; cp < ncp; cp += gridDim.x) {
+    const int64_t b = off[cp];
+    const int n = (int)(off[cp + 1] - b), nk = (int)(koff[cp + 1] - koff[cp]);
+    if (nk == 0) continue;
+    int before = 0;
+    for (int k0 = 0; k0 < n; k0 += 256) {
+      const int k = k0 + (int)threadIdx.x;
+      const bool ok = k < n && keep[b + k];
+      const uint64_t m = __ballot(ok);
+      __syncthreads();   // the last round's `base` is read
+      if (lane == 0) base[wave + 1] = __popcll(m);
+      __syncthreads();
+      int at = before;
+      for (int w = 0; w < wave; ++w) at += base[w + 1];
+      if (ok) from[at + __popcll(m & (((uint64_t)1 << lane) - 1))] = (int16_t)k;
+      for (int w = 0; w < 4; ++w) before += base[w + 1];
+    }
+    __syncthreads();
+    double* o = out + koff[cp] * (D + 1);
+    for (int i = threadIdx.x; i < nk * (D + 1); i += 256) {
+      const int r = i / (D + 1), l = i - r * (D + 1);
+      const double a = src[(b + from[r]) * (D + 1) + l];
+      o[i] = a;
+      if (l < D && a != 0.0) atomicAdd(&nz[l], 1u);
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x < D) atomicAdd(&cnt[threadIdx.x], (unsigned long long)nz[threadIdx.x]);
 }
 
 template <int SU, int SV, int SW>
@@ -229,19 +326,20 @@ static int generate_t(dgv_ctx* ctx, const AgenConsts& C, double min_sens) {
     for (int64_t Y = X; Y < nc; ++Y) cps.push_back(make_int2((int)X, (int)Y));
   const int64_t ncp = (int64_t)cps.size();
   int2* d_cps = nullptr;
-  uint32_t* d_cnt = nullptr;
-  int64_t* d_off = nullptr;
-  uint64_t* d_list = nullptr;
+  uint2* d_cnt = nullptr;
+  int64_t *d_off = nullptr, *d_moff = nullptr;
+  uint16_t* d_code = nullptr;
+  int16_t* d_rank = nullptr;
+  uint64_t* d_mains = nullptr;
   double *d_raw = nullptr, *d_pairs = nullptr;
   uint8_t* d_keep = nullptr;
-  int64_t* d_dst = nullptr;
   int32_t* d_kcnt = nullptr;
   uint16_t* d_seg = nullptr;
   unsigned long long* d_bcnt = nullptr;
   int rc = DGV_OK;
   auto cleanup = [&]() {
-    hipFree(d_cps); hipFree(d_cnt); hipFree(d_off); hipFree(d_list); hipFree(d_raw); hipFree(d_keep);
-    hipFree(d_dst); hipFree(d_kcnt); hipFree(d_seg); hipFree(d_bcnt);
+    hipFree(d_cps); hipFree(d_cnt); hipFree(d_off); hipFree(d_moff); hipFree(d_code); hipFree(d_rank);
+    hipFree(d_mains); hipFree(d_raw); hipFree(d_keep); hipFree(d_kcnt); hipFree(d_seg); hipFree(d_bcnt);
   };
 #define AG_HIP(call)                                                                           \
   do {                                                                                         \
@@ -253,66 +351,69 @@ static int generate_t(dgv_ctx* ctx, const AgenConsts& C, double min_sens) {
                        std::string("A-array generator: ") + #call + ": " + hipGetErrorString(e_)); \
     }                                                                                          \
   } while (0)
-  NodeGeo G{ctx->d_u, ctx->d_v, ctx->d_w, ctx->d_gwts};
+  const NodeGeo G{ctx->d_u, ctx->d_v, ctx->d_w, ctx->d_gwts};
+  const CellDims dims{g.Mv, g.Mw, nc};
   hipStream_t st = ctx->stream;
+  if (ncp >= (int64_t)1 << 31) return set_error(ctx, DGV_ERR_UNSUPPORTED, "A-array generator: too many cell pairs");
   AG_HIP(hipMalloc(&d_cps, sizeof(int2) * ncp));
-  AG_HIP(hipMemcpy(d_cps, cps.data(), sizeof(int2) * ncp, hipMemcpyHostToDevice));
-  AG_HIP(hipMalloc(&d_cnt, sizeof(uint32_t) * ncp));
-  const unsigned gcp = (unsigned)((ncp + 127) / 128);
-  hipLaunchKernelGGL(k_count<D>, dim3(gcp), dim3(128), 0, st, C, ncp, d_cps, G, d_cnt);
+  AG_HIP(hipMemcpyAsync(d_cps, cps.data(), sizeof(int2) * ncp, hipMemcpyHostToDevice, st));
+  AG_HIP(hipMalloc(&d_cnt, sizeof(uint2) * ncp));
+  hipLaunchKernelGGL((k_count<SU, SV, SW>), dim3((unsigned)ncp), dim3(64), 0, st, C, dims, d_cps, G, d_cnt);
   AG_HIP(hipGetLastError());
-  std::vector<uint32_t> cnt(ncp);
-  AG_HIP(hipMemcpyAsync(cnt.data(), d_cnt, sizeof(uint32_t) * ncp, hipMemcpyDeviceToHost, st));
+  std::vector<uint2> cnt(ncp);
+  AG_HIP(hipMemcpyAsync(cnt.data(), d_cnt, sizeof(uint2) * ncp, hipMemcpyDeviceToHost, st));
   AG_HIP(hipStreamSynchronize(st));
-  std::vector<int64_t> off(ncp + 1, 0);
-  for (int64_t i = 0; i < ncp; ++i) off[i + 1] = off[i] + cnt[i];
-  const int64_t np = off[ncp];
+  std::vector<int64_t> off(ncp + 1, 0), moff(ncp + 1, 0);
+  for (int64_t i = 0; i < ncp; ++i) {
+    off[i + 1] = off[i] + cnt[i].x;
+    moff[i + 1] = moff[i] + cnt[i].y;
+  }
+  const int64_t np = off[ncp], nmain = moff[ncp];
   AG_HIP(hipMalloc(&d_off, sizeof(int64_t) * (ncp + 1)));
-  AG_HIP(hipMemcpy(d_off, off.data(), sizeof(int64_t) * (ncp + 1), hipMemcpyHostToDevice));
-  AG_HIP(hipMalloc(&d_list, sizeof(uint64_t) * std::max<int64_t>(np, 1)));
-  hipLaunchKernelGGL(k_list<D>, dim3(gcp), dim3(128), 0, st, C, ncp, d_cps, G, d_off, d_list);
+  AG_HIP(hipMalloc(&d_moff, sizeof(int64_t) * (ncp + 1)));
+  AG_HIP(hipMemcpyAsync(d_off, off.data(), sizeof(int64_t) * (ncp + 1), hipMemcpyHostToDevice, st));
+  AG_HIP(hipMemcpyAsync(d_moff, moff.data(), sizeof(int64_t) * (ncp + 1), hipMemcpyHostToDevice, st));
+  AG_HIP(hipMalloc(&d_code, sizeof(uint16_t) * std::max<int64_t>(np, 1)));
+  AG_HIP(hipMalloc(&d_rank, sizeof(int16_t) * D * D * ncp));
+  AG_HIP(hipMalloc(&d_mains, sizeof(uint64_t) * std::max<int64_t>(nmain, 1)));
+  hipLaunchKernelGGL((k_list<SU, SV, SW>), dim3((unsigned)ncp), dim3(64), 0, st, C, dims, d_cps, G, d_off, d_moff,
+                     d_code, d_rank, d_mains);
   AG_HIP(hipGetLastError());
   AG_HIP(hipMalloc(&d_raw, sizeof(double) * (D + 1) * std::max<int64_t>(np, 1)));
   AG_HIP(hipMalloc(&d_keep, std::max<int64_t>(np, 1)));
   // integrate in slices so that each launch stays short
   const int64_t slice = 1 << 22;
-  for (int64_t b = 0; b < np; b += slice) {
-    const int64_t n = std::min(slice, np - b);
+  for (int64_t b = 0; b < nmain; b += slice) {
+    const int64_t n = std::min(slice, nmain - b);
     k_integrate<SU, SV, SW><<<dim3((unsigned)((n + 127) / 128)), dim3(128), 0, st>>>(
-        C, n, d_cps, G, d_list + b, min_sens, d_raw + b * (D + 1), d_keep + b);
+        C, dims, n, d_cps, G, d_mains + b, d_off, d_rank, min_sens, d_raw, d_keep);
     AG_HIP(hipGetLastError());
   }
   // compaction
-  std::vector<uint8_t> keep(np);
-  AG_HIP(hipMemcpyAsync(keep.data(), d_keep, np, hipMemcpyDeviceToHost, st));
-  AG_HIP(hipStreamSynchronize(st));
-  std::vector<int64_t> dst(np);
-  int64_t nk = 0;
-  for (int64_t k = 0; k < np; ++k) { dst[k] = nk; nk += keep[k]; }
-  AG_HIP(hipMalloc(&d_dst, sizeof(int64_t) * std::max<int64_t>(np, 1)));
-  AG_HIP(hipMemcpy(d_dst, dst.data(), sizeof(int64_t) * np, hipMemcpyHostToDevice));
-  AG_HIP(hipMalloc(&d_pairs, sizeof(double) * (D + 1) * (nk + kPairPad)));
-  AG_HIP(hipMemsetAsync(d_pairs + (D + 1) * nk, 0, sizeof(double) * (D + 1) * kPairPad, st));
-  if (np > 0)
-    hipLaunchKernelGGL(k_compact<D>, dim3(stride_blocks(np, 256)), dim3(256), 0, st, np, d_keep, d_dst, d_raw,
-                       d_pairs);
   AG_HIP(hipMalloc(&d_kcnt, sizeof(int32_t) * ncp));
   AG_HIP(hipMalloc(&d_seg, sizeof(uint16_t) * (D + 1) * ncp));
-  hipLaunchKernelGGL(k_segments<D>, dim3(gcp), dim3(128), 0, st, ncp, d_off, d_list, d_keep, d_kcnt, d_seg);
   AG_HIP(hipMalloc(&d_bcnt, sizeof(unsigned long long) * D));
-  AG_HIP(hipMemsetAsync(d_bcnt, 0, sizeof(unsigned long long) * D, st));
-  if (nk > 0) hipLaunchKernelGGL(k_count_basis<D>, dim3(1024), dim3(256), 0, st, nk, d_pairs, d_bcnt);
+  hipLaunchKernelGGL(k_kept<D>, dim3((unsigned)ncp), dim3(64), 0, st, d_off, d_code, d_keep, d_kcnt, d_seg);
   AG_HIP(hipGetLastError());
   std::vector<int32_t> kcnt(ncp);
   std::vector<uint16_t> seg((size_t)ncp * (D + 1));
-  std::vector<unsigned long long> bcnt(D);
   AG_HIP(hipMemcpyAsync(kcnt.data(), d_kcnt, sizeof(int32_t) * ncp, hipMemcpyDeviceToHost, st));
   AG_HIP(hipMemcpyAsync(seg.data(), d_seg, sizeof(uint16_t) * (D + 1) * ncp, hipMemcpyDeviceToHost, st));
+  AG_HIP(hipStreamSynchronize(st));
+  std::vector<int64_t>& koff = moff;
+  for (int64_t i = 0; i < ncp; ++i) koff[i + 1] = koff[i] + kcnt[i];
+  const int64_t nk = koff[ncp];
+  AG_HIP(hipMemcpyAsync(d_moff, koff.data(), sizeof(int64_t) * (ncp + 1), hipMemcpyHostToDevice, st));
+  AG_HIP(hipMalloc(&d_pairs, sizeof(double) * (D + 1) * (nk + kPairPad)));
+  AG_HIP(hipMemsetAsync(d_pairs + (D + 1) * nk, 0, sizeof(double) * (D + 1) * kPairPad, st));
+  AG_HIP(hipMemsetAsync(d_bcnt, 0, sizeof(unsigned long long) * D, st));
+  hipLaunchKernelGGL(k_compact<D>, dim3((unsigned)std::min<int64_t>(ncp, 4096)), dim3(256), 0, st, ncp, d_off, d_moff,
+                     d_keep, d_raw, d_pairs, d_bcnt);
+  AG_HIP(hipGetLastError());
+  std::vector<unsigned long long> bcnt(D);
   AG_HIP(hipMemcpyAsync(bcnt.data(), d_bcnt, sizeof(unsigned long long) * D, hipMemcpyDeviceToHost, st));
   AG_HIP(hipStreamSynchronize(st));
   cleanup();
-  d_cps = nullptr; d_cnt = nullptr; d_off = nullptr; d_list = nullptr; d_raw = nullptr; d_keep = nullptr;
-  d_dst = nullptr; d_kcnt = nullptr; d_seg = nullptr; d_bcnt = nullptr;
   // blocks (one per cell pair with kept pairs) and groups
   free_plan(ctx);
   free_pairblock(ctx);

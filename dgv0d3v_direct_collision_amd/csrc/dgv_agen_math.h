@@ -246,48 +246,72 @@ DGV_HD inline void sphere_integrals(const AgenConsts& C, const double cen[3], do
   }
 }
 
-// Raw values Atemp_l (before min_sens and the weights) of one pair, or -1 if
-// the pair fails SetA_DGV's prefilter (dgvtools_mod.f90:527-530).
+// Raw values Atemp_l (before min_sens and the weights) of one pair from its sphere
+// integrals S_l: the gain 2 S_l less the loss 4 pi (phi_l(xi) + phi_l(xi1)).
 template <int SU, int SV, int SW>
-DGV_HD inline int pair_raw(const AgenConsts& C, const double x[3], const double y[3], double* raw, double* dsph_out) {
+DGV_HD inline void raw_from_sphere(const AgenConsts& C, const double x[3], const double y[3], const double* S,
+                                   double* raw) {
   const double fourpi = 12.566370614359172953850573533118;
+  for (int iu = 0; iu < SU; ++iu)
+    for (int iv = 0; iv < SV; ++iv)
+      for (int iw = 0; iw < SW; ++iw) {
+        const int l = (iu * SV + iv) * SW + iw;
+        const double loss = basis_at(C, iu, iv, iw, x[0], x[1], x[2]) + basis_at(C, iu, iv, iw, y[0], y[1], y[2]);
+        raw[l] = 2.0 * S[l] - fourpi * loss;
+      }
+}
+
+// The same for the moment test functions psi = 1,u,v,w,|u|^2 over the whole sphere
+// (dgvtools_mod.f90:267-274): closed forms of int psi(c + r k) dk; the value is
+// every basis function's.
+DGV_HD inline double raw_moment(int mode, const double x[3], const double y[3], double r) {
+  const double fourpi = 12.566370614359172953850573533118;
+  const double cen[3] = {0.5 * (x[0] + y[0]), 0.5 * (x[1] + y[1]), 0.5 * (x[2] + y[2])};
+  double S, px, py;
+  switch (mode) {
+    case 1: S = fourpi; px = 1.0; py = 1.0; break;
+    case 2: S = fourpi * cen[0]; px = x[0]; py = y[0]; break;
+    case 3: S = fourpi * cen[1]; px = x[1]; py = y[1]; break;
+    case 4: S = fourpi * cen[2]; px = x[2]; py = y[2]; break;
+    default:
+      S = fourpi * (cen[0] * cen[0] + cen[1] * cen[1] + cen[2] * cen[2] + r * r);
+      px = x[0] * x[0] + x[1] * x[1] + x[2] * x[2];
+      py = y[0] * y[0] + y[1] * y[1] + y[2] * y[2];
+      break;
+  }
+  return 2.0 * S - fourpi * (px + py);
+}
+
+// |xi - xi1| of a pair, or -1 if it fails SetA_DGV's prefilter
+// (dgvtools_mod.f90:527-530).  Exchanging one component of the two nodes changes
+// no bit of it, nor of the pair's midpoint.
+DGV_HD inline double pair_distance(const AgenConsts& C, const double x[3], const double y[3]) {
   const double d0 = x[0] - y[0], d1 = x[1] - y[1], d2 = x[2] - y[2];
   const double dsph = sqrt(d0 * d0 + d1 * d1 + d2 * d2);
   const double s0 = x[0] + y[0] - C.u0 - C.u1, s1 = x[1] + y[1] - C.v0 - C.v1, s2 = x[2] + y[2] - C.w0 - C.w1;
   const double dist2 = sqrt(s0 * s0 + s1 * s1 + s2 * s2);
   const double e0 = C.u1 - C.u0, e1 = C.v1 - C.v0, e2 = C.w1 - C.w0;
   const double dphi = sqrt(e0 * e0 + e1 * e1 + e2 * e2);
-  *dsph_out = dsph;
+  if ((dist2 > dsph + dphi) || (dist2 + dphi < dsph) || (dsph > C.Trad)) return -1.0;
+  return dsph;
+}
+
+// Raw values Atemp_l of one pair; -1 if the pair fails the prefilter.
+template <int SU, int SV, int SW>
+DGV_HD inline int pair_raw(const AgenConsts& C, const double x[3], const double y[3], double* raw, double* dsph_out) {
   constexpr int D = SU * SV * SW;
-  if ((dist2 > dsph + dphi) || (dist2 + dphi < dsph) || (dsph > C.Trad)) return -1;
-  const double cen[3] = {0.5 * (x[0] + y[0]), 0.5 * (x[1] + y[1]), 0.5 * (x[2] + y[2])};
-  const double r = 0.5 * dsph;
+  const double dsph = pair_distance(C, x, y);
+  *dsph_out = dsph;
+  if (dsph < 0.0) return -1;
   if (C.moment_mode != 0) {
-    // moment test functions psi = 1,u,v,w,|u|^2 over the whole sphere
-    // (dgvtools_mod.f90:267-274): closed forms of int psi(c + r k) dk
-    double S, px, py;
-    switch (C.moment_mode) {
-      case 1: S = fourpi; px = 1.0; py = 1.0; break;
-      case 2: S = fourpi * cen[0]; px = x[0]; py = y[0]; break;
-      case 3: S = fourpi * cen[1]; px = x[1]; py = y[1]; break;
-      case 4: S = fourpi * cen[2]; px = x[2]; py = y[2]; break;
-      default:
-        S = fourpi * (cen[0] * cen[0] + cen[1] * cen[1] + cen[2] * cen[2] + r * r);
-        px = x[0] * x[0] + x[1] * x[1] + x[2] * x[2];
-        py = y[0] * y[0] + y[1] * y[1] + y[2] * y[2];
-        break;
-    }
-    for (int l = 0; l < D; ++l) raw[l] = 2.0 * S - fourpi * (px + py);
+    const double v = raw_moment(C.moment_mode, x, y, 0.5 * dsph);
+    for (int l = 0; l < D; ++l) raw[l] = v;
     return 0;
   }
-  sphere_integrals<SU, SV, SW>(C, cen, r, raw);
-  for (int iu = 0; iu < SU; ++iu)
-    for (int iv = 0; iv < SV; ++iv)
-      for (int iw = 0; iw < SW; ++iw) {
-        const int l = (iu * SV + iv) * SW + iw;
-        const double loss = basis_at(C, iu, iv, iw, x[0], x[1], x[2]) + basis_at(C, iu, iv, iw, y[0], y[1], y[2]);
-        raw[l] = 2.0 * raw[l] - fourpi * loss;
-      }
+  const double cen[3] = {0.5 * (x[0] + y[0]), 0.5 * (x[1] + y[1]), 0.5 * (x[2] + y[2])};
+  double S[D];
+  sphere_integrals<SU, SV, SW>(C, cen, 0.5 * dsph, S);
+  raw_from_sphere<SU, SV, SW>(C, x, y, S, raw);
   return 0;
 }
 
