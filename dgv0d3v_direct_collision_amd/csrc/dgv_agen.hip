@@ -467,6 +467,8 @@ static int generate_t(dgv_ctx* ctx, const AgenConsts& C, double min_sens) {
   DGV_HIP(ctx, hipMalloc(&pb.d_groups, sizeof(Group) * std::max<size_t>(pb.groups.size(), 1)));
   DGV_HIP(ctx, hipMemcpy(pb.d_groups, pb.groups.data(), sizeof(Group) * pb.groups.size(), hipMemcpyHostToDevice));
   ctx->has_a = true;
+  rc = build_quads(ctx);
+  if (rc) return rc;
   rc = build_plan(ctx, ctx->tile);
 #undef AG_HIP
   return rc;

@@ -92,7 +92,8 @@ int dgv_ctx_create(const dgv_grid_desc* grid, int device, dgv_ctx** out) {
     if (hipEventCreate(&ctx->ev[i]) != hipSuccess) return fail(DGV_ERR_HIP, "hipEventCreate failed");
   const size_t nb = sizeof(double) * g.N;
   if (hipMalloc(&ctx->d_gwts, nb) || hipMalloc(&ctx->d_u, nb) || hipMalloc(&ctx->d_v, nb) ||
-      hipMalloc(&ctx->d_w, nb) || hipMalloc(&ctx->d_f, nb) || hipMalloc(&ctx->d_q, nb))
+      hipMalloc(&ctx->d_w, nb) || hipMalloc(&ctx->d_f, nb) || hipMalloc(&ctx->d_q, nb) ||
+      hipMalloc(&ctx->d_ft, 2 * nb))
     return fail(DGV_ERR_NOMEM, "hipMalloc failed");
   for (int i = 0; i < 6; ++i)
     if (hipMalloc(&ctx->d_tmp[i], nb)) return fail(DGV_ERR_NOMEM, "hipMalloc failed");
@@ -119,7 +120,7 @@ void dgv_ctx_destroy(dgv_ctx* ctx) {
   free_pairblock(ctx);
   free_linear_vectors(ctx);
   hipFree(ctx->d_gwts); hipFree(ctx->d_u); hipFree(ctx->d_v); hipFree(ctx->d_w);
-  hipFree(ctx->d_f); hipFree(ctx->d_q); hipFree(ctx->d_red); hipFree(ctx->d_hi);
+  hipFree(ctx->d_f); hipFree(ctx->d_q); hipFree(ctx->d_ft); hipFree(ctx->d_red); hipFree(ctx->d_hi);
   for (int i = 0; i < 6; ++i) hipFree(ctx->d_tmp[i]);
   for (int i = 0; i < 4; ++i)
     if (ctx->ev[i]) hipEventDestroy(ctx->ev[i]);
@@ -300,6 +301,8 @@ int dgv_ctx_set_kernel(dgv_ctx* ctx, int kernel) {
   if (kernel < DGV_KERNEL_AUTO || kernel > DGV_KERNEL_MFMA) return set_error(ctx, DGV_ERR_ARG, "unknown kernel");
   ctx->kernel = kernel;
   if (ctx->rk_graph) { hipGraphExecDestroy(ctx->rk_graph); ctx->rk_graph = nullptr; }
+  // the merged and the pair-block evaluators have their own work items
+  if (ctx->has_a && ctx->plan.quad != quad_wanted(ctx)) return build_plan(ctx, ctx->tile);
   return DGV_OK;
 }
 

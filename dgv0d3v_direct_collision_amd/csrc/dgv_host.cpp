@@ -144,6 +144,7 @@ void bump_aarray_generation(dgv_ctx* ctx) {
 void free_pairblock(dgv_ctx* ctx) {
   bump_aarray_generation(ctx);
   free_linear(ctx);
+  free_quads(ctx);
   PairBlock& pb = ctx->pb;
   hipFree(pb.d_pairs); hipFree(pb.d_blocks); hipFree(pb.d_group_blocks); hipFree(pb.d_groups);
   pb.d_pairs = nullptr; pb.d_blocks = nullptr; pb.d_group_blocks = nullptr; pb.d_groups = nullptr;
@@ -160,9 +161,8 @@ void free_pairblock(dgv_ctx* ctx) {
 
 void free_plan(dgv_ctx* ctx) {
   Plan& p = ctx->plan;
-  hipFree(p.d_items); hipFree(p.d_partial); hipFree(p.d_cell_ptr); hipFree(p.d_cell_rows);
-  p.d_items = nullptr; p.d_partial = nullptr; p.d_cell_ptr = nullptr; p.d_cell_rows = nullptr;
-  p.items.clear(); p.nrows = 0; p.ncell_rows = 0; p.pairs_per_item = 0;
+  hipFree(p.d_items); hipFree(p.d_qitems); hipFree(p.d_partial); hipFree(p.d_cell_ptr); hipFree(p.d_cell_rows);
+  p = Plan();
   if (ctx->rk_graph) { hipGraphExecDestroy(ctx->rk_graph); ctx->rk_graph = nullptr; }
 }
 
@@ -312,6 +312,7 @@ int upload_pairblock(dgv_ctx* ctx, std::vector<double>& pairs) {
   DGV_HIP(ctx, hipMalloc(&pb.d_groups, sizeof(Group) * std::max<size_t>(pb.groups.size(), 1)));
   DGV_HIP(ctx, hipMemcpy(pb.d_groups, pb.groups.data(), sizeof(Group) * pb.groups.size(), hipMemcpyHostToDevice));
   ctx->has_a = true;
+  if (int rc = build_quads(ctx)) return rc;
   return build_plan(ctx, ctx->tile);
 }
 
@@ -387,8 +388,8 @@ int build_pairblock_from_records(dgv_ctx* ctx, const int32_t* capphi, int64_t nc
 // order, which fixes the order of the final FP64 sum.
 int build_plan(dgv_ctx* ctx, int32_t ppi) {
   free_plan(ctx);
+  if (quad_wanted(ctx)) return build_quad_plan(ctx, ppi);
   const PairBlock& pb = ctx->pb;
-  const Grid& g = ctx->g;
   Plan& P = ctx->plan;
   if (ppi <= 0) ppi = 2048;
   P.pairs_per_item = ppi;
@@ -449,41 +450,48 @@ int build_plan(dgv_ctx* ctx, int32_t ppi) {
       P.items[pos].prow = (int64_t)pos * 64;
     }
   P.nrows = (int64_t)P.items.size() * 64;
-  // per-cell row lists
-  std::vector<int64_t> cnt(g.ncells + 1, 0);
+  std::vector<int64_t> row0;
+  std::vector<const Group*> grp;
+  std::vector<int32_t> cell0;
   for (const WorkItem& it : P.items) {
     if (it.chunk < 0) continue;
-    const Group& G = pb.groups[it.group];
-    const int n = std::min(64, G.ncells - it.chunk * 64);
-    for (int l = 0; l < n; ++l) {
-      int r = it.chunk * 64 + l;
-      const int cw = G.lo[2] + r % G.ext[2]; r /= G.ext[2];
-      const int cv = G.lo[1] + r % G.ext[1]; r /= G.ext[1];
-      const int cu = G.lo[0] + r;
-      cnt[((int64_t)cu * g.Mv + cv) * g.Mw + cw + 1]++;
-    }
+    row0.push_back(it.prow);
+    grp.push_back(&pb.groups[it.group]);
+    cell0.push_back(it.chunk * 64);
   }
-  for (int64_t c = 0; c < g.ncells; ++c) cnt[c + 1] += cnt[c];
-  std::vector<int32_t> rows(cnt[g.ncells]);
-  std::vector<int64_t> pos(cnt.begin(), cnt.end() - 1);
-  for (const WorkItem& it : P.items) {
-    if (it.chunk < 0) continue;
-    const Group& G = pb.groups[it.group];
-    const int n = std::min(64, G.ncells - it.chunk * 64);
-    for (int l = 0; l < n; ++l) {
-      int r = it.chunk * 64 + l;
-      const int cw = G.lo[2] + r % G.ext[2]; r /= G.ext[2];
-      const int cv = G.lo[1] + r % G.ext[1]; r /= G.ext[1];
-      const int cu = G.lo[0] + r;
-      const int64_t cell = ((int64_t)cu * g.Mv + cv) * g.Mw + cw;
-      if (it.prow + l > INT32_MAX) return set_error(ctx, DGV_ERR_UNSUPPORTED, "too many partial rows");
-      rows[pos[cell]++] = (int32_t)(it.prow + l);
-    }
-  }
-  P.ncell_rows = (int64_t)rows.size();
   DGV_HIP(ctx, hipSetDevice(ctx->device));
   DGV_HIP(ctx, hipMalloc(&P.d_items, sizeof(WorkItem) * std::max<size_t>(P.items.size(), 1)));
   DGV_HIP(ctx, hipMemcpy(P.d_items, P.items.data(), sizeof(WorkItem) * P.items.size(), hipMemcpyHostToDevice));
+  return plan_cell_rows(ctx, row0, grp, cell0, 64);
+}
+
+// The partial sums' buffer and the per-cell lists of the rows to add, in item
+// order: item k holds the cells cell0[k] .. cell0[k] + width - 1 of group grp[k]'s
+// box in the rows row0[k] ..
+int plan_cell_rows(dgv_ctx* ctx, const std::vector<int64_t>& row0, const std::vector<const Group*>& grp,
+                   const std::vector<int32_t>& cell0, int width) {
+  const Grid& g = ctx->g;
+  Plan& P = ctx->plan;
+  std::vector<int64_t> cnt(g.ncells + 1, 0);
+  auto for_cells = [&](size_t k, auto&& fn) {
+    const Group& G = *grp[k];
+    const int n = std::min(width, G.ncells - cell0[k]);
+    for (int l = 0; l < n; ++l) {
+      int r = cell0[k] + l;
+      const int cw = G.lo[2] + r % G.ext[2]; r /= G.ext[2];
+      const int cv = G.lo[1] + r % G.ext[1]; r /= G.ext[1];
+      const int cu = G.lo[0] + r;
+      fn(((int64_t)cu * g.Mv + cv) * g.Mw + cw, l);
+    }
+  };
+  for (size_t k = 0; k < row0.size(); ++k) for_cells(k, [&](int64_t c, int) { cnt[c + 1]++; });
+  for (int64_t c = 0; c < g.ncells; ++c) cnt[c + 1] += cnt[c];
+  std::vector<int32_t> rows(cnt[g.ncells]);
+  std::vector<int64_t> pos(cnt.begin(), cnt.end() - 1);
+  if (P.nrows > INT32_MAX) return set_error(ctx, DGV_ERR_UNSUPPORTED, "too many partial rows");
+  for (size_t k = 0; k < row0.size(); ++k)
+    for_cells(k, [&](int64_t c, int l) { rows[pos[c]++] = (int32_t)(row0[k] + l); });
+  P.ncell_rows = (int64_t)rows.size();
   if (hipMalloc(&P.d_partial, sizeof(double) * std::max<int64_t>(P.nrows * g.D, 1)) != hipSuccess)
     return set_error(ctx, DGV_ERR_NOMEM, "hipMalloc(partial sums) failed");
   DGV_HIP(ctx, hipMalloc(&P.d_cell_ptr, sizeof(int64_t) * (g.ncells + 1)));

@@ -137,16 +137,53 @@ struct PairBlock {
   std::vector<int64_t> nrec_basis;    // per canonical basis function
 };
 
+// Header of a block of the merged layout (dgv_quad.h): its first step, its steps,
+// the low and high corner cells (offsets from the canonical cell, a <= b) and
+// the dimensions in which they coincide (bit d).
+struct alignas(16) QuadBlk {
+  int64_t sbeg;
+  int32_t nst;
+  int8_t a[3], b[3];
+  uint8_t same;
+  uint8_t pad;
+  int32_t npairs;          // node pairs merged into the block
+};
+
+// Work item of the merged layout: nblk blocks from block `blk` of a group on (or,
+// with one block, its steps s0 .. s1 - 1) for 32 cells of the group's box.  The
+// group's box and the first block's header are copied in: one read starts an item.
+struct alignas(16) QuadItem {
+  int32_t group, chunk;    // chunk < 0: empty slot
+  int32_t blk, nblk, s0, s1;
+  int32_t lo[3], ext[3], ncells;
+  int64_t prow;            // first partial row (32 rows per item)
+  QuadBlk first;
+};
+
 // Work decomposition of one evaluation (depends on tile size).
 struct Plan {
   int32_t pairs_per_item = 0;
+  bool quad = false;                  // items of the merged layout
+  bool transpose = false;             // ... which read f transposed
   std::vector<WorkItem> items;
-  int64_t nrows = 0;                  // partial rows = 64 * items
+  std::vector<QuadItem> qitems;
+  int64_t nrows = 0;                  // partial rows: 64 (merged layout: 32) per item
   WorkItem* d_items = nullptr;
+  QuadItem* d_qitems = nullptr;
   double* d_partial = nullptr;        // nrows * D doubles (FP64 partial sums)
   int64_t* d_cell_ptr = nullptr;      // CSR over output cells of partial rows
   int32_t* d_cell_rows = nullptr;
   int64_t ncell_rows = 0;
+};
+
+// The merged layout of a context's A-array (dgv_quad.hip).
+struct QuadLayout {
+  bool use = false;                   // enough pairs merge for the merged evaluator
+  int64_t nquads = 0, nsteps = 0;
+  std::vector<QuadBlk> blocks;        // in group order
+  std::vector<Group> groups;          // bbeg, bend: ranges of `blocks`
+  double* d_steps = nullptr;
+  QuadBlk* d_blocks = nullptr;
 };
 
 struct FmaItem;
@@ -186,6 +223,7 @@ struct dgv_ctx {
   bool has_a = false;
   uint64_t a_gen = 0;
   dgv::PairBlock pb;
+  dgv::QuadLayout quad;
   dgv::Plan plan;
   int32_t tile = 0;          // pairs per work item (0 = default)
   int kernel = DGV_KERNEL_AUTO;
@@ -199,6 +237,7 @@ struct dgv_ctx {
   // scratch
   double* d_f = nullptr;
   double* d_q = nullptr;
+  double* d_ft = nullptr;         // two VDFs transposed, for the merged evaluator
   double* d_tmp[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
   double* d_red = nullptr;        // moment reduction scratch
   double* d_hi = nullptr;         // high-moment reduction scratch (on first use)
@@ -240,6 +279,15 @@ int build_pairblock_from_records(dgv_ctx* ctx, const int32_t* capphi, int64_t nc
                                  int64_t nrec, int index_base);
 int upload_pairblock(dgv_ctx* ctx, std::vector<double>& pairs);
 int build_plan(dgv_ctx* ctx, int32_t pairs_per_item);
+int plan_cell_rows(dgv_ctx* ctx, const std::vector<int64_t>& row0, const std::vector<const Group*>& grp,
+                   const std::vector<int32_t>& cell0, int width);
+// merged layout (dgv_quad.hip): built with every A-array; quad_wanted: the
+// evaluator that the context's kernel setting selects is the merged one
+int build_quads(dgv_ctx* ctx);
+void free_quads(dgv_ctx* ctx);
+int build_quad_plan(dgv_ctx* ctx, int32_t pairs_per_item);
+bool quad_wanted(const dgv_ctx* ctx);
+int launch_main_quad(dgv_ctx* ctx, const double* d_f, const double* d_g, double* partial);
 void free_pairblock(dgv_ctx* ctx);
 void free_plan(dgv_ctx* ctx);
 int ensure_record_layout(dgv_ctx* ctx);

@@ -333,39 +333,42 @@ __global__ __launch_bounds__(64 * kPbWaves) void k_pb_mfma(const WorkItem* __res
     }
 }
 
-// Final FP64 reduction, one wave per output cell: lane j sums the cell's
-// partial rows j, j+64, ... in order (all D basis functions at once), then a
-// fixed binary tree over the 64 lanes in LDS; Q = (2 * sum) / w, times
-// `scale` (the spatial operator's (d/L)^2 N dt, spat_oper_mod.f90:65-66).
+// Final FP64 reduction, one workgroup per output cell: W lanes read a partial
+// row (contiguous), kRedThreads / W rows side by side in list order, then a fixed
+// tree over the row groups; Q = (2 * sum) / w, times `scale` (the spatial
+// operator's (d/L)^2 N dt, spat_oper_mod.f90:65-66).
+constexpr int kRedThreads = 512;
 template <int D>
-__global__ __launch_bounds__(64) void k_pb_reduce(int64_t ncells, const int64_t* __restrict__ cell_ptr,
-                                                  const int32_t* __restrict__ cell_rows,
-                                                  const double* __restrict__ partial,
-                                                  const double* __restrict__ gwts, double scale,
-                                                  double* __restrict__ q) {
-  __shared__ double red[64 * (D + 1)];
+__global__ __launch_bounds__(kRedThreads) void k_pb_reduce(int64_t ncells, const int64_t* __restrict__ cell_ptr,
+                                                           const int32_t* __restrict__ cell_rows,
+                                                           const double* __restrict__ partial,
+                                                           const double* __restrict__ gwts, double scale,
+                                                           double* __restrict__ q) {
+  constexpr int W = D > 8 ? 32 : D > 1 ? 8 : 1, NG = kRedThreads / W;
+  static_assert(D <= 32, "a row fits its lanes");
+  __shared__ double red[kRedThreads];
   const int64_t c = blockIdx.x;
-  const int lane = threadIdx.x;
+  const int l = threadIdx.x % W, g = threadIdx.x / W;
   const int64_t b = cell_ptr[c], e = cell_ptr[c + 1];
-  double s[D];
+  double s = 0.0;
+  if (l < D) {
+    int64_t k = b + g;
+    for (; k + 3 * NG < e; k += 4 * NG) {   // four rows in flight
+      double v[4];
 #pragma unroll
-  for (int l = 0; l < D; ++l) s[l] = 0.0;
-  for (int64_t k = b + lane; k < e; k += 64) {
-    const double* row = partial + (int64_t)cell_rows[k] * D;
+      for (int i = 0; i < 4; ++i) v[i] = partial[(int64_t)cell_rows[k + i * NG] * D + l];
 #pragma unroll
-    for (int l = 0; l < D; ++l) s[l] = s[l] + row[l];
-  }
-#pragma unroll
-  for (int l = 0; l < D; ++l) red[lane * (D + 1) + l] = s[l];
-  __syncthreads();
-  for (int h = 32; h > 0; h >>= 1) {
-    if (lane < h) {
-#pragma unroll
-      for (int l = 0; l < D; ++l) red[lane * (D + 1) + l] = red[lane * (D + 1) + l] + red[(lane + h) * (D + 1) + l];
+      for (int i = 0; i < 4; ++i) s += v[i];
     }
+    for (; k < e; k += NG) s += partial[(int64_t)cell_rows[k] * D + l];
+  }
+  red[threadIdx.x] = s;
+  __syncthreads();
+  for (int h = NG / 2; h > 0; h >>= 1) {
+    if (g < h) red[threadIdx.x] += red[threadIdx.x + h * W];
     __syncthreads();
   }
-  for (int l = lane; l < D; l += 64) {
+  if (g == 0 && l < D) {
     double v = (2.0 * red[l]) / gwts[c * D + l];
     if (scale != 1.0) v = v * scale;
     q[c * D + l] = v;
@@ -424,6 +427,7 @@ static int launch_main_pairblock(dgv_ctx* ctx, const double* d_f, bool mfma, con
   const PairBlock& pb = ctx->pb;
   const Plan& P = ctx->plan;
   double* const part = partial ? partial : P.d_partial;
+  if (P.quad) return launch_main_quad(ctx, d_f, d_g, part);
   const int nitems = (int)P.items.size();
   if (nitems == 0) return DGV_OK;
   if (mfma) {
@@ -480,7 +484,7 @@ static int launch_reduce(dgv_ctx* ctx, double* d_q, double scale, const double* 
   switch (g.D) {
 #define DGV_RED_CASE(DD)                                                                               \
   case DD:                                                                                             \
-    hipLaunchKernelGGL(k_pb_reduce<DD>, dim3((unsigned)g.ncells), dim3(64), 0, ctx->stream, g.ncells,  \
+    hipLaunchKernelGGL(k_pb_reduce<DD>, dim3((unsigned)g.ncells), dim3(kRedThreads), 0, ctx->stream, g.ncells, \
                        P.d_cell_ptr, P.d_cell_rows, part, ctx->d_gwts, scale, d_q);                    \
     break;
     DGV_RED_CASE(1)
@@ -521,6 +525,10 @@ static int resolve_kernel(const dgv_ctx* ctx) {
   if (k == DGV_KERNEL_PAIRBLOCK && !pairblock_supported(D)) k = DGV_KERNEL_RECORD;
   return k;
 }
+
+// The merged layout serves the matrix-core evaluator wherever it was built; the
+// pair-block and record kernels stay as they are chosen.
+bool quad_wanted(const dgv_ctx* ctx) { return ctx->quad.use && resolve_kernel(ctx) == DGV_KERNEL_MFMA; }
 
 // The dominant kernel alone (no final reduction), for timing.
 int launch_eval_main_only(dgv_ctx* ctx, const double* d_f) {

@@ -55,6 +55,15 @@ __global__ void k_pair_index(int D, const BlockHdr* __restrict__ blocks, const d
   for (int i = threadIdx.x; i < DD; i += blockDim.x) out[i] = t[i];
 }
 
+int launch_pair_index(dgv_ctx* ctx, int16_t* d_idx) {
+  const int64_t nb = (int64_t)ctx->pb.blocks.size();
+  if (nb > 0)
+    hipLaunchKernelGGL(k_pair_index, dim3((unsigned)nb), dim3(256), 0, ctx->stream, ctx->g.D, ctx->pb.d_blocks,
+                       ctx->pb.d_pairs, d_idx);
+  DGV_HIP(ctx, hipGetLastError());
+  return DGV_OK;
+}
+
 // One wave per item; lane = column cell.  The coefficients and the index
 // table entries are wave-uniform (scalar loads); fm of the partner cell is the
 // lane's own (0 where that cell is off the grid: the record is then skipped,
@@ -274,10 +283,7 @@ static int ensure_fma_plan(dgv_ctx* ctx) {
   DGV_HIP(ctx, hipSetDevice(ctx->device));
   if (hipMalloc(&L.d_pidx, sizeof(int16_t) * (size_t)std::max<int64_t>(nb, 1) * D * D) != hipSuccess)
     return set_error(ctx, DGV_ERR_NOMEM, "hipMalloc(pair index tables) failed");
-  if (nb > 0)
-    hipLaunchKernelGGL(k_pair_index, dim3((unsigned)nb), dim3(256), 0, ctx->stream, D, pb.d_blocks, pb.d_pairs,
-                       L.d_pidx);
-  DGV_HIP(ctx, hipGetLastError());
+  if (int rc = launch_pair_index(ctx, L.d_pidx)) return rc;
   // block lists keyed by the offset (a for term 1, b for term 2)
   auto key = [](const int8_t* e) { return ((e[0] + 128) << 16) | ((e[1] + 128) << 8) | (e[2] + 128); };
   std::map<int, std::pair<std::vector<int32_t>, std::vector<int32_t>>> lists;

@@ -174,6 +174,7 @@ static int truncate_aarray(dgv_ctx* ctx, const TruncArgs& ta) {
   ctx->exp_valid = false;
   ctx->exp_idx.clear();
   ctx->exp_val.clear();
+  if (int rc = build_quads(ctx)) return rc;
   return build_plan(ctx, ctx->tile);
 }
 
@@ -206,7 +207,8 @@ int dgv_ctx_aarray_abs(dgv_ctx* ctx) {
   ctx->exp_valid = false;
   ctx->exp_idx.clear();
   ctx->exp_val.clear();
-  return DGV_OK;
+  if (int rc = build_quads(ctx)) return rc;
+  return build_plan(ctx, ctx->tile);
 }
 
 
