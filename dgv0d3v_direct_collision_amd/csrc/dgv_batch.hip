@@ -18,7 +18,9 @@
 // and f are rounded to FP32, products and the per-block sums run on
 // v_mfma_f32_16x16x4_f32, and the sums of every 32 pairs are folded into an
 // FP32 (hi, lo) pair with the two-sum of Knuth; the item writes hi + lo in FP64.
-// FP64: two waves per item, block sums added into an FP64 running total.
+// FP64: two waves per item, block sums added into an FP64 running total; where the
+// grids' A-arrays have a merged layout (dgv_quad.h) k_quad_batch evaluates it
+// instead, for 32 instances per item.
 // INT8_SPLIT: the same contraction in exact integer arithmetic (k_batch_i8).  A
 // second
 // kernel adds the items of each (cell, instance) in a fixed order in FP64 and
@@ -31,7 +33,7 @@
 #include <numeric>
 #include <vector>
 
-#include "dgv_internal.h"
+#include "dgv_quad.h"
 
 namespace dgv {
 
@@ -47,6 +49,9 @@ struct BatchGridDev {
   const uint32_t* codes;
   const double* bscale;
   const int64_t* pbeg16;
+  // merged layout: blist then lists quad blocks
+  const QuadBlk* qblocks;
+  const double* qsteps;
   int64_t foff;            // offset of this grid in the packed buffers
   int64_t eoff;            // offset of this grid in the per-(cell, instance) exponents (foff / D)
   int32_t Bpad, Mv, Mw, D;
@@ -54,7 +59,8 @@ struct BatchGridDev {
 
 // Work item: one cell's segment of blocks for up to kChunksPerItem chunks of
 // 64 instances (vc0 .. vc0 + nvc - 1); chunk k of the item writes the partial
-// rows prow + 64 k .. prow + 64 k + 63.
+// rows prow + 64 k .. prow + 64 k + 63.  Merged layout: one chunk of 32 instances,
+// partial rows prow .. prow + 31.
 struct BatchItem {
   int32_t grid, cell, b0, b1;  // blist range of the segment
   int32_t vc0, nvc;            // chunks of 64 instances
@@ -116,6 +122,7 @@ struct dgv_batch {
   std::vector<uint64_t> a_gen;     // each grid's A-array generation at creation
   int device = 0;                  // kept here: destroy must not read a grid context (it may be gone)
   int precision = DGV_FP64;
+  bool quad = false;               // FP64 on the grids' merged layouts
   int32_t ninst = 0;
   std::vector<int32_t> inst_grid, inst_local;
   std::vector<int32_t> nin, Bpad;
@@ -145,6 +152,7 @@ struct dgv_batch {
   int32_t nproj_task = 0;
   int project = 0;                        // project every evaluation's Q (FP64)
   int* d_counter = nullptr;
+  int32_t* d_nin = nullptr;        // instances per grid
   double* d_stage = nullptr;       // one instance's values (host copies)
   int ncu = 256;
   hipStream_t stream = nullptr;
@@ -1048,6 +1056,123 @@ __global__ __launch_bounds__(64) void k_batch_reduce(int64_t ntask, const int32_
   }
 }
 
+// FP64 on the merged layout: persistent workgroups of four waves, an item = one
+// cell's quad blocks of one run for 32 instances.  The columns of quad_walk are
+// instances: a staged row is 256 contiguous bytes of the packed f.
+template <int D>
+__global__ __launch_bounds__(256, 2) void k_quad_batch(const BatchItem* __restrict__ items, const QueueBounds QB,
+                                                       const BatchGridDev* __restrict__ grids,
+                                                       const double* __restrict__ f, double* __restrict__ partial,
+                                                       int* __restrict__ counter, const int32_t* __restrict__ nin) {
+  constexpr int NW = 4, NI = (D + 1) / 2, SL = 8 / NW, RT = (D + 15) / 16;
+  __shared__ __attribute__((aligned(16))) double lf[quad_rows<D>() * kQuadRow];
+  __shared__ int s_item;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int odd = lane >> 5, col = lane & 31;
+  for (int i = threadIdx.x; i < kQuadRow; i += 64 * NW) lf[8 * D * kQuadRow + i] = 0.0;
+  int q = blockIdx.x % kQueues, left = kQueues;   // this workgroup's XCD queue first
+  for (;;) {
+    if (threadIdx.x == 0) s_item = take_item(counter, QB, q, left);
+    __syncthreads();
+    const int id = __builtin_amdgcn_readfirstlane(s_item);
+    __syncthreads();
+    if (id < 0) return;
+    const BatchItem& it = items[id];
+    const BatchGridDev& G = grids[it.grid];
+    const int Mv = G.Mv, Mw = G.Mw, cell = it.cell, ncols = min(kQuadCols, nin[it.grid] - it.vc0 * kQuadCols);
+    const int32_t* list = G.blist + it.b0;
+    const QuadBlk* blocks = G.qblocks;
+    const uint32_t sp = (uint32_t)G.Bpad * 8;
+    const double* F = f + G.foff + (int64_t)it.vc0 * kQuadCols;
+    // rows odd, odd + 2, ... of the lane's column (with an odd D the last round's odd
+    // lanes repeat the last row)
+    const uint32_t goff = (uint32_t)odd * sp + (uint32_t)col * 8, glast = D % 2 ? (uint32_t)col * 8 : goff;
+    const uint32_t loff = (uint32_t)(odd * kQuadRow + col) * 8, llast = D % 2 ? (uint32_t)col * 8 : loff;
+    double v[SL][NI];
+    auto header = [&](int i) { return blocks[list[i]]; };
+    auto fetch = [&](const QuadBlk& B) {
+#pragma unroll
+      for (int k = 0; k < SL; ++k) {
+        const int slot = wave + NW * k;
+        if (slot & B.same) continue;   // the cell of a lower slot: its rows are used
+        const int du = slot & 1 ? B.b[0] : B.a[0], dv = slot & 2 ? B.b[1] : B.a[1], dw = slot & 4 ? B.b[2] : B.a[2];
+        const __amdgpu_buffer_rsrc_t R = ring_rsrc(F + (int64_t)(cell + (du * Mv + dv) * Mw + dw) * D * (sp / 8));
+#pragma unroll
+        for (int i = 0; i < NI; ++i) v[k][i] = ring_f64(R, i + 1 < NI ? goff : glast, (uint32_t)(2 * i) * sp);
+      }
+    };
+    auto store = [&](const QuadBlk& B) {
+#pragma unroll
+      for (int k = 0; k < SL; ++k) {
+        const int slot = wave + NW * k;
+        if (slot & B.same) continue;
+        char* dst = reinterpret_cast<char*>(lf) + slot * D * kQuadRow * 8;
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+          *reinterpret_cast<double*>(dst + (i + 1 < NI ? loff : llast) + 2 * i * kQuadRow * 8) = v[k][i];
+      }
+    };
+    const int n = it.b1 - it.b0;
+    auto walk = [&](auto ct) {
+      constexpr int CT = decltype(ct)::value;
+      qd4 acc[RT][CT];
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int c = 0; c < CT; ++c) acc[rt][c] = qd4{0.0, 0.0, 0.0, 0.0};
+      quad_walk<D, false, NW, CT>(n, header(0), 0, INT_MAX, G.qsteps, lf, lf, header, fetch, store, acc);
+      quad_flush<D, NW, CT>(lf, acc, ncols, partial + it.prow * D);
+    };
+    if (ncols > 16) walk(std::integral_constant<int, 2>{});
+    else walk(std::integral_constant<int, 1>{});
+  }
+}
+
+// One workgroup per (grid, cell, chunk of 32 instances): the items' partial rows in
+// item order (contiguous reads), Q = (2 s) / w * scale to the packed layout.
+template <int D>
+__global__ __launch_bounds__(256) void k_quad_batch_reduce(const int32_t* __restrict__ key,
+                                                           const int64_t* __restrict__ ptr,
+                                                           const int32_t* __restrict__ rows,
+                                                           const BatchGridDev* __restrict__ grids,
+                                                           const int32_t* __restrict__ nin,
+                                                           const double* __restrict__ partial, double scale,
+                                                           double* __restrict__ q) {
+  constexpr int NE = (kQuadCols * D + 255) / 256;
+  __shared__ double t[kQuadCols * D];
+  const int64_t task = blockIdx.x;
+  const int g = key[3 * task], c = key[3 * task + 1], v0 = key[3 * task + 2] * kQuadCols;
+  const BatchGridDev& G = grids[g];
+  const int ncols = min(kQuadCols, nin[g] - v0);
+  double s[NE];
+#pragma unroll
+  for (int i = 0; i < NE; ++i) s[i] = 0.0;
+  for (int64_t k = ptr[task]; k < ptr[task + 1]; ++k) {
+    const double* row = partial + (int64_t)rows[k] * D;
+#pragma unroll
+    for (int i = 0; i < NE; ++i) {
+      const int e = (int)threadIdx.x + 256 * i;
+      if (e < ncols * D) s[i] += row[e];
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NE; ++i) {
+    const int e = (int)threadIdx.x + 256 * i;
+    if (e < ncols * D) t[e] = s[i];
+  }
+  __syncthreads();
+  double* Q = q + G.foff + v0;
+  for (int e = threadIdx.x; e < kQuadCols * D; e += 256) {
+    const int l = e / kQuadCols, col = e % kQuadCols;
+    if (col >= ncols) continue;
+    const int64_t node = (int64_t)c * D + l;
+    double x = (2.0 * t[col * D + l]) / G.gwts[node];
+    if (scale != 1.0) x = x * scale;
+    Q[node * G.Bpad + col] = x;
+  }
+}
+
 // out = t0 + t1 + ... over the packed buffers (as k_lincomb)
 struct BLinTerm {
   const double* x;
@@ -1176,6 +1301,23 @@ static void destroy_plan(dgv_batch* b, BatchPlan& P) {
   if (&P == &b->plan && b->graph) { hipGraphExecDestroy(b->graph); b->graph = nullptr; }
 }
 
+// Pairs per run of the merged batch: about 2048 steps (2 MB of coefficients, shared
+// through one XCD's 4 MB L2 by the cells running on it), less where a small batch
+// would not give each of the 512 workgroups four items.
+static int32_t auto_tile(const dgv_batch* b, const std::vector<int32_t>* cells) {
+  double pairs = 0, steps = 0, items = 0;   // items: (cell, chunk) walks of a whole array
+  for (size_t g = 0; g < b->grids.size(); ++g) {
+    if (b->nin[g] == 0) continue;
+    pairs += (double)b->grids[g]->pb.npairs;
+    steps += (double)b->grids[g]->quad.nsteps;
+    items += (double)(cells ? (int64_t)cells->size() : b->grids[g]->g.ncells) * ((b->nin[g] + kQuadCols - 1) / kQuadCols);
+  }
+  const double per_walk = steps / std::max<double>(1, (double)b->grids.size());
+  const double runs = std::max(per_walk / 2048.0, 4.0 * 512.0 / std::max(items, 1.0));
+  const double tile = pairs / std::max<double>(1, (double)b->grids.size()) / std::max(runs, 1.0);
+  return (int32_t)std::min(1e9, std::max(256.0, tile));
+}
+
 // Per cell and grid: blocks whose box contains the cell, cut into segments;
 // items = segments x chunks of 64 instances.  Segments are global: the grid's
 // blocks in (a, b) order -- the order of every cell's list -- are cut into runs
@@ -1188,7 +1330,7 @@ static void destroy_plan(dgv_batch* b, BatchPlan& P) {
 static int build_batch_plan(dgv_batch* b, BatchPlan& P, int32_t tile, const std::vector<int32_t>* cells = nullptr) {
   if (int rc = batch_check_grids(b)) return rc;
   destroy_plan(b, P);
-  if (tile <= 0) tile = 1 << 20;
+  if (tile <= 0) tile = b->quad ? auto_tile(b, cells) : 1 << 20;
   P.tile = tile;
   std::vector<BatchItem> items;
   int64_t nrows = 0;
@@ -1202,8 +1344,19 @@ static int build_batch_plan(dgv_batch* b, BatchPlan& P, int32_t tile, const std:
     const PairBlock& pb = ctx->pb;
     const std::vector<int64_t>& cp = b->cell_ptr[gi];
     const std::vector<int32_t>& blist = b->h_blist[gi];
-    const int nchunk = b->Bpad[gi] / 64;
-    {
+    const int nchunk = b->quad ? (b->nin[gi] + kQuadCols - 1) / kQuadCols : b->Bpad[gi] / 64;
+    if (b->quad) {   // the quad blocks' own order
+      const QuadLayout& L = ctx->quad;
+      const double per_step = (double)pb.npairs / (double)std::max<int64_t>(L.nsteps, 1);
+      run_of[gi].assign(L.blocks.size(), 0);
+      double acc = 0;
+      int32_t run = 0;
+      for (size_t k = 0; k < L.blocks.size(); ++k) {
+        run_of[gi][k] = run;
+        acc += L.blocks[k].nst * per_step;
+        if (acc >= tile) { ++run; acc = 0; }
+      }
+    } else {
       std::vector<int32_t> order(pb.blocks.size());
       std::iota(order.begin(), order.end(), 0);
       std::sort(order.begin(), order.end(), [&](int32_t x, int32_t y) {
@@ -1238,7 +1391,8 @@ static int build_batch_plan(dgv_batch* b, BatchPlan& P, int32_t tile, const std:
           s0 = k + 1;
         }
       const bool fp32 = b->precision == DGV_FP32_COMP || b->precision == DGV_FP32_F64ACC;
-      const int chpi = fp32 ? chunks_per_item<true>() : chunks_per_item<false>();   // INT8_SPLIT: as FP64
+      const int chpi = b->quad ? 1 : fp32 ? chunks_per_item<true>() : chunks_per_item<false>();   // INT8_SPLIT: as FP64
+      const int width = b->quad ? kQuadCols : 64;
       for (int vc0 = 0; vc0 < nchunk; vc0 += chpi) {
         const int nvc = std::min(chpi, nchunk - vc0);
         std::vector<int64_t> first;   // first partial row of each segment's item
@@ -1247,14 +1401,14 @@ static int build_batch_plan(dgv_batch* b, BatchPlan& P, int32_t tile, const std:
           it.grid = (int32_t)gi; it.cell = (int32_t)c; it.b0 = sg.first; it.b1 = sg.second;
           it.vc0 = vc0; it.nvc = nvc;
           it.prow = nrows;
-          nrows += 64 * nvc;
+          nrows += width * nvc;
           if (nrows > INT32_MAX) return berr(b, DGV_ERR_UNSUPPORTED, "too many batch work items");
           first.push_back(it.prow);
           items.push_back(it);
         }
         for (int k = 0; k < nvc; ++k) {
           key.push_back((int32_t)gi); key.push_back((int32_t)c); key.push_back(vc0 + k);
-          for (int64_t r : first) rrows.push_back((int32_t)(r + 64 * k));
+          for (int64_t r : first) rrows.push_back((int32_t)(r + width * k));
           rptr.push_back((int64_t)rrows.size());
         }
       }
@@ -1352,7 +1506,14 @@ static int batch_eval_dev(dgv_batch* b, const BatchPlan& P, const double* d_f, d
 #define DGV_BATCH_LAUNCH(DD, MM)                                                                          \
   hipLaunchKernelGGL((k_batch_mfma<DD, MM>), dim3(nwg), blk, 0, st, P.d_items, P.queues, b->d_grids, d_f, \
                      b->d_f32, P.d_partial, b->d_counter)
-    if (b->precision == DGV_INT8_SPLIT) {
+    if (b->quad) {
+      if (D == 27)
+        hipLaunchKernelGGL(k_quad_batch<27>, dim3(nwg), blk, 0, st, P.d_items, P.queues, b->d_grids, d_f,
+                           P.d_partial, b->d_counter, b->d_nin);
+      else
+        hipLaunchKernelGGL(k_quad_batch<8>, dim3(nwg), blk, 0, st, P.d_items, P.queues, b->d_grids, d_f,
+                           P.d_partial, b->d_counter, b->d_nin);
+    } else if (b->precision == DGV_INT8_SPLIT) {
       if (D == 27)
         hipLaunchKernelGGL(k_batch_i8<27>, dim3(nwg), blk, 0, st, P.d_items, P.queues, b->d_grids, b->d_fhat,
                            b->d_fexp, P.d_partial, b->d_counter);
@@ -1370,7 +1531,14 @@ static int batch_eval_dev(dgv_batch* b, const BatchPlan& P, const double* d_f, d
     }
 #undef DGV_BATCH_LAUNCH
   }
-  if (reduce && P.nred > 0) {
+  if (reduce && P.nred > 0 && b->quad) {
+    if (D == 27)
+      hipLaunchKernelGGL(k_quad_batch_reduce<27>, dim3((unsigned)P.nred), dim3(256), 0, st, P.d_red_key, P.d_red_ptr,
+                         P.d_red_rows, b->d_grids, b->d_nin, P.d_partial, scale, d_q);
+    else
+      hipLaunchKernelGGL(k_quad_batch_reduce<8>, dim3((unsigned)P.nred), dim3(256), 0, st, P.d_red_key, P.d_red_ptr,
+                         P.d_red_rows, b->d_grids, b->d_nin, P.d_partial, scale, d_q);
+  } else if (reduce && P.nred > 0) {
     if (D == 27)
       hipLaunchKernelGGL(k_batch_reduce<27>, dim3((unsigned)P.nred), dim3(64), 0, st, P.nred, P.d_red_key,
                          P.d_red_ptr, P.d_red_rows, b->d_grids, P.d_partial, scale, d_q);
@@ -1466,6 +1634,8 @@ int dgv_batch_create(dgv_ctx* const* grids, int32_t ngrids, const int32_t* grid_
   for (int g = 0; g < ngrids; ++g) b->a_gen.push_back(grids[g]->a_gen);
   b->device = grids[0]->device;
   b->precision = precision;
+  b->quad = precision == DGV_FP64;
+  for (int g = 0; g < ngrids; ++g) b->quad = b->quad && grids[g]->quad.use;
   b->ninst = ninstances;
   b->nin.assign(ngrids, 0);
   b->inst_grid.resize(ninstances);
@@ -1510,6 +1680,9 @@ int dgv_batch_create(dgv_ctx* const* grids, int32_t ngrids, const int32_t* grid_
   if (i8 && (hipMalloc(&b->d_fhat, nb) || hipMalloc(&b->d_fexp, sizeof(int32_t) * std::max<int64_t>(b->total / D, 1))))
     return fail(DGV_ERR_NOMEM, "hipMalloc(fixed-point buffers)");
   if (hipMalloc(&b->d_counter, sizeof(int) * kQueues)) return fail(DGV_ERR_NOMEM, "hipMalloc(counter)");
+  if (hipMalloc(&b->d_nin, sizeof(int32_t) * ngrids) ||
+      hipMemcpy(b->d_nin, b->nin.data(), sizeof(int32_t) * ngrids, hipMemcpyHostToDevice))
+    return fail(DGV_ERR_NOMEM, "hipMalloc(instance counts)");
   {
     int64_t nmax = 1;
     for (int g = 0; g < ngrids; ++g) nmax = std::max<int64_t>(nmax, grids[g]->g.N);
@@ -1526,7 +1699,8 @@ int dgv_batch_create(dgv_ctx* const* grids, int32_t ngrids, const int32_t* grid_
     const dgv_ctx* ctx = grids[g];
     const PairBlock& pb = ctx->pb;
     std::vector<int64_t> cnt(ctx->g.ncells + 1, 0);
-    for (const Group& G : pb.groups)
+    const std::vector<Group>& groups = b->quad ? ctx->quad.groups : pb.groups;
+    for (const Group& G : groups)
       for (int r = 0; r < G.ncells; ++r) {
         int rr = r;
         const int cw = G.lo[2] + rr % G.ext[2]; rr /= G.ext[2];
@@ -1537,17 +1711,18 @@ int dgv_batch_create(dgv_ctx* const* grids, int32_t ngrids, const int32_t* grid_
     for (int64_t c = 0; c < ctx->g.ncells; ++c) cnt[c + 1] += cnt[c];
     std::vector<int32_t> blist(cnt.back());
     std::vector<int64_t> pos(cnt.begin(), cnt.end() - 1);
-    for (const Group& G : pb.groups)
+    for (const Group& G : groups)
       for (int r = 0; r < G.ncells; ++r) {
         int rr = r;
         const int cw = G.lo[2] + rr % G.ext[2]; rr /= G.ext[2];
         const int cv = G.lo[1] + rr % G.ext[1]; rr /= G.ext[1];
         const int cu = G.lo[0] + rr;
         const int64_t cell = ((int64_t)cu * ctx->g.Mv + cv) * ctx->g.Mw + cw;
-        for (int k = G.bbeg; k < G.bend; ++k) blist[pos[cell]++] = pb.group_blocks[k];
+        for (int k = G.bbeg; k < G.bend; ++k) blist[pos[cell]++] = b->quad ? k : pb.group_blocks[k];
       }
     // each cell's blocks ordered by (a, b): runs of equal a share the staged f[c + a]
-    for (int64_t c = 0; c < ctx->g.ncells; ++c)
+    // (quad blocks keep their own order)
+    for (int64_t c = 0; c < ctx->g.ncells && !b->quad; ++c)
       std::sort(blist.begin() + cnt[c], blist.begin() + cnt[c + 1], [&](int32_t x, int32_t y) {
         const BlockHdr &X = pb.blocks[x], &Y = pb.blocks[y];
         for (int d = 0; d < 3; ++d) if (X.a[d] != Y.a[d]) return X.a[d] < Y.a[d];
@@ -1603,6 +1778,8 @@ int dgv_batch_create(dgv_ctx* const* grids, int32_t ngrids, const int32_t* grid_
       if (hipMemsetAsync(b->d_pairs32[g] + n, 0, sizeof(float) * pad, b->stream))
         return fail(DGV_ERR_HIP, "hipMemsetAsync(FP32 coefficient padding)");
     }
+    gd[g].qblocks = ctx->quad.d_blocks;
+    gd[g].qsteps = ctx->quad.d_steps;
     gd[g].pairs64 = pb.d_pairs;
     gd[g].pairs32 = b->d_pairs32[g];
     gd[g].blocks = pb.d_blocks;
@@ -1655,7 +1832,7 @@ void dgv_batch_destroy(dgv_batch* b) {
   if (b->stream) hipStreamSynchronize(b->stream);
   destroy_plan(b, b->plan);
   destroy_plan(b, b->probe);
-  hipFree(b->d_f); hipFree(b->d_q); hipFree(b->d_f32); hipFree(b->d_counter); hipFree(b->d_grids);
+  hipFree(b->d_f); hipFree(b->d_q); hipFree(b->d_f32); hipFree(b->d_counter); hipFree(b->d_nin); hipFree(b->d_grids);
   hipFree(b->d_proj); hipFree(b->d_proj_task); hipFree(b->d_stage);
   for (int i = 0; i < 4; ++i) hipFree(b->d_tmp[i]);
   for (auto p : b->d_blist) hipFree(p);

@@ -24,6 +24,8 @@
 //                16-bit LDS byte offsets, the rows of x0 y0 x1 y1 x2 y2 x3 y3 (the
 //                zero row for both nodes of an absent pair).
 #pragma once
+#include <type_traits>
+
 #include "dgv_internal.h"
 
 namespace dgv {

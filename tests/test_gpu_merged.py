@@ -127,3 +127,47 @@ def test_infinite_and_nan_values_stay_where_they_were():
             assert np.array_equal(np.isfinite(q), np.isfinite(p))
     finally:
         d.close()
+
+
+@pytest.mark.parametrize("counts", [(1, 0), (16, 1), (17, 33), (64, 15)], ids=str)
+def test_batch_on_merged_layouts(counts):
+    """FP64 batches of two grids (32-instance chunks, a chunk of at most 16 columns,
+    a grid without instances), every tile, against the single-VDF evaluator; and
+    the same with one grid whose array does not merge."""
+    import dgv0d3v_direct_collision_amd as dgv
+    from tests.helpers import synthetic_aarray
+    G = oracle.Geometry((2, 3, 2), 3, (-1.2, 1.2))
+    a, c = dgv.DGV((4, 3, 3), 3, (-2.0, 2.0)), dgv.DGV((2, 3, 2), 3, (-1.2, 1.2))
+    try:
+        a.generate_aarray(nquad=16)
+        for merged in (True, False):
+            print(f"\n[merged] batch {counts} both grids merge: {merged}", flush=True)
+            if merged:
+                c.generate_aarray(nquad=16)
+            else:
+                c.set_aarray(*synthetic_aarray(G, seed=4))
+            which = np.repeat([0, 1], counts).astype(np.int32)
+            rng = np.random.default_rng(sum(counts))
+            fs = [rng.random([a, c][k].nnodes) for k in which]
+            ref = [[a, c][k].EvalCollisionPeriodicAPlus_DGV(f) for k, f in zip(which, fs)]
+            b = dgv.DGVBatch([a, c], which, dgv.DGV_FP64)
+            for i, f in enumerate(fs):
+                b.set_f(i, f)
+            for tile in (0, 1, 5000, 1 << 24):
+                b.set_tile(tile)
+                b.eval_q()
+                err = max(rel_l2(b.get_q(i), r) for i, r in enumerate(ref))
+                assert err <= TOL, (counts, merged, tile, err)
+            b.set_probe_cells([0, 5])
+            b.eval_q_probe()
+            assert rel_l2(b.get_q(0), ref[0]) <= TOL
+            b.rk_run(1e-4, 2, rkmts=2)
+            f = fs[0].copy()
+            a.rkmts = 2
+            for _ in range(2):
+                (a if which[0] == 0 else c).TimeIntegratorORK_SH_DGV(f, 1e-4)
+            assert rel_l2(b.get_f(0), f) <= TOL
+            b.close()
+    finally:
+        a.close()
+        c.close()
