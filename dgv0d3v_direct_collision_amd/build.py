@@ -23,6 +23,7 @@ HIPFLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-Wall",
 # (the batched kernel folds them on the VALU every few steps and reads them
 # without v_accvgpr_read moves).
 FILE_FLAGS = {"dgv_batch.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+              "dgv_linear.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
               "dgv_quad.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
               "dgv_kernels.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 

@@ -132,59 +132,176 @@ __global__ __launch_bounds__(64) void k_fma_build(const FmaItem* __restrict__ it
   }
 }
 
-// fc = 2 f . fmA for nv vectors: split over row chunks of kGemvRows, FP64
-// partial sums per chunk, then a fixed-order sum of the chunks.
-constexpr int kGemvRows = 256;
-constexpr int kGemvMaxVec = 8;
+// fc = 2 f . fmA for nv vectors on the matrix cores: C[v][i] = sum_r f[v][r] fmA[r][i]
+// with v_mfma_f64_16x16x4_f64, A = 16 vectors x 4 rows r (from LDS), B = 4 rows x 16
+// columns i, straight from fmA (a lane's two columns are one 16-byte load, a row's
+// 32 columns 256 contiguous bytes).  A workgroup of four waves takes 128 columns, 16
+// VT vectors and a chunk of rows; the chunks' sums are added in order by k_fma_sum.
+// One pass serves up to kLinVec vectors: up to about 50 the reading of fmA bounds it,
+// above them the matrix cores.  27^3 nodes (3.1 GB): 2 vectors 0.55 ms (5.6 TB/s), 32
+// 0.63, 64 0.94, 128 1.78, 256 3.46 ms (57 TFLOP/s); a pass over fmA per 8 vectors
+// on the vector units took 0.62, 3.1, 6.2, 12.4 and 24.7 ms.
+// rows of fmA per LDS tile of f (32 and 64 rows for the smaller vector tiles: 1-3 %
+// slower at 27^3 nodes, no faster at 15^3)
+constexpr int kLinRows = 16;
+constexpr int kLinCols = 128;    // columns per workgroup
+constexpr int kLinVec = 256;     // vectors per pass
 
-template <int NV>
-__global__ __launch_bounds__(256) void k_fma_gemv(int64_t N, const double* __restrict__ fma,
-                                                  const double* __restrict__ f, int64_t ldf,
-                                                  double* __restrict__ part) {
-  constexpr int kU = 16;  // row loads in flight per thread
-  __shared__ double fs[NV][kGemvRows];
+typedef double ld2 __attribute__((ext_vector_type(2)));
+typedef double ld4 __attribute__((ext_vector_type(4)));
+
+template <int VT>
+__global__ __launch_bounds__(256, 2) void k_fma_rows(int64_t N, int nv, int colblocks, int vblocks, int64_t chunk,
+                                                     const double* __restrict__ fma, const double* __restrict__ f,
+                                                     int64_t ldf, double* __restrict__ part) {
+  constexpr int BM = 16 * VT, P = kLinRows + 2;   // LDS pitch: 16 vectors x 2 rows cover the 64 banks once
+  constexpr int NL = BM * kLinRows / 256;         // f values per thread and tile
+  constexpr int KS = kLinRows / 4;
+  __shared__ double fs[2][BM * P];
+  // the vector blocks of one (column block, chunk) read the same fmA: neighbours on one XCD
+  const int w = blockIdx.x, x = w & 7, y = w >> 3;
+  const int vb = y % vblocks, pos = (y / vblocks) * 8 + x;
+  const int cb = pos % colblocks;
+  const int64_t ck = pos / colblocks;
+  const int64_t r0 = ck * chunk, r1 = min(N, r0 + chunk);
+  if (r0 >= r1) return;   // the grid is padded to whole groups of eight
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int kk = lane >> 4, jj = lane & 15;
+  const int64_t col = (int64_t)cb * kLinCols + wave * 32 + 2 * jj;
+  const int64_t cl = min(col, N - 2);            // the last columns' pair is read inside the row
+  const int v0 = vb * BM;
+  // this thread's f elements of a tile: vectors fr + FR i, row fc
+  constexpr int FR = 256 / kLinRows;
+  const int fr = threadIdx.x / kLinRows, fc = threadIdx.x % kLinRows;
+  double fv[NL];
+  auto fload = [&](int64_t r) {
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const int v = v0 + fr + FR * i;
+      fv[i] = (v < nv && r + fc < r1) ? f[(int64_t)v * ldf + r + fc] : 0.0;
+    }
+  };
+  auto fstore = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < NL; ++i) fs[b][(fr + FR * i) * P + fc] = fv[i];
+  };
+  ld2 bt[2][KS];
+  auto bload = [&](int b, int64_t r) {
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      const double* p = fma + min(r + 4 * k + kk, N - 1) * N + cl;   // rows past the chunk meet zeros of f
+      __builtin_memcpy(&bt[b][k], p, 16);
+    }
+  };
+  ld4 acc[VT][2];
+#pragma unroll
+  for (int t = 0; t < VT; ++t) acc[t][0] = acc[t][1] = ld4{0.0, 0.0, 0.0, 0.0};
+  fload(r0);
+  bload(0, r0);
+  int cur = 0;
+  auto tile = [&](int b, int64_t r) {   // b: this tile's buffers (constant after unrolling)
+    fstore(b);
+    __syncthreads();
+    if (r + kLinRows < r1) {
+      fload(r + kLinRows);
+      bload(b ^ 1, r + kLinRows);
+    }
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      double a[VT];
+#pragma unroll
+      for (int t = 0; t < VT; ++t) a[t] = fs[b][(16 * t + jj) * P + 4 * k + kk];
+#pragma unroll
+      for (int t = 0; t < VT; ++t) {
+        acc[t][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[t], bt[b][k][0], acc[t][0], 0, 0, 0);
+        acc[t][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[t], bt[b][k][1], acc[t][1], 0, 0, 0);
+      }
+    }
+  };
+  for (int64_t r = r0; r < r1; r += 2 * kLinRows) {
+    tile(0, r);
+    if (r + kLinRows < r1) tile(1, r + kLinRows);
+  }
+  // output layout: element e of lane jj + 16 kk is row (vector) 4 e + kk, columns col, col + 1
+  double* out = part + ck * nv * N;
+#pragma unroll
+  for (int t = 0; t < VT; ++t)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int v = v0 + 16 * t + 4 * e + kk;
+      if (v >= nv) continue;
+      if (col < N) out[(int64_t)v * N + col] = cl == col ? acc[t][0][e] : acc[t][1][e];
+      if (col + 1 < N) out[(int64_t)v * N + col + 1] = acc[t][1][e];
+    }
+}
+
+// One vector on the vector units: no rows of zeros to multiply (15^3 nodes: 19.8
+// us against 22.8; 27^3 nodes the same, both at the card's read rate).  Adds a
+// column's rows one after the other, as the matrix cores do: the sums are the
+// same to the last bit.
+__global__ __launch_bounds__(256) void k_fma_gemv(int64_t N, int64_t chunk, const double* __restrict__ fma,
+                                                  const double* __restrict__ f, double* __restrict__ part) {
+  constexpr int kU = 16;     // row loads in flight per thread
+  constexpr int kF = 256;    // rows of f in LDS
+  __shared__ double fs[kF];
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t r0 = (int64_t)blockIdx.y * kGemvRows;
-  const int nr = (int)(r0 + kGemvRows < N ? kGemvRows : N - r0);
-  for (int t = threadIdx.x; t < NV * kGemvRows; t += 256) {
-    const int v = t / kGemvRows, rr = t % kGemvRows;
-    fs[v][rr] = rr < nr ? f[v * ldf + r0 + rr] : 0.0;
+  const int64_t r0 = (int64_t)blockIdx.y * chunk, r1 = min(N, r0 + chunk);
+  const double* col = fma + (i < N ? i : N - 1);
+  double acc = 0.0;
+  for (int64_t b = r0; b < r1; b += kF) {
+    const int nr = (int)min((int64_t)kF, r1 - b);
+    __syncthreads();
+    fs[threadIdx.x] = (int)threadIdx.x < nr ? f[b + threadIdx.x] : 0.0;
+    __syncthreads();
+    int r = 0;
+    for (; r + kU <= nr; r += kU) {
+      double m[kU];
+#pragma unroll
+      for (int u = 0; u < kU; ++u) m[u] = col[(b + r + u) * N];
+#pragma unroll
+      for (int u = 0; u < kU; ++u) acc = __fma_rn(fs[r + u], m[u], acc);
+    }
+    for (; r < nr; ++r) acc = __fma_rn(fs[r], col[(b + r) * N], acc);
   }
-  __syncthreads();
-  const double* col = fma + r0 * N + (i < N ? i : N - 1);
-  double acc[NV];
+  if (i < N) part[(int64_t)blockIdx.y * N + i] = acc;
+}
+
+__global__ void k_fma_sum(int64_t N, int nchunk, int nv, const double* __restrict__ part, double* __restrict__ fc,
+                          int64_t ldq) {
+  const int64_t n = N * nv, step = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += step) {
+    double s = 0.0;
+    int c = 0;
+    for (; c + 8 <= nchunk; c += 8) {   // eight loads in flight, added in order
+      double x[8];
 #pragma unroll
-  for (int v = 0; v < NV; ++v) acc[v] = 0.0;
-  int r = 0;
-  for (; r + kU <= nr; r += kU) {
-    double m[kU];
+      for (int i = 0; i < 8; ++i) x[i] = part[(int64_t)(c + i) * n + t];
 #pragma unroll
-    for (int u = 0; u < kU; ++u) m[u] = col[(int64_t)(r + u) * N];
-#pragma unroll
-    for (int u = 0; u < kU; ++u)
-#pragma unroll
-      for (int v = 0; v < NV; ++v) acc[v] = __fma_rn(fs[v][r + u], m[u], acc[v]);
-  }
-  for (; r < nr; ++r) {
-    const double m = col[(int64_t)r * N];
-#pragma unroll
-    for (int v = 0; v < NV; ++v) acc[v] = __fma_rn(fs[v][r], m, acc[v]);
-  }
-  if (i < N) {
-#pragma unroll
-    for (int v = 0; v < NV; ++v) part[((int64_t)v * gridDim.y + blockIdx.y) * N + i] = acc[v];
+      for (int i = 0; i < 8; ++i) s += x[i];
+    }
+    for (; c < nchunk; ++c) s += part[(int64_t)c * n + t];
+    const int64_t v = t / N;
+    fc[v * ldq + (t - v * N)] = 2.0 * s;
   }
 }
 
-__global__ void k_fma_gemv_sum(int64_t N, int nchunk, int nv, const double* __restrict__ part,
-                               double* __restrict__ fc, int64_t ldq) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= N) return;
-  for (int v = 0; v < nv; ++v) {
-    double s = 0.0;
-    for (int c = 0; c < nchunk; ++c) s += part[((int64_t)v * nchunk + c) * N + i];
-    fc[v * ldq + i] = 2.0 * s;
-  }
+// How a pass over nv vectors is cut: vector tiles per workgroup (0: k_fma_gemv) and
+// chunks of rows.  The chunks depend on N alone, so that a vector's result does not
+// depend on how many are passed with it: about two rounds of workgroups for one
+// vector tile, 256 rows at least.
+struct LinPlan {
+  int vt, vblocks, colblocks, nchunk;
+  int64_t chunk;
+};
+static LinPlan lin_plan(int64_t N, int nv) {
+  LinPlan p;
+  p.vt = nv == 1 ? 0 : nv <= 16 ? 1 : nv <= 32 ? 2 : nv <= 64 ? 4 : 8;
+  p.vblocks = p.vt == 0 ? 1 : (nv + 16 * p.vt - 1) / (16 * p.vt);
+  p.colblocks = (int)((N + kLinCols - 1) / kLinCols);
+  const int64_t s = std::max<int64_t>(1, std::min<int64_t>(N / 256, 2048 / p.colblocks));
+  p.chunk = ((N + s - 1) / s + kLinRows - 1) / kLinRows * kLinRows;
+  p.nchunk = (int)((N + p.chunk - 1) / p.chunk);
+  return p;
 }
 
 // maxwelveldist (distributions_mod.f90:83-94) at every node
@@ -373,24 +490,33 @@ int eval_linear_dev(dgv_ctx* ctx, const double* d_f, int64_t ldf, double* d_fc, 
   LinearState& L = ctx->lin;
   if (!L.fma_valid) return set_error(ctx, DGV_ERR_STATE, "EvalCollisionLinear: no linearised operator (PrepareFMA)");
   const int64_t N = ctx->g.N;
-  const int nchunk = (int)((N + kGemvRows - 1) / kGemvRows);
-  if (!L.d_part &&
-      hipMalloc(&L.d_part, sizeof(double) * (size_t)kGemvMaxVec * nchunk * std::max<int64_t>(N, 1)) != hipSuccess) {
-    L.d_part = nullptr;
-    return set_error(ctx, DGV_ERR_NOMEM, "hipMalloc(GEMV partials) failed");
-  }
-  const dim3 grid((unsigned)((N + 255) / 256), (unsigned)nchunk);
-  for (int v0 = 0; v0 < nvec; v0 += kGemvMaxVec) {
-    const int nv = std::min(kGemvMaxVec, nvec - v0);
-    const double* f = d_f + v0 * ldf;
-    switch (nv) {
-#define DGV_GEMV_CASE(K) \
-  case K: hipLaunchKernelGGL(k_fma_gemv<K>, grid, dim3(256), 0, ctx->stream, N, L.d_fma, f, ldf, L.d_part); break;
-      DGV_GEMV_CASE(1) DGV_GEMV_CASE(2) DGV_GEMV_CASE(3) DGV_GEMV_CASE(4)
-      DGV_GEMV_CASE(5) DGV_GEMV_CASE(6) DGV_GEMV_CASE(7) DGV_GEMV_CASE(8)
-#undef DGV_GEMV_CASE
+  if (!L.d_part) {   // sums of the chunks, for the largest pass
+    int64_t most = 1;
+    for (int nv = 1; nv <= kLinVec; ++nv) most = std::max<int64_t>(most, (int64_t)lin_plan(N, nv).nchunk * nv * N);
+    if (hipMalloc(&L.d_part, sizeof(double) * (size_t)most) != hipSuccess) {
+      L.d_part = nullptr;
+      return set_error(ctx, DGV_ERR_NOMEM, "hipMalloc(partial products) failed");
     }
-    hipLaunchKernelGGL(k_fma_gemv_sum, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, ctx->stream, N, nchunk, nv,
+  }
+  for (int v0 = 0; v0 < nvec; v0 += kLinVec) {
+    const int nv = std::min(kLinVec, nvec - v0);
+    const double* f = d_f + v0 * ldf;
+    const LinPlan p = lin_plan(N, nv);
+    const unsigned nwg = (unsigned)(((int64_t)p.colblocks * p.nchunk + 7) / 8 * 8 * p.vblocks);
+    switch (p.vt) {
+      case 0:
+        hipLaunchKernelGGL(k_fma_gemv, dim3((unsigned)((N + 255) / 256), p.nchunk), dim3(256), 0, ctx->stream, N,
+                           p.chunk, L.d_fma, f, L.d_part);
+        break;
+#define DGV_LIN_CASE(VT)                                                                                        \
+  case VT:                                                                                                      \
+    hipLaunchKernelGGL(k_fma_rows<VT>, dim3(nwg), dim3(256), 0, ctx->stream, N, nv, p.colblocks, p.vblocks, p.chunk, \
+                       L.d_fma, f, ldf, L.d_part);                                                              \
+    break;
+      DGV_LIN_CASE(1) DGV_LIN_CASE(2) DGV_LIN_CASE(4) DGV_LIN_CASE(8)
+#undef DGV_LIN_CASE
+    }
+    hipLaunchKernelGGL(k_fma_sum, dim3(stride_blocks(N * nv, 64)), dim3(64), 0, ctx->stream, N, p.nchunk, nv,
                        L.d_part, d_fc + v0 * ldq, ldq);
   }
   DGV_HIP(ctx, hipGetLastError());
