@@ -192,11 +192,11 @@ struct FmaItem;
 // CheckSolutionMode_DGV).  Built on first use, dropped with the A-array.
 struct LinearState {
   double* d_fma = nullptr;        // N x N, fmA(r, i) at r * N + i
-  int16_t* d_pidx = nullptr;      // per block: pair index of (p, q) or -1
   FmaItem* d_items = nullptr;
-  int32_t* d_l1 = nullptr;        // block lists by a-offset / b-offset
-  int32_t* d_l2 = nullptr;
-  double* d_part = nullptr;       // GEMV partial sums
+  int64_t* d_beg = nullptr;       // per (row offset, node): its entries in d_desc
+  uint2* d_desc = nullptr;        // (pair, byte offset of the partner in d_halo)
+  double* d_halo = nullptr;       // fm with a halo of zeros
+  double* d_part = nullptr;       // partial products of eval_linear_dev
   int64_t nitems = 0;
   bool fma_valid = false;
   double* d_vec[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};  // fm, new Maxwellian, Df, scratch, reduction

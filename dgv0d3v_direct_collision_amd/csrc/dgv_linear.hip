@@ -16,9 +16,10 @@
 //   term 1: sum over blocks with a = e, pairs (s, q):  T[l] fm[c+b][q]
 //   term 2: sum over blocks with b = e, pairs (p, s):  T[l] fm[c+a][p]
 // (the reference's two scatter-adds per record, lines 447-448), then the
-// division by w_i (line 458).  A work item owns (e, s, 64 column cells) and
-// writes its entries once.  A per-block table idx[p*D+q] (pair index or -1)
-// lets term 2 walk a block by q as term 1 walks it by p.
+// division by w_i (line 458).  For one (e, s) that is a matrix product over all
+// those pairs, 27 basis functions by the column cells: its list of (pair, offset of
+// the partner's fm) is laid out once per A-array, and fm is read from a copy with
+// a halo of zeros around the grid, so that partners off the grid add nothing.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -29,12 +30,25 @@
 
 namespace dgv {
 
+typedef double ld2 __attribute__((ext_vector_type(2)));
+typedef double ld4 __attribute__((ext_vector_type(4)));
+
+// The column cells of one row offset e (their box), for the workgroup's four rows
+// s = 4 sgroup .. and 64 of the cells
 struct FmaItem {
-  int32_t e[3];
-  int32_t s;
+  int32_t e[3], sgroup;
   int32_t lo[3], ext[3];
-  int32_t ncells, chunk;
-  int32_t l1b, l1e, l2b, l2e;  // ranges in the block lists with a = e and b = e
+  int32_t ncells, chunk;   // chunk < 0: empty slot
+  int32_t elin, pad;       // index of e among the (2 M - 1) offsets per dimension
+};
+
+// The grid with a halo of M - 1 cells of zeros on every side
+struct FmaDims {
+  int32_t Mu, Mv, Mw;
+  __host__ __device__ int eu() const { return 3 * Mu - 2; }
+  __host__ __device__ int ev() const { return 3 * Mv - 2; }
+  __host__ __device__ int ew() const { return 3 * Mw - 2; }
+  __host__ __device__ int64_t ncext() const { return (int64_t)eu() * ev() * ew(); }
 };
 
 __global__ void k_pair_index(int D, const BlockHdr* __restrict__ blocks, const double* __restrict__ pairs,
@@ -64,71 +78,190 @@ int launch_pair_index(dgv_ctx* ctx, int16_t* d_idx) {
   return DGV_OK;
 }
 
-// One wave per item; lane = column cell.  The coefficients and the index
-// table entries are wave-uniform (scalar loads); fm of the partner cell is the
-// lane's own (0 where that cell is off the grid: the record is then skipped,
-// as the reference's bounds tests skip it).
-template <int D>
-__global__ __launch_bounds__(64) void k_fma_build(const FmaItem* __restrict__ items, const int32_t* __restrict__ l1,
-                                                  const int32_t* __restrict__ l2, const BlockHdr* __restrict__ blocks,
-                                                  const double* __restrict__ pairs, const int16_t* __restrict__ pidx,
-                                                  const double* __restrict__ fm, const double* __restrict__ gwts,
-                                                  int Mu, int Mv, int Mw, int64_t N, double* __restrict__ out) {
-  const FmaItem it = items[blockIdx.x];
-  const int lane = threadIdx.x;
-  const int cl = it.chunk * 64 + lane;
-  const bool active = cl < it.ncells;
-  int r = active ? cl : 0;
-  const int cw = it.lo[2] + r % it.ext[2];
-  r /= it.ext[2];
-  const int cv = it.lo[1] + r % it.ext[1];
-  r /= it.ext[1];
-  const int cu = it.lo[0] + r;
-  const int s = it.s;
-  double acc[D];
-#pragma unroll
-  for (int l = 0; l < D; ++l) acc[l] = 0.0;
+// fm with its halo, node of the cell outer: X[t][cell of the extended grid]; a last
+// plane t = D of zeros is the partner of the lists' padding
+__global__ void k_fma_halo(FmaDims g, int D, const double* __restrict__ fm, double* __restrict__ X) {
+  const int64_t nc = g.ncext(), n = nc * (D + 1), step = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += step) {
+    const int t = (int)(i / nc);
+    const int64_t c = i - t * nc;
+    const int w = (int)(c % g.ew()) - (g.Mw - 1), v = (int)(c / g.ew() % g.ev()) - (g.Mv - 1),
+              u = (int)(c / ((int64_t)g.ew() * g.ev())) - (g.Mu - 1);
+    const bool in = t < D && u >= 0 && u < g.Mu && v >= 0 && v < g.Mv && w >= 0 && w < g.Mw;
+    X[i] = in ? fm[(int64_t)((u * g.Mv + v) * g.Mw + w) * D + t] : 0.0;
+  }
+}
 
-  for (int k = it.l1b; k < it.l1e; ++k) {
-    const int bi = l1[k];
-    const BlockHdr* B = blocks + bi;
-    const int yu = cu + B->b[0], yv = cv + B->b[1], yw = cw + B->b[2];
-    const bool ok = yu >= 0 && yu < Mu && yv >= 0 && yv < Mv && yw >= 0 && yw < Mw;
-    const double* fy = fm + (int64_t)(ok ? (yu * Mv + yv) * Mw + yw : 0) * D;
-    const int16_t* ix = pidx + (int64_t)bi * D * D + s * D;
-    const double* P = pairs + B->pbeg * (D + 1);
-    for (int q = 0; q < D; ++q) {
-      const int j = ix[q];
-      if (j < 0) continue;
-      const double x = ok ? fy[q] : 0.0;
-      const double* T = P + (int64_t)j * (D + 1);
-#pragma unroll
-      for (int l = 0; l < D; ++l) acc[l] = __fma_rn(T[l], x, acc[l]);
+// One workgroup per row offset e: the entries (pair, byte offset in X of the
+// partner relative to the column cell) of every s, blocks in list order, pairs in
+// the order of the partner's node.  Without `desc` only counts them.
+template <int D>
+__global__ __launch_bounds__(256) void k_fma_lists(FmaDims g, const int32_t* __restrict__ p1, const int32_t* __restrict__ l1,
+                                                   const int32_t* __restrict__ p2, const int32_t* __restrict__ l2,
+                                                   const BlockHdr* __restrict__ blocks,
+                                                   const double* __restrict__ pairs, uint32_t zero_pair,
+                                                   const int64_t* __restrict__ beg, uint2* __restrict__ desc,
+                                                   uint32_t* __restrict__ cnt) {
+  __shared__ int32_t tab[D * D];
+  __shared__ uint32_t off[D];
+  const int64_t e = blockIdx.x;
+  const int nc = (int)g.ncext();
+  auto xoff = [&](const int8_t* o, int t) {
+    return (uint32_t)((t * nc + (o[0] * g.ev() + o[1]) * g.ew() + o[2]) * 8);
+  };
+  if (threadIdx.x < D) off[threadIdx.x] = 0;
+  __syncthreads();
+  for (int k = p1[e]; k < p1[e + 1]; ++k) {
+    const BlockHdr& B = blocks[l1[k]];
+    if (desc)
+      for (int j = threadIdx.x; j < B.npairs; j += 256) {
+        const int code = (int)(__double_as_longlong(pairs[(B.pbeg + j) * (D + 1) + D]) & 0xffff);
+        const int s = code >> 8;
+        desc[beg[e * D + s] + off[s] + (j - B.seg[s])] = make_uint2((uint32_t)(B.pbeg + j), xoff(B.b, code & 255));
+      }
+    __syncthreads();
+    if (threadIdx.x < D) off[threadIdx.x] += B.seg[threadIdx.x + 1] - B.seg[threadIdx.x];
+    __syncthreads();
+  }
+  for (int k = p2[e]; k < p2[e + 1]; ++k) {
+    const BlockHdr& B = blocks[l2[k]];
+    for (int i = threadIdx.x; i < D * D; i += 256) tab[i] = -1;
+    __syncthreads();
+    for (int j = threadIdx.x; j < B.npairs; j += 256) {
+      const int code = (int)(__double_as_longlong(pairs[(B.pbeg + j) * (D + 1) + D]) & 0xffff);
+      tab[(code >> 8) * D + (code & 255)] = j;
+    }
+    __syncthreads();
+    if (threadIdx.x < D) {
+      const int s = threadIdx.x;
+      uint32_t r = off[s];
+      for (int p = 0; p < D; ++p) {
+        const int j = tab[p * D + s];
+        if (j < 0) continue;
+        if (desc) desc[beg[e * D + s] + r] = make_uint2((uint32_t)(B.pbeg + j), xoff(B.a, p));
+        ++r;
+      }
+      off[s] = r;
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x < D) {
+    const int64_t i = e * D + threadIdx.x;
+    if (!desc) {
+      cnt[i] = off[threadIdx.x];
+    } else {   // the list's end: a pair of zero coefficients, the plane of zeros
+      for (int64_t k = beg[i] + off[threadIdx.x]; k < beg[i + 1]; ++k) desc[k] = make_uint2(zero_pair, (uint32_t)(D * nc * 8));
     }
   }
-  for (int k = it.l2b; k < it.l2e; ++k) {
-    const int bi = l2[k];
-    const BlockHdr* B = blocks + bi;
-    const int xu = cu + B->a[0], xv = cv + B->a[1], xw = cw + B->a[2];
-    const bool ok = xu >= 0 && xu < Mu && xv >= 0 && xv < Mv && xw >= 0 && xw < Mw;
-    const double* fx = fm + (int64_t)(ok ? (xu * Mv + xv) * Mw + xw : 0) * D;
-    const int16_t* ix = pidx + (int64_t)bi * D * D + s;
-    const double* P = pairs + B->pbeg * (D + 1);
-    for (int p = 0; p < D; ++p) {
-      const int j = ix[p * D];
-      if (j < 0) continue;
-      const double x = ok ? fx[p] : 0.0;
-      const double* T = P + (int64_t)j * (D + 1);
+}
+
+// One wave per (e, s, 64 column cells): A = 16 basis functions x 4 pairs, B = 4 pairs
+// x 16 cells of v_mfma_f64_16x16x4_f64, two row tiles and CT column tiles.  The list
+// entries are two rings ahead, the operands one.  The gathers of fm bound it (seven
+// loads per eight products, matrix cores busy 52 %), and half the products meet the
+// halo's zeros: 65 ms at 27^3 nodes against 148 ms with one lane per cell and
+// scalar coefficients.
+constexpr int kFmaRing = 4;                  // also the lists' padding in steps
+constexpr int kFmaListPad = 4 * 2 * kFmaRing;   // entries past the last list that the rings read
+
+template <int D, int CT>
+__device__ __forceinline__ void fma_walk(int64_t nsteps, const uint2* __restrict__ list, const double* __restrict__ pairs,
+                                         const double* __restrict__ X, const uint32_t (&xb)[4], int jj, int kk,
+                                         ld4 (&acc)[(D + 15) / 16][4]) {
+  constexpr int RT = (D + 15) / 16, R = kFmaRing;
+  uint2 d[R];
+  double a[R][RT], b[R][CT];
+  auto entry = [&](int u, int64_t i) { d[u] = list[4 * i + kk]; };
+  auto operands = [&](int u) {
+    const double* T = pairs + (int64_t)d[u].x * (D + 1) + jj;
 #pragma unroll
-      for (int l = 0; l < D; ++l) acc[l] = __fma_rn(T[l], x, acc[l]);
+    for (int rt = 0; rt < RT; ++rt) a[u][rt] = T[16 * rt];   // rows past D: dropped on output
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+      b[u][ct] = *reinterpret_cast<const double*>(reinterpret_cast<const char*>(X) + (uint32_t)(xb[ct] + d[u].y));
+  };
+#pragma unroll
+  for (int u = 0; u < R; ++u) entry(u, u);
+#pragma unroll
+  for (int u = 0; u < R; ++u) {
+    operands(u);
+    entry(u, u + R);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  for (int64_t i = 0; i < nsteps; i += R) {   // lists are padded to whole rounds
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+          acc[rt][ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u][rt], b[u][ct], acc[rt][ct], 0, 0, 0);
+      // loads in slot order: the waits count them
+      __builtin_amdgcn_sched_barrier(0);
+      operands(u);
+      entry(u, i + u + 2 * R);
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
-  if (active) {
-    const int64_t row = (int64_t)(((cu + it.e[0]) * Mv + (cv + it.e[1])) * Mw + (cw + it.e[2])) * D + s;
-    const int64_t col = (int64_t)((cu * Mv + cv) * Mw + cw) * D;
+}
+
+template <int D>
+__global__ __launch_bounds__(256, 2) void k_fma_build(const FmaItem* __restrict__ items, FmaDims g,
+                                                      const int64_t* __restrict__ beg, const uint2* __restrict__ desc,
+                                                      const double* __restrict__ pairs, const double* __restrict__ X,
+                                                      const double* __restrict__ gwts, int64_t N,
+                                                      double* __restrict__ out) {
+  constexpr int RT = (D + 15) / 16;
+  const FmaItem& it = items[blockIdx.x];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int s = it.sgroup * 4 + wave, chunk = it.chunk;
+  if (chunk < 0 || s >= D) return;
+  const int kk = lane >> 4, jj = lane & 15;
+  const int ncols = min(64, it.ncells - chunk * 64);
+  const int ct_n = (ncols + 15) / 16;
+  uint32_t xb[4];
+  int32_t cell[4];
+#pragma unroll
+  for (int ct = 0; ct < 4; ++ct) {
+    const int c = chunk * 64 + 16 * ct + jj;
+    int r = c < it.ncells ? c : chunk * 64;   // idle columns follow the chunk's first cell
+    const int cw = it.lo[2] + r % it.ext[2];
+    r /= it.ext[2];
+    const int cv = it.lo[1] + r % it.ext[1];
+    r /= it.ext[1];
+    const int cu = it.lo[0] + r;
+    cell[ct] = c < it.ncells ? (cu * g.Mv + cv) * g.Mw + cw : -1;
+    xb[ct] = (uint32_t)((((cu + g.Mu - 1) * g.ev() + cv + g.Mv - 1) * g.ew() + cw + g.Mw - 1) * 8);
+  }
+  ld4 acc[RT][4];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+    for (int ct = 0; ct < 4; ++ct) acc[rt][ct] = ld4{0.0, 0.0, 0.0, 0.0};
+  const int64_t b0 = beg[(int64_t)it.elin * D + s], b1 = beg[(int64_t)it.elin * D + s + 1];
+  const uint2* list = desc + b0;
+  const int64_t nsteps = (b1 - b0) / 4;
+  if (nsteps > 0) {
+    switch (ct_n) {
+      case 1: fma_walk<D, 1>(nsteps, list, pairs, X, xb, jj, kk, acc); break;
+      case 2: fma_walk<D, 2>(nsteps, list, pairs, X, xb, jj, kk, acc); break;
+      case 3: fma_walk<D, 3>(nsteps, list, pairs, X, xb, jj, kk, acc); break;
+      default: fma_walk<D, 4>(nsteps, list, pairs, X, xb, jj, kk, acc); break;
+    }
+  }
+  const int de = (it.e[0] * g.Mv + it.e[1]) * g.Mw + it.e[2];
+#pragma unroll
+  for (int ct = 0; ct < 4; ++ct) {
+    if (cell[ct] < 0) continue;
+    const int64_t row = (int64_t)(cell[ct] + de) * D + s, col = (int64_t)cell[ct] * D;
     double* o = out + row * N + col;
 #pragma unroll
-    for (int l = 0; l < D; ++l) o[l] = acc[l] / gwts[col + l];
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int l = 16 * rt + 4 * k + kk;   // FP64 output layout
+        if (l < D) o[l] = acc[rt][ct][k] / gwts[col + l];
+      }
   }
 }
 
@@ -146,9 +279,6 @@ __global__ __launch_bounds__(64) void k_fma_build(const FmaItem* __restrict__ it
 constexpr int kLinRows = 16;
 constexpr int kLinCols = 128;    // columns per workgroup
 constexpr int kLinVec = 256;     // vectors per pass
-
-typedef double ld2 __attribute__((ext_vector_type(2)));
-typedef double ld4 __attribute__((ext_vector_type(4)));
 
 template <int VT>
 __global__ __launch_bounds__(256, 2) void k_fma_rows(int64_t N, int nv, int colblocks, int vblocks, int64_t chunk,
@@ -361,9 +491,9 @@ __global__ void k_sum_scale(int64_t n, const double* __restrict__ x, const doubl
 
 void free_linear(dgv_ctx* ctx) {
   LinearState& L = ctx->lin;
-  hipFree(L.d_fma); hipFree(L.d_pidx); hipFree(L.d_items); hipFree(L.d_l1); hipFree(L.d_l2);
+  hipFree(L.d_fma); hipFree(L.d_items); hipFree(L.d_beg); hipFree(L.d_desc); hipFree(L.d_halo);
   hipFree(L.d_part);
-  L.d_fma = nullptr; L.d_pidx = nullptr; L.d_items = nullptr; L.d_l1 = nullptr; L.d_l2 = nullptr;
+  L.d_fma = nullptr; L.d_items = nullptr; L.d_beg = nullptr; L.d_desc = nullptr; L.d_halo = nullptr;
   L.d_part = nullptr;
   L.nitems = 0;
   L.fma_valid = false;
@@ -388,67 +518,141 @@ static int ensure_vectors(dgv_ctx* ctx) {
   return DGV_OK;
 }
 
-// Block index tables, block lists by offset and the work items (once per A-array).
-static int ensure_fma_plan(dgv_ctx* ctx) {
+// The lists of every (e, s) and the work items (once per A-array).
+template <int D>
+static int build_fma_plan(dgv_ctx* ctx) {
   LinearState& L = ctx->lin;
-  if (L.d_items) return DGV_OK;
   const Grid& g = ctx->g;
   const PairBlock& pb = ctx->pb;
-  const int D = g.D;
-  if (D > 64) return set_error(ctx, DGV_ERR_UNSUPPORTED, "PrepareFMA: more than 64 nodes per cell");
-  const int64_t nb = (int64_t)pb.blocks.size();
-  DGV_HIP(ctx, hipSetDevice(ctx->device));
-  if (hipMalloc(&L.d_pidx, sizeof(int16_t) * (size_t)std::max<int64_t>(nb, 1) * D * D) != hipSuccess)
-    return set_error(ctx, DGV_ERR_NOMEM, "hipMalloc(pair index tables) failed");
-  if (int rc = launch_pair_index(ctx, L.d_pidx)) return rc;
-  // block lists keyed by the offset (a for term 1, b for term 2)
-  auto key = [](const int8_t* e) { return ((e[0] + 128) << 16) | ((e[1] + 128) << 8) | (e[2] + 128); };
-  std::map<int, std::pair<std::vector<int32_t>, std::vector<int32_t>>> lists;
-  for (int64_t bi = 0; bi < nb; ++bi) {
-    const BlockHdr& B = pb.blocks[bi];
-    if (B.seg[D] == 0) continue;
-    lists[key(B.a)].first.push_back((int32_t)bi);
-    lists[key(B.b)].second.push_back((int32_t)bi);
-  }
-  std::vector<int32_t> l1, l2;
-  std::vector<FmaItem> items;
+  const FmaDims dims{g.Mu, g.Mv, g.Mw};
   const int M[3] = {g.Mu, g.Mv, g.Mw};
-  for (auto& kv : lists) {
-    const int e[3] = {((kv.first >> 16) & 255) - 128, ((kv.first >> 8) & 255) - 128, (kv.first & 255) - 128};
-    FmaItem it{};
-    int ncells = 1;
-    for (int d = 0; d < 3; ++d) {
-      const int lo = std::max(0, -e[d]), hi = std::min(M[d], M[d] - e[d]);
-      it.e[d] = e[d];
-      it.lo[d] = lo;
-      it.ext[d] = std::max(0, hi - lo);
-      ncells *= it.ext[d];
-    }
-    if (ncells == 0) continue;
-    it.ncells = ncells;
-    it.l1b = (int32_t)l1.size();
-    l1.insert(l1.end(), kv.second.first.begin(), kv.second.first.end());
-    it.l1e = (int32_t)l1.size();
-    it.l2b = (int32_t)l2.size();
-    l2.insert(l2.end(), kv.second.second.begin(), kv.second.second.end());
-    it.l2e = (int32_t)l2.size();
-    for (int s = 0; s < D; ++s)
-      for (int c = 0; c * 64 < ncells; ++c) {
-        it.s = s;
-        it.chunk = c;
-        items.push_back(it);
-      }
+  const int64_t ne = (int64_t)(2 * M[0] - 1) * (2 * M[1] - 1) * (2 * M[2] - 1);
+  if (pb.npairs >= (int64_t)UINT32_MAX || dims.ncext() * (D + 1) * 8 > (int64_t)INT32_MAX)
+    return set_error(ctx, DGV_ERR_UNSUPPORTED, "PrepareFMA: grid or A-array too large");
+  DGV_HIP(ctx, hipSetDevice(ctx->device));
+  // block lists by offset (a for term 1, b for term 2), blocks in layout order
+  auto elin = [&](const int8_t* o) {
+    return ((int64_t)(o[0] + M[0] - 1) * (2 * M[1] - 1) + (o[1] + M[1] - 1)) * (2 * M[2] - 1) + (o[2] + M[2] - 1);
+  };
+  const int64_t nb = (int64_t)pb.blocks.size();
+  std::vector<int32_t> ptr[2], list[2];
+  for (int t = 0; t < 2; ++t) {
+    ptr[t].assign(ne + 1, 0);
+    for (const BlockHdr& B : pb.blocks) ptr[t][elin(t ? B.b : B.a) + 1]++;
+    for (int64_t e = 0; e < ne; ++e) ptr[t][e + 1] += ptr[t][e];
+    list[t].resize(std::max<int64_t>(nb, 1));
+    std::vector<int32_t> at(ptr[t].begin(), ptr[t].end() - 1);
+    for (int64_t k = 0; k < nb; ++k) list[t][at[elin(t ? pb.blocks[k].b : pb.blocks[k].a)]++] = (int32_t)k;
   }
+  // items: every (row cell, column cell) pair of the grid belongs to one e, so the
+  // whole operator is written, zeros included
+  std::vector<FmaItem> items;
+  std::vector<int64_t> epairs(ne, 0);
+  for (const BlockHdr& B : pb.blocks) {
+    epairs[elin(B.a)] += B.npairs;
+    epairs[elin(B.b)] += B.npairs;
+  }
+  constexpr int NS = (D + 3) / 4, kXcd = 8;
+  std::vector<FmaItem> col[kXcd];
+  std::vector<int64_t> order(ne);
+  std::vector<FmaItem> proto(ne);
+  int64_t k = 0;
+  for (int e0 = -(M[0] - 1); e0 < M[0]; ++e0)
+    for (int e1 = -(M[1] - 1); e1 < M[1]; ++e1)
+      for (int e2 = -(M[2] - 1); e2 < M[2]; ++e2, ++k) {
+        FmaItem it{};
+        const int e[3] = {e0, e1, e2};
+        it.ncells = 1;
+        for (int d = 0; d < 3; ++d) {
+          it.e[d] = e[d];
+          it.lo[d] = std::max(0, -e[d]);
+          it.ext[d] = std::min(M[d], M[d] - e[d]) - it.lo[d];
+          it.ncells *= it.ext[d];
+        }
+        it.elin = (int32_t)k;
+        proto[k] = it;
+        order[k] = k;
+      }
+  // an offset's items read the same coefficients: one XCD's L2 (workgroup i runs on
+  // XCD i % 8), the heaviest offsets first
+  auto work = [&](int64_t e) { return epairs[e] * ((proto[e].ncells + 15) / 16) + 64 * (int64_t)proto[e].ncells; };
+  std::stable_sort(order.begin(), order.end(), [&](int64_t x, int64_t y) { return work(x) > work(y); });
+  int64_t xload[kXcd] = {};
+  for (int64_t e : order) {
+    const int x = (int)(std::min_element(xload, xload + kXcd) - xload);
+    FmaItem it = proto[e];
+    for (int sg = 0; sg < NS; ++sg)
+      for (int c = 0; c * 64 < it.ncells; ++c) {
+        it.sgroup = sg;
+        it.chunk = c;
+        col[x].push_back(it);
+      }
+    xload[x] += work(e);
+  }
+  size_t nslot = 0;
+  for (auto& v : col) nslot = std::max(nslot, v.size());
+  FmaItem none{};
+  none.chunk = -1;
+  items.assign(nslot * kXcd, none);
+  for (int x = 0; x < kXcd; ++x)
+    for (size_t i = 0; i < col[x].size(); ++i) items[i * kXcd + x] = col[x][i];
   L.nitems = (int64_t)items.size();
-  if (hipMalloc(&L.d_items, sizeof(FmaItem) * std::max<size_t>(items.size(), 1)) != hipSuccess ||
-      hipMalloc(&L.d_l1, sizeof(int32_t) * std::max<size_t>(l1.size(), 1)) != hipSuccess ||
-      hipMalloc(&L.d_l2, sizeof(int32_t) * std::max<size_t>(l2.size(), 1)) != hipSuccess)
+  int32_t *d_ptr[2] = {}, *d_list[2] = {};
+  uint32_t* d_cnt = nullptr;
+  auto drop = [&]() {
+    for (int t = 0; t < 2; ++t) { hipFree(d_ptr[t]); hipFree(d_list[t]); }
+    hipFree(d_cnt);
+  };
+  auto nomem = [&]() {
+    drop();
+    hipFree(L.d_items); hipFree(L.d_beg); hipFree(L.d_desc); hipFree(L.d_halo);
+    L.d_items = nullptr; L.d_beg = nullptr; L.d_desc = nullptr; L.d_halo = nullptr;
     return set_error(ctx, DGV_ERR_NOMEM, "hipMalloc(fmA plan) failed");
-  DGV_HIP(ctx, hipMemcpyAsync(L.d_items, items.data(), sizeof(FmaItem) * items.size(), hipMemcpyHostToDevice,
-                              ctx->stream));
-  DGV_HIP(ctx, hipMemcpyAsync(L.d_l1, l1.data(), sizeof(int32_t) * l1.size(), hipMemcpyHostToDevice, ctx->stream));
-  DGV_HIP(ctx, hipMemcpyAsync(L.d_l2, l2.data(), sizeof(int32_t) * l2.size(), hipMemcpyHostToDevice, ctx->stream));
-  DGV_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  };
+  bool ok = hipMalloc(&L.d_beg, sizeof(int64_t) * (ne * D + 1)) == hipSuccess &&
+            hipMalloc(&d_cnt, sizeof(uint32_t) * ne * D) == hipSuccess &&
+            hipMalloc(&L.d_halo, sizeof(double) * dims.ncext() * (D + 1)) == hipSuccess;
+  for (int t = 0; t < 2; ++t)
+    ok = ok && hipMalloc(&d_ptr[t], sizeof(int32_t) * (ne + 1)) == hipSuccess &&
+         hipMalloc(&d_list[t], sizeof(int32_t) * list[t].size()) == hipSuccess;
+  if (!ok) return nomem();
+  hipStream_t st = ctx->stream;
+  hipError_t e = hipSuccess;
+  for (int t = 0; t < 2 && e == hipSuccess; ++t) {
+    e = hipMemcpyAsync(d_ptr[t], ptr[t].data(), sizeof(int32_t) * (ne + 1), hipMemcpyHostToDevice, st);
+    if (e == hipSuccess)
+      e = hipMemcpyAsync(d_list[t], list[t].data(), sizeof(int32_t) * list[t].size(), hipMemcpyHostToDevice, st);
+  }
+  std::vector<uint32_t> cnt(ne * D);
+  std::vector<int64_t> beg(ne * D + 1, 0);
+  auto lists = [&](uint2* desc) {
+    hipLaunchKernelGGL(k_fma_lists<D>, dim3((unsigned)ne), dim3(256), 0, st, dims, d_ptr[0], d_list[0], d_ptr[1],
+                       d_list[1], pb.d_blocks, pb.d_pairs, (uint32_t)pb.npairs, L.d_beg, desc, d_cnt);
+    return hipGetLastError();
+  };
+  if (e == hipSuccess) e = lists(nullptr);
+  if (e == hipSuccess) e = hipMemcpyAsync(cnt.data(), d_cnt, sizeof(uint32_t) * ne * D, hipMemcpyDeviceToHost, st);
+  if (e == hipSuccess) e = hipStreamSynchronize(st);
+  if (e == hipSuccess) {
+    constexpr int64_t round = 4 * kFmaRing;
+    for (int64_t i = 0; i < ne * D; ++i) beg[i + 1] = beg[i] + (cnt[i] + round - 1) / round * round;
+    if (hipMalloc(&L.d_desc, sizeof(uint2) * (beg[ne * D] + kFmaListPad)) != hipSuccess ||
+        hipMalloc(&L.d_items, sizeof(FmaItem) * std::max<size_t>(items.size(), 1)) != hipSuccess)
+      return nomem();
+    // past the last list: pair 0, read ahead and never multiplied
+    e = hipMemsetAsync(L.d_desc + beg[ne * D], 0, sizeof(uint2) * kFmaListPad, st);
+    if (e == hipSuccess) e = hipMemcpyAsync(L.d_beg, beg.data(), sizeof(int64_t) * beg.size(), hipMemcpyHostToDevice, st);
+    if (e == hipSuccess)
+      e = hipMemcpyAsync(L.d_items, items.data(), sizeof(FmaItem) * items.size(), hipMemcpyHostToDevice, st);
+    if (e == hipSuccess) e = lists(L.d_desc);
+    if (e == hipSuccess) e = hipStreamSynchronize(st);
+  }
+  drop();
+  if (e != hipSuccess) {
+    hipFree(L.d_items);
+    L.d_items = nullptr;
+    return set_error(ctx, DGV_ERR_HIP, std::string("fmA plan: ") + hipGetErrorString(e));
+  }
   return DGV_OK;
 }
 
@@ -458,7 +662,7 @@ int prepare_fma_dev(dgv_ctx* ctx, const double* d_fm) {
   const Grid& g = ctx->g;
   const int D = g.D;
   if (D != 8 && D != 27) return set_error(ctx, DGV_ERR_UNSUPPORTED, "PrepareFMA: 2 or 3 nodes per dimension only");
-  int rc = ensure_fma_plan(ctx);
+  int rc = L.d_items ? DGV_OK : D == 27 ? build_fma_plan<27>(ctx) : build_fma_plan<8>(ctx);
   if (rc) return rc;
   rc = ensure_vectors(ctx);
   if (rc) return rc;
@@ -469,17 +673,15 @@ int prepare_fma_dev(dgv_ctx* ctx, const double* d_fm) {
   }
   if (d_fm != L.d_vec[0])
     DGV_HIP(ctx, hipMemcpyAsync(L.d_vec[0], d_fm, sizeof(double) * N, hipMemcpyDeviceToDevice, ctx->stream));
-  DGV_HIP(ctx, hipMemsetAsync(L.d_fma, 0, sizeof(double) * (size_t)N * N, ctx->stream));
-  if (L.nitems > 0) {
-    if (D == 27)
-      hipLaunchKernelGGL(k_fma_build<27>, dim3((unsigned)L.nitems), dim3(64), 0, ctx->stream, L.d_items, L.d_l1,
-                         L.d_l2, ctx->pb.d_blocks, ctx->pb.d_pairs, L.d_pidx, L.d_vec[0], ctx->d_gwts, g.Mu, g.Mv,
-                         g.Mw, N, L.d_fma);
-    else
-      hipLaunchKernelGGL(k_fma_build<8>, dim3((unsigned)L.nitems), dim3(64), 0, ctx->stream, L.d_items, L.d_l1,
-                         L.d_l2, ctx->pb.d_blocks, ctx->pb.d_pairs, L.d_pidx, L.d_vec[0], ctx->d_gwts, g.Mu, g.Mv,
-                         g.Mw, N, L.d_fma);
-  }
+  const FmaDims dims{g.Mu, g.Mv, g.Mw};
+  hipLaunchKernelGGL(k_fma_halo, dim3(stride_blocks(dims.ncext() * (D + 1), 256)), dim3(256), 0, ctx->stream, dims, D,
+                     L.d_vec[0], L.d_halo);
+  if (D == 27)
+    hipLaunchKernelGGL(k_fma_build<27>, dim3((unsigned)L.nitems), dim3(256), 0, ctx->stream, L.d_items, dims, L.d_beg,
+                       L.d_desc, ctx->pb.d_pairs, L.d_halo, ctx->d_gwts, N, L.d_fma);
+  else
+    hipLaunchKernelGGL(k_fma_build<8>, dim3((unsigned)L.nitems), dim3(256), 0, ctx->stream, L.d_items, dims, L.d_beg,
+                       L.d_desc, ctx->pb.d_pairs, L.d_halo, ctx->d_gwts, N, L.d_fma);
   DGV_HIP(ctx, hipGetLastError());
   L.fma_valid = true;
   L.nprepare++;
