@@ -62,9 +62,9 @@ struct BatchGridDev {
 // rows prow + 64 k .. prow + 64 k + 63.  Where an item has fewer chunks than its
 // workgroup has waves for (FP32 modes and INT8_SPLIT), its blocks are cut into
 // `parts` shares of about equal pairs and the waves of a share take all its
-// chunks; share p writes the rows prow + 64 (k + p nvc) ...  Without the shares
+// chunks; the shares' sums are added in LDS, in order.  Without the shares
 // half (INT8_SPLIT, up to 64 instances) or three quarters (FP32) of the waves
-// idled: 64 instances on 27^3 nodes INT8_SPLIT 757 -> 553 ms, 16 on 9^3 nodes FP32
+// idled: 64 instances on 27^3 nodes INT8_SPLIT 757 -> 479 ms, 16 on 9^3 nodes FP32
 // 0.99 -> 0.30 ms; full items are untouched.  Merged layout: one
 // chunk of 32 instances, partial rows prow .. prow + 31.
 constexpr int kMaxParts = 4;
@@ -72,11 +72,11 @@ struct BatchItem {
   int32_t grid, cell, b0, b1;  // blist range of the segment
   int32_t vc0, nvc;            // chunks of 64 instances
   int64_t prow;                // first partial row
-  int32_t parts, cut[kMaxParts - 1];   // share p: cut[p - 1] .. cut[p] (b0 and b1 at the ends)
+  int32_t parts, cut[kMaxParts + 1];   // share p: cut[p] .. cut[p + 1]
 };
-__device__ __forceinline__ int2 item_share(const BatchItem& it, int p) {
-  return make_int2(p == 0 ? it.b0 : it.cut[p - 1], p == it.parts - 1 ? it.b1 : it.cut[p]);
-}
+// share p of an item, by scalar loads (an index into a copy of the item would put
+// it in scratch memory, and the block walk with it on vector loads)
+__device__ __forceinline__ int2 item_share(const BatchItem* it, int p) { return make_int2(it->cut[p], it->cut[p + 1]); }
 
 // The batched kernels' eight work queues: items beg[q] .. beg[q + 1] - 1.  A
 // queue holds whole runs of blocks (every cell's items of a run), so the
@@ -290,9 +290,9 @@ __global__ __launch_bounds__(64 * kWavesPerItem) void k_batch_mfma(const BatchIt
   using V4 = typename std::conditional<FP32, bf4, bd4>::type;
   typedef T VB __attribute__((ext_vector_type(CT)));
   static_assert(sizeof(VB) == 16, "one 16-byte LDS read per lane and step");
-  __shared__ T lfa[CH][D * 64], lfb[CH][D * 64];
+  __shared__ __attribute__((aligned(16))) T lf[2][CH][D * 64];   // f(c+a) | f(c+b) of each chunk
   __shared__ int s_item;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kk = lane >> 4, jj = lane & 15;
   const int ch = wave / WPC;                     // this wave's chunk within the item
   const int sub = wave % WPC;                    // its part of the chunk's staging / columns
@@ -325,7 +325,7 @@ __global__ __launch_bounds__(64 * kWavesPerItem) void k_batch_mfma(const BatchIt
     const int part = FP32 ? ch / it.nvc : 0, vc = FP32 ? ch - part * it.nvc : ch;
     const bool active = FP32 ? part < it.parts : ch < it.nvc;
     const bool in_step = !FP32 || it.parts == 1;
-    const int2 share = FP32 && active ? item_share(it, part) : make_int2(it.b0, it.b1);
+    const int2 share = FP32 && active ? item_share(items + id, part) : make_int2(it.b0, it.b1);
     const int Mv = G.Mv, Mw = G.Mw;
     const int c = it.cell;
     const int cw = c % Mw, cv = (c / Mw) % Mv, cu = c / (Mw * Mv);
@@ -341,8 +341,8 @@ __global__ __launch_bounds__(64 * kWavesPerItem) void k_batch_mfma(const BatchIt
         if constexpr (FP32) lo[rt][ct] = V4{0, 0, 0, 0};
         if constexpr (ACC64) hd[rt][ct] = bd4{0, 0, 0, 0};
       }
-    T* la = lfa[ch];
-    T* lb = lfb[ch];
+    T* la = lf[0][ch];
+    T* lb = lf[1][ch];
     int prev_xc = -1;   // the cell whose f is in la (blocks come ordered by a)
     // fold a round's matrix-core sums into the FP32 (hi, lo) pair, or into the
     // FP64 sums (the next round's first products start a fresh sum, so acc
@@ -570,22 +570,56 @@ __global__ __launch_bounds__(64 * kWavesPerItem) void k_batch_mfma(const BatchIt
       }
     }
 #undef FOLD
+    // output layouts: FP64 row 4e + lane/16, FP32 row 4 (lane/16) + e
+    double sum[RT][CT][4];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if constexpr (ACC64) sum[rt][ct][e] = hd[rt][ct][e];
+          else if constexpr (FP32) sum[rt][ct][e] = (double)hi[rt][ct][e] + (double)lo[rt][ct][e];
+          else sum[rt][ct][e] = hi[rt][ct][e];
+        }
+    if (FP32 && it.parts > 1) {   // the shares' sums, added by the first share's wave of the chunk
+      static_assert(!FP32 || sizeof(lf) >= sizeof(double) * CH * D * 64, "the staged rows make room for the sums");
+      double* slab = reinterpret_cast<double*>(&lf[0][0][0]);
+      auto at = [&](int w, int rt, int ct, int e) -> double* {
+        return slab + ((int64_t)w * D + f32_row_fn<D>(rt, 4 * kk + e)) * 64 + col0 + CT * jj + ct;
+      };
+      __syncthreads();   // every wave is done with its staged rows
+      if (active && part > 0) {
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (f32_row_fn<D>(rt, 4 * kk + e) < D) *at(ch, rt, ct, e) = sum[rt][ct][e];
+      }
+      __syncthreads();
+      if (part > 0) continue;
+      for (int p = 1; p < it.parts; ++p)
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (f32_row_fn<D>(rt, 4 * kk + e) < D) sum[rt][ct][e] += *at(vc + p * it.nvc, rt, ct, e);
+    }
     if (!active) continue;
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
       for (int ct = 0; ct < CT; ++ct) {
         const int v = col0 + CT * jj + ct;
-        double* out = partial + (it.prow + 64 * ch + v) * D;
+        double* out = partial + (it.prow + 64 * vc + v) * D;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          // output layouts: FP64 row 4e + lane/16, FP32 row 4 (lane/16) + e
           const int l = FP32 ? f32_row_fn<D>(rt, 4 * kk + e) : 16 * rt + 4 * e + kk;
-          if (l < D) {
-            if constexpr (ACC64) out[l] = hd[rt][ct][e];
-            else if constexpr (FP32) out[l] = (double)hi[rt][ct][e] + (double)lo[rt][ct][e];
-            else out[l] = hi[rt][ct][e];
-          }
+          if (l < D) out[l] = sum[rt][ct][e];
         }
       }
   }
@@ -776,7 +810,7 @@ __global__ __launch_bounds__(256) void k_batch_i8(const BatchItem* __restrict__ 
   __shared__ __attribute__((aligned(16))) double s_sa[4][2][32];         // [wave][block parity]: row scales
   __shared__ __attribute__((aligned(16))) int s_fe[4][2][64];            // [wave][parity]: exponents of f(c+a), f(c+b)
   __shared__ int s_item;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kk = lane >> 4, jj = lane & 15;
   const int ch = wave / WPC, sub = wave % WPC;
   const int lcol = sub * 32 + 2 * jj;              // the lane's instances in the chunk: lcol, lcol + 1
@@ -792,8 +826,8 @@ __global__ __launch_bounds__(256) void k_batch_i8(const BatchItem* __restrict__ 
     if (id < 0) return;
     const BatchItem it = items[id];
     const int part = ch / it.nvc, vc = ch - part * it.nvc;   // the wave's share of the blocks and its chunk
-    if (part >= it.parts) continue;
-    const int2 share = item_share(it, part);
+    const bool active = part < it.parts;   // a chunk without work: its columns lie past the grid's instances
+    const int2 share = active ? item_share(items + id, part) : make_int2(0, 0);
     const BatchGridDev G = grids[it.grid];
     const int Mv = G.Mv, Mw = G.Mw;
     const int c = it.cell;
@@ -1028,11 +1062,36 @@ __global__ __launch_bounds__(256) void k_batch_i8(const BatchItem* __restrict__ 
 #undef I8_LOAD
 #undef I8_LOAD_R
     }
+    if (it.parts > 1) {   // the shares' sums, added by the first share's waves of the chunk
+      // (every staged row has been waited for, so a wave's own buffers are free)
+      static_assert(sizeof(s_f[0]) >= sizeof(double) * 64 * RT * CT * 4, "the staged rows make room for the sums");
+      auto at = [&](int w, int rt, int ct, int e) -> double* {
+        return reinterpret_cast<double*>(&s_f[w][0][0][0]) + ((rt * CT + ct) * 4 + e) * 64 + lane;
+      };
+      if (part > 0) {
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) *at(wave, rt, ct, e) = tot[rt][ct][e];
+      }
+      __syncthreads();
+      if (part > 0) continue;
+      for (int p = 1; p < it.parts; ++p)
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) tot[rt][ct][e] += *at(wave + p * it.nvc * WPC, rt, ct, e);
+    }
+    if (!active) continue;
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
       for (int ct = 0; ct < CT; ++ct) {
-        double* out = partial + (it.prow + 64 * ch + lcol + ct) * D;
+        double* out = partial + (it.prow + 64 * vc + lcol + ct) * D;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int l = 16 * rt + 4 * kk + e;   // int32 16x16 output: row 4 (lane / 16) + e
@@ -1320,10 +1379,63 @@ static void destroy_plan(dgv_batch* b, BatchPlan& P) {
   if (&P == &b->plan && b->graph) { hipGraphExecDestroy(b->graph); b->graph = nullptr; }
 }
 
-// Pairs per run of the merged batch: about 2048 steps (2 MB of coefficients, shared
+static int chunks_of_item(const dgv_batch* b) {   // chunks per item of the batch's kernel
+  const bool fp32 = b->precision == DGV_FP32_COMP || b->precision == DGV_FP32_F64ACC;
+  return b->quad ? 1 : fp32 ? chunks_per_item<true>() : chunks_per_item<false>();   // INT8_SPLIT: as FP64
+}
+static int shares_of_item(const dgv_batch* b, int nvc) {   // shares of an item of nvc chunks
+  return b->quad || b->precision == DGV_FP64 ? 1 : chunks_of_item(b) / nvc;
+}
+
+// Pairs per run.  Merged batch: about 2048 steps (2 MB of coefficients, shared
 // through one XCD's 4 MB L2 by the cells running on it), less where a small batch
 // would not give each of the 512 workgroups four items.
+// Otherwise: 4096 pairs for each wave of an item, which keeps the runs of the
+// cells on one XCD close enough together to meet in L2 (27^3 nodes, 64 instances
+// INT8_SPLIT: 479 ms with 1 M pairs a run, 375 with 64 K; 256 instances FP32: 1478
+// and 1434), down to 1024 where the 512 workgroups would get fewer than three
+// items each (9^3 nodes, 64 instances, INT8_SPLIT: 2.29 ms with one item per cell, 0.22
+// with 8 K pairs a run, 0.30 with 2 K; 15^3 nodes, 256 instances, FP32: 59 ms with 1 M,
+// 13.7 with 16 K, 15.0 with 2 K); but no more partial sums than a quarter of the
+// coefficients' bytes or 1 GB, and at most 1 M pairs.
 static int32_t auto_tile(const dgv_batch* b, const std::vector<int32_t>* cells) {
+  if (!b->quad) {
+    const int D = b->grids[0]->g.D;
+    const int chpi = chunks_of_item(b);
+    const double coef = b->precision == DGV_INT8_SPLIT ? 128.0 * ((D + 15) / 16) : b->precision == DGV_FP64 ? 8.0 * (D + 1) : 4.0 * (D + 2);
+    // walk: pairs walked by the waves of all items; whole: the same if every block held every cell
+    double walk = 0, whole = 0, bytes = 0, rows = 0;
+    for (size_t g = 0; g < b->grids.size(); ++g) {
+      if (b->nin[g] == 0) continue;
+      const auto& pb = b->grids[g]->pb;
+      const std::vector<int64_t>& cp = b->cell_ptr[g];
+      const std::vector<int32_t>& bl = b->h_blist[g];
+      double listed = 0, ncells = 0;
+      auto add = [&](int64_t c) {
+        ++ncells;
+        for (int64_t k = cp[c]; k < cp[c + 1]; ++k) listed += pb.blocks[bl[k]].npairs;
+      };
+      if (cells) {
+        for (int32_t c : *cells)
+          if (c >= 0 && c < b->grids[g]->g.ncells) add(c);
+      } else {
+        for (int64_t c = 0; c < b->grids[g]->g.ncells; ++c) add(c);
+      }
+      const int nchunk = b->Bpad[g] / 64;
+      for (int vc0 = 0; vc0 < nchunk; vc0 += chpi) {
+        walk += listed / shares_of_item(b, std::min(chpi, nchunk - vc0));
+        whole += ncells * (double)pb.npairs;
+      }
+      rows += 64.0 * nchunk * listed;   // rows times tile
+      bytes += coef * (double)pb.npairs;
+    }
+    if (walk <= 0) return 1 << 20;
+    const double per_wave = std::min(4096.0, std::max(1024.0, walk / (3 * 512.0)));
+    // a cell's part of a run is about twice its share of the pairs: blocks near in
+    // order lie near in space (27^3 nodes: 297 K items of 64 K pairs, 9.1e9 pairs walked)
+    const double fit = 2 * rows * D * 8 / std::max(1e9, bytes / 4);
+    return (int32_t)std::min(1048576.0, std::max(per_wave * whole / walk, fit));
+  }
   double pairs = 0, steps = 0, items = 0;   // items: (cell, chunk) walks of a whole array
   for (size_t g = 0; g < b->grids.size(); ++g) {
     if (b->nin[g] == 0) continue;
@@ -1349,7 +1461,8 @@ static int32_t auto_tile(const dgv_batch* b, const std::vector<int32_t>* cells) 
 static int build_batch_plan(dgv_batch* b, BatchPlan& P, int32_t tile, const std::vector<int32_t>* cells = nullptr) {
   if (int rc = batch_check_grids(b)) return rc;
   destroy_plan(b, P);
-  if (tile <= 0) tile = b->quad ? auto_tile(b, cells) : 1 << 20;
+  const bool automatic = tile <= 0;
+  if (automatic) tile = auto_tile(b, cells);
   P.tile = tile;
   std::vector<BatchItem> items;
   int64_t nrows = 0;
@@ -1409,12 +1522,11 @@ static int build_batch_plan(dgv_batch* b, BatchPlan& P, int32_t tile, const std:
           segs.push_back({(int32_t)s0, (int32_t)(k + 1)});
           s0 = k + 1;
         }
-      const bool fp32 = b->precision == DGV_FP32_COMP || b->precision == DGV_FP32_F64ACC;
-      const int chpi = b->quad ? 1 : fp32 ? chunks_per_item<true>() : chunks_per_item<false>();   // INT8_SPLIT: as FP64
+      const int chpi = chunks_of_item(b);
       const int width = b->quad ? kQuadCols : 64;
       for (int vc0 = 0; vc0 < nchunk; vc0 += chpi) {
         const int nvc = std::min(chpi, nchunk - vc0);
-        const int parts = fp32 || b->precision == DGV_INT8_SPLIT ? chpi / nvc : 1;
+        const int parts = shares_of_item(b, nvc);
         std::vector<int64_t> first;   // first partial row of each segment's item
         for (auto& sg : segs) {
           BatchItem it{};
@@ -1422,25 +1534,26 @@ static int build_batch_plan(dgv_batch* b, BatchPlan& P, int32_t tile, const std:
           it.vc0 = vc0; it.nvc = nvc;
           it.prow = nrows;
           it.parts = parts;
+          it.cut[0] = it.b0;
+          it.cut[parts] = it.b1;
           if (parts > 1) {
             int64_t all = 0, acc = 0;
             for (int32_t k = it.b0; k < it.b1; ++k) all += pb.blocks[blist[k]].npairs;
             int p = 1;
             for (int32_t k = it.b0; k < it.b1 && p < parts; ++k) {
               acc += pb.blocks[blist[k]].npairs;
-              while (p < parts && acc * parts >= all * p) it.cut[p++ - 1] = k + 1;
+              while (p < parts && acc * parts >= all * p) it.cut[p++] = k + 1;
             }
-            for (; p < parts; ++p) it.cut[p - 1] = it.b1;
+            for (; p < parts; ++p) it.cut[p] = it.b1;
           }
-          nrows += width * nvc * parts;
+          nrows += width * nvc;
           if (nrows > INT32_MAX) return berr(b, DGV_ERR_UNSUPPORTED, "too many batch work items");
           first.push_back(it.prow);
           items.push_back(it);
         }
         for (int k = 0; k < nvc; ++k) {
           key.push_back((int32_t)gi); key.push_back((int32_t)c); key.push_back(vc0 + k);
-          for (int64_t r : first)
-            for (int p = 0; p < parts; ++p) rrows.push_back((int32_t)(r + width * (k + p * nvc)));
+          for (int64_t r : first) rrows.push_back((int32_t)(r + width * k));
           rptr.push_back((int64_t)rrows.size());
         }
       }
@@ -1497,7 +1610,12 @@ static int build_batch_plan(dgv_batch* b, BatchPlan& P, int32_t tile, const std:
   P.nred = (int64_t)rptr.size() - 1;
   BHIP(b, hipMalloc(&P.d_items, sizeof(BatchItem) * std::max<size_t>(P.items.size(), 1)));
   BHIP(b, hipMemcpy(P.d_items, P.items.data(), sizeof(BatchItem) * P.items.size(), hipMemcpyHostToDevice));
-  if (hipMalloc(&P.d_partial, sizeof(double) * std::max<int64_t>(P.nrows * D, 1)) != hipSuccess)
+  if (hipMalloc(&P.d_partial, sizeof(double) * std::max<int64_t>(P.nrows * D, 1)) != hipSuccess) {
+    P.d_partial = nullptr;
+    (void)hipGetLastError();
+    if (automatic && !b->quad && tile < (1 << 20)) return build_batch_plan(b, P, 1 << 20, cells);   // the fewest rows
+  }
+  if (!P.d_partial)
     return berr(b, DGV_ERR_NOMEM, "hipMalloc(batch partial sums) failed");
   BHIP(b, hipMalloc(&P.d_red_rows, sizeof(int32_t) * std::max<size_t>(rrows.size(), 1)));
   BHIP(b, hipMemcpy(P.d_red_rows, rrows.data(), sizeof(int32_t) * rrows.size(), hipMemcpyHostToDevice));
