@@ -775,21 +775,6 @@ constexpr int kI8Ring = 6;   // even: the x dwords alternate by step parity; 6 m
 __device__ __forceinline__ constexpr int i8_vmcnt(int n) { return (n & 15) | (7 << 4) | (15 << 8) | ((n >> 4) << 14); }
 constexpr int kI8LgkmZero = 15 | (7 << 4) | (3 << 14);
 
-// Direct global-to-LDS loads: lane l's 16 (4) bytes from g land at LDS byte
-// address lds + 16 l (4 l).  Written out so that the compiler does not hold the
-// wave's LDS reads of the other buffers behind them; the kernel orders them
-// itself (vector-memory count waits before the staged data is read).
-__device__ __forceinline__ void i8_lds_load16(const void* g, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(g) : "memory", "m0");
-}
-__device__ __forceinline__ void i8_lds_load4(const void* g, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(g) : "memory", "m0");
-}
-template <typename T>
-__device__ __forceinline__ uint32_t lds_addr(T* p) {
-  return (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) T*)p));
-}
-
 template <int D>
 __global__ __launch_bounds__(256) void k_batch_i8(const BatchItem* __restrict__ items, const QueueBounds QB,
                                                   const BatchGridDev* __restrict__ grids,
@@ -874,15 +859,15 @@ __global__ __launch_bounds__(256) void k_batch_i8(const BatchItem* __restrict__ 
 #pragma unroll
         for (int i = 0; i < ROWS / 4; ++i) {
           const int p = min(4 * i + kk, D - 1);
-          i8_lds_load16(src + p * Bpad, lb + i * 1024);
+          lds_load16(src + p * Bpad, lb + i * 1024);
         }
       };
       // ... and of a block's row scales and the exponents of its two cells
       auto stage_scales = [&](const Hdr& h, int par) {
         const char* sa = reinterpret_cast<const char*>(G.bscale + (int64_t)h.blk * 16 * RT) + ((lane * 4) & (16 * RT * 8 - 1));
-        i8_lds_load4(sa, lds_addr(&s_sa[wave][par][0]));
+        lds_load4(sa, lds_addr(&s_sa[wave][par][0]));
         const int32_t* se = FE + (int64_t)(lane < 32 ? h.xc : h.yc) * Bpad + vcol0 + (lane & 31);
-        i8_lds_load4(se, lds_addr(&s_fe[wave][par][0]));
+        lds_load4(se, lds_addr(&s_fe[wave][par][0]));
       };
       // the cell held by each f buffer
       int tag_a0 = -1, tag_a1 = -1, tag_b0 = -1, tag_b1 = -1;

@@ -80,6 +80,21 @@ __device__ __forceinline__ void ring_i32x2(__amdgpu_buffer_rsrc_t r, uint32_t la
   b = (int)v[1];
 }
 
+// Direct global-to-LDS loads: lane l's 16 (4) bytes from g land at LDS byte
+// address lds + 16 l (4 l).  Written out so that the compiler does not hold the
+// wave's LDS reads of the other buffers behind them; the kernel orders them
+// itself (vector-memory count waits before the staged data is read).
+__device__ __forceinline__ void lds_load16(const void* g, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(g) : "memory", "m0");
+}
+__device__ __forceinline__ void lds_load4(const void* g, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(g) : "memory", "m0");
+}
+template <typename T>
+__device__ __forceinline__ uint32_t lds_addr(T* p) {
+  return (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) T*)p));
+}
+
 // Blocks for a grid-stride loop over n items. HIP limits one grid dimension to
 // fewer than 2^32 work-items, and the coefficient arrays of a 33^3 grid already
 // hold more elements than that, so element-wise kernels stride over a capped grid.

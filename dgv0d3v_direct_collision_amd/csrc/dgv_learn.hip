@@ -48,78 +48,94 @@ __device__ __forceinline__ float gelu_d(float z) {
 }
 
 // ---------------------------------------------------------------------------------
-// C[s][m][n] = sum_{k in chunk s} A[m][k] B[n][k].  Block tile 128 x 128, k step
-// 64, four waves each owning a 64 x 64 quadrant as 4 x 4 MFMA tiles of 16 x 16.
-// Requirements (checked by the host): M, N multiples of 128, K and kchunk
+// C[s][m][n] = sum_{k in chunk s} A[m][k] B[n][k].  Block tile GT x GT, k step 64, four
+// waves each owning a quadrant of 16 x 16 MFMA tiles.  A training step's products
+// are small (256 x 1024 x 3456 and the like), so what bounds them is the latency of
+// a K step's loads over a handful of steps on a part of the chip: the K steps go
+// straight to LDS, GT_RING - 1 of them in flight, and small products take tiles of
+// 64 (four times the workgroups).  The tile does not enter the order of an element's
+// sum.  Rows are 128 bytes of LDS; the 16-byte piece c of row r lies at c ^ (r % 8), so that
+// the sixteen rows of a matrix operand read different banks.
+// Requirements (checked by the host): M, N multiples of GT_PAD, K and kchunk
 // multiples of 64, lda and ldb multiples of 8.
-constexpr int GT_M = 128, GT_N = 128, GT_K = 64, G_SLD = GT_K + 8;
+constexpr int GT_PAD = 128, GT_K = 64, kGradRing = 3;
 
+template <int GT>
+constexpr int gt_tiles() { return GT / 32; }   // MFMA tiles of a wave in each direction
+
+// One workgroup's tile at (m0, n0) over nst K steps from kb0, in acc; sm holds GT_RING steps
+template <int GT, int GT_RING>
+__device__ __forceinline__ void gemm_tile(int m0, int n0, int kb0, int nst, const uint16_t* __restrict__ A, int64_t lda,
+                                          const uint16_t* __restrict__ B, int64_t ldb, uint16_t (*sm)[2 * GT * GT_K],
+                                          f4_t (&acc)[gt_tiles<GT>()][gt_tiles<GT>()]) {
+  constexpr int kWaveLoads = GT / 16;   // a wave's loads per K step: 8 rows each of the 2 GT rows of A and B
+  constexpr int TI = gt_tiles<GT>();
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = (wave >> 1) * (GT / 2), wn = (wave & 1) * (GT / 2);
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TI; ++j) acc[i][j] = f4_t{0.f, 0.f, 0.f, 0.f};
+  // waves 0, 1 load the rows of A, waves 2, 3 those of B; lane l the piece of row l / 8
+  // that belongs at position l % 8
+  const int row0 = 8 * kWaveLoads * (wave & 1) + (lane >> 3), piece = (lane & 7) ^ (lane >> 3);
+  const uint16_t* src = (wave < 2 ? A + (int64_t)(m0 + row0) * lda : B + (int64_t)(n0 + row0) * ldb) + kb0 + 8 * piece;
+  const int64_t step8 = 8 * (wave < 2 ? lda : ldb);
+  const uint32_t base = lds_addr(&sm[0][0]) + (uint32_t)wave * kWaveLoads * 8 * GT_K * 2;
+  auto issue = [&](int st) {
+    const uint32_t d = base + (uint32_t)(st % GT_RING) * (2 * GT * GT_K * 2);
+#pragma unroll
+    for (int j = 0; j < kWaveLoads; ++j) lds_load16(src + j * step8 + (int64_t)st * GT_K, d + j * 1024);
+  };
+  for (int st = 0; st < GT_RING - 1 && st < nst; ++st) issue(st);
+  for (int st = 0; st < nst; ++st) {
+    // the step has landed (only later steps are still in flight), and the LDS reads of the
+    // step before are done in every wave: its buffer is free for the step GT_RING - 1 ahead
+    const int later = min(nst - 1 - st, GT_RING - 2);
+    if (later >= 2) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(2 * kWaveLoads) : "memory");
+    else if (later == 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kWaveLoads) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (st + GT_RING - 1 < nst) issue(st + GT_RING - 1);
+    const uint16_t* sA = sm[st % GT_RING];
+    const uint16_t* sB = sA + GT * GT_K;
+#pragma unroll
+    for (int kk = 0; kk < GT_K; kk += 32) {
+      bf16x8_t af[TI], bv[TI];
+      const int ko = ((kk / 8 + (lane >> 4)) ^ (lane & 7)) * 8;
+#pragma unroll
+      for (int t = 0; t < TI; ++t) {
+        af[t] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(sA + (wm + 16 * t + (lane & 15)) * GT_K + ko));
+        bv[t] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(sB + (wn + 16 * t + (lane & 15)) * GT_K + ko));
+      }
+#pragma unroll
+      for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TI; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bv[j], acc[i][j], 0, 0, 0);
+    }
+  }
+  static_assert(GT_RING == 3 || GT_RING == 4, "the waits count up to two later steps");
+}
+
+template <int GT, int GT_RING>
 __global__ __launch_bounds__(256) void k_gemm_nt(int M, int N, int K, int kchunk, const uint16_t* __restrict__ A,
                                                  int64_t lda, const uint16_t* __restrict__ B, int64_t ldb,
                                                  float* __restrict__ C) {
-  __shared__ __attribute__((aligned(16))) uint16_t sA[GT_M * G_SLD];
-  __shared__ __attribute__((aligned(16))) uint16_t sB[GT_N * G_SLD];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int n0 = blockIdx.x * GT_N, m0 = blockIdx.y * GT_M;
+  constexpr int TI = gt_tiles<GT>();
+  __shared__ __attribute__((aligned(16))) uint16_t sm[GT_RING][2 * GT * GT_K];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int n0 = blockIdx.x * GT, m0 = blockIdx.y * GT;
   const int kb0 = blockIdx.z * kchunk;
-  const int kend = min(K, kb0 + kchunk);
-  const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
-  f4_t acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f4_t{0.f, 0.f, 0.f, 0.f};
-  // thread t moves the 16-byte vectors t + 256 i (row v / 8, columns 8 (v % 8) ..) of both tiles
-  const int lr = tid >> 3, lc = (tid & 7) * 8;
-  const uint16_t* Ag = A + (int64_t)(m0 + lr) * lda + lc;
-  const uint16_t* Bg = B + (int64_t)(n0 + lr) * ldb + lc;
-  uint4 ra0, ra1, ra2, ra3, rb0, rb1, rb2, rb3;
-#define GEMM_GLOAD(kb)                                                      \
-  do {                                                                      \
-    ra0 = *reinterpret_cast<const uint4*>(Ag + (kb));                       \
-    ra1 = *reinterpret_cast<const uint4*>(Ag + 32 * lda + (kb));            \
-    ra2 = *reinterpret_cast<const uint4*>(Ag + 64 * lda + (kb));            \
-    ra3 = *reinterpret_cast<const uint4*>(Ag + 96 * lda + (kb));            \
-    rb0 = *reinterpret_cast<const uint4*>(Bg + (kb));                       \
-    rb1 = *reinterpret_cast<const uint4*>(Bg + 32 * ldb + (kb));            \
-    rb2 = *reinterpret_cast<const uint4*>(Bg + 64 * ldb + (kb));            \
-    rb3 = *reinterpret_cast<const uint4*>(Bg + 96 * ldb + (kb));            \
-  } while (0)
-  if (kb0 < kend) GEMM_GLOAD(kb0);
-  for (int kb = kb0; kb < kend; kb += GT_K) {
-    __syncthreads();
-    *reinterpret_cast<uint4*>(sA + lr * G_SLD + lc) = ra0;
-    *reinterpret_cast<uint4*>(sA + (lr + 32) * G_SLD + lc) = ra1;
-    *reinterpret_cast<uint4*>(sA + (lr + 64) * G_SLD + lc) = ra2;
-    *reinterpret_cast<uint4*>(sA + (lr + 96) * G_SLD + lc) = ra3;
-    *reinterpret_cast<uint4*>(sB + lr * G_SLD + lc) = rb0;
-    *reinterpret_cast<uint4*>(sB + (lr + 32) * G_SLD + lc) = rb1;
-    *reinterpret_cast<uint4*>(sB + (lr + 64) * G_SLD + lc) = rb2;
-    *reinterpret_cast<uint4*>(sB + (lr + 96) * G_SLD + lc) = rb3;
-    __syncthreads();
-    if (kb + GT_K < kend) GEMM_GLOAD(kb + GT_K);
-#pragma unroll
-    for (int kk = 0; kk < GT_K; kk += 32) {
-      bf16x8_t af[4], bv[4];
-      const int ko = kk + 8 * (lane >> 4);
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        af[t] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(sA + (wm + 16 * t + (lane & 15)) * G_SLD + ko));
-        bv[t] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(sB + (wn + 16 * t + (lane & 15)) * G_SLD + ko));
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bv[j], acc[i][j], 0, 0, 0);
-    }
-  }
-#undef GEMM_GLOAD
+  const int wm = (wave >> 1) * (GT / 2), wn = (wave & 1) * (GT / 2);
+  f4_t acc[TI][TI];
+  gemm_tile<GT, GT_RING>(m0, n0, kb0, (min(K, kb0 + kchunk) - kb0) / GT_K, A, lda, B, ldb, sm, acc);
   // output layout of the 16 x 16 FP32 tile: lane holds rows 4 (lane / 16) + e of column lane % 16
   float* Cs = C + (int64_t)blockIdx.z * M * N;
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < TI; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < TI; ++j)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int m = m0 + wm + 16 * i + 4 * (lane >> 4) + e;
@@ -129,125 +145,133 @@ __global__ __launch_bounds__(256) void k_gemm_nt(int M, int N, int K, int kchunk
 }
 
 // ---------------------------------------------------------------------------------
-// Epilogues over 64 x 64 tiles of an M x N result, 256 threads: thread (c, rg)
-// handles column n0 + c of rows m0 + rg + 4 i.  Transposed copies go through LDS.
-enum { EPI_GELU = 0, EPI_LINEAR = 1, EPI_BWD_GELU = 2 };
+// Epilogues over tiles of 64 rows x 16 columns of an M x N result, 256 threads:
+// thread (c, rg) handles column n0 + c of rows m0 + rg + 16 i.  The partial sums of a
+// thread's four rows are in flight together, and the tile is narrow because the
+// results are small (256 x 1024: 256 workgroups): what bounds the kernel is the latency
+// of its loads.  Transposed copies and column sums go through LDS.  Column sums run
+// over the rows g, g + 4, ... in order for g = 0 .. 3, then over g.
+// (Tiles of 64 x 64 with one row's loads at a time took 15-27 us for 256 x 1024 and
+// 256 x 3456 results, and the loss was a pass of its own, 9 us.)
+enum { EPI_GELU = 0, EPI_BWD_GELU = 1, EPI_LOSS = 2, EPI_OUT = 3 };
 
 struct EpiArgs {
   const float* part;   // [S][M][N] partial sums
   int S, M, N;
   const float* bias;   // [N] (forward)
   const float* zin;    // [M][N] pre-activation (backward)
-  float* zout;         // [M][N] pre-activation (GELU) or output (LINEAR)
+  float* zout;         // [M][N] pre-activation (GELU)
   uint16_t* h;         // [M][N] BF16: GELU(z) or dz
   uint16_t* ht;        // [N][M] BF16 transposed copy
-  float* dbpart;       // [M / 64][N] column sums of dz (backward)
+  float* dbpart;       // [M / 64][N] column sums of dz (backward, loss)
+  // rows of the caller, [mvalid][ld] doubles, nvalid columns: the target Q (LOSS,
+  // t = (float)(q scale), dz = gscale (y - t)) or the output (OUT, q = scale y)
+  double* q;
+  int64_t ld;
+  int mvalid, nvalid;
+  double scale;
+  float gscale;
+  double* losspart;    // LOSS: the tile's sum of squared differences
 };
 
-__global__ __launch_bounds__(256) void k_epilogue(EpiArgs a, int mode) {
-  __shared__ uint16_t tile[64][66];
-  __shared__ float cs[4][64];
-  const int n0 = blockIdx.x * 64, m0 = blockIdx.y * 64;
-  const int c = threadIdx.x & 63, rg = threadIdx.x >> 6;
+// Column tile of a workgroup: workgroups go to the eight XCDs in turn, so each XCD takes a
+// run of neighbouring tiles (gridDim.x is a multiple of 8), whose halves of a 128-byte line meet in its L2
+__device__ __forceinline__ int xcd_column() { return (int)(blockIdx.x % 8) * (int)(gridDim.x / 8) + (int)(blockIdx.x / 8); }
+
+template <int MODE>
+__global__ __launch_bounds__(256) void k_epilogue(EpiArgs a) {
+  constexpr bool DZ = MODE == EPI_BWD_GELU || MODE == EPI_LOSS;
+  __shared__ alignas(8) uint16_t tile[16][68];   // [column][row]; 136-byte rows keep 8-byte reads aligned
+  __shared__ float dzs[DZ ? 64 : 1][17];
+  __shared__ float cs[4][16];
+  __shared__ double red[MODE == EPI_LOSS ? 256 : 1];
+  const int n0 = xcd_column() * 16, m0 = blockIdx.y * 64;
+  const int c = threadIdx.x & 15, rg = threadIdx.x >> 4;
   const int64_t MN = (int64_t)a.M * a.N;
-  float colsum = 0.f;
-  for (int i = 0; i < 16; ++i) {
-    const int r = rg + 4 * i;
-    const int64_t idx = (int64_t)(m0 + r) * a.N + n0 + c;
-    // partials in a fixed order: four running sums (k mod 4), then ((0 + 1) + (2 + 3))
-    float q0 = 0.f, q1 = 0.f, q2 = 0.f, q3 = 0.f;
-    int k = 0;
-    for (; k + 4 <= a.S; k += 4) {
-      q0 += a.part[(int64_t)k * MN + idx];
-      q1 += a.part[(int64_t)(k + 1) * MN + idx];
-      q2 += a.part[(int64_t)(k + 2) * MN + idx];
-      q3 += a.part[(int64_t)(k + 3) * MN + idx];
-    }
-    if (k < a.S) q0 += a.part[(int64_t)k * MN + idx];
-    if (k + 1 < a.S) q1 += a.part[(int64_t)(k + 1) * MN + idx];
-    if (k + 2 < a.S) q2 += a.part[(int64_t)(k + 2) * MN + idx];
-    const float s = (q0 + q1) + (q2 + q3);
-    if (mode == EPI_GELU) {
-      const float z = s + a.bias[n0 + c];
-      a.zout[idx] = z;
-      const uint16_t hb = f2bf(gelu(z));
-      a.h[idx] = hb;
-      tile[c][r] = hb;
-    } else if (mode == EPI_LINEAR) {
-      a.zout[idx] = s + a.bias[n0 + c];
-    } else {
-      const float dz = s * gelu_d(a.zin[idx]);
-      const uint16_t hb = f2bf(dz);
-      a.h[idx] = hb;
-      tile[c][r] = hb;
-      colsum += dz;
-    }
+  int64_t idx[4];
+  float other[4];   // the rows' pre-activations or targets, loaded beside the partial sums
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int m = m0 + rg + 16 * i, n = n0 + c;
+    idx[i] = (int64_t)m * a.N + n;
+    other[i] = 0.f;
+    if constexpr (MODE == EPI_BWD_GELU) other[i] = a.zin[idx[i]];
+    if constexpr (MODE == EPI_LOSS)
+      if (m < a.mvalid && n < a.nvalid) other[i] = (float)(a.q[(int64_t)m * a.ld + n] * a.scale);
   }
-  if (mode == EPI_LINEAR) return;
-  cs[rg][c] = colsum;
-  __syncthreads();
-  for (int i = 0; i < 16; ++i) {
-    const int rr = rg + 4 * i;
-    a.ht[(int64_t)(n0 + rr) * a.M + m0 + c] = tile[rr][c];
-  }
-  if (mode == EPI_BWD_GELU && rg == 0)
-    a.dbpart[(int64_t)blockIdx.y * a.N + n0 + c] = ((cs[0][c] + cs[1][c]) + cs[2][c]) + cs[3][c];
-}
-
-// Mean-squared-error gradient of the output: dz = gscale (y - t) on the valid
-// rows / columns, written as BF16 in both orientations, its column sums, and
-// the tile's sum of squared differences.
-__global__ __launch_bounds__(256) void k_loss(const float* __restrict__ y, const float* __restrict__ t, int M, int N,
-                                              int mvalid, int nvalid, float gscale, uint16_t* __restrict__ dz,
-                                              uint16_t* __restrict__ dzt, float* __restrict__ dbpart,
-                                              double* __restrict__ losspart) {
-  __shared__ uint16_t tile[64][66];
-  __shared__ float cs[4][64];
-  __shared__ double red[256];
-  const int n0 = blockIdx.x * 64, m0 = blockIdx.y * 64;
-  const int c = threadIdx.x & 63, rg = threadIdx.x >> 6;
-  float colsum = 0.f;
+  // partials in a fixed order: four running sums (k mod 4), then ((0 + 1) + (2 + 3))
+  float q[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) q[i][j] = 0.f;
+  int k = 0;
+  for (; k + 4 <= a.S; k += 4)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) q[i][j] += a.part[(int64_t)(k + j) * MN + idx[i]];
+#pragma unroll
+  for (int j = 0; j < 3; ++j)
+    if (k + j < a.S) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) q[i][j] += a.part[(int64_t)(k + j) * MN + idx[i]];
+    }
+  const float bias = DZ && MODE != EPI_LOSS ? 0.f : a.bias[n0 + c];
   double sq = 0.0;
-  for (int i = 0; i < 16; ++i) {
-    const int r = rg + 4 * i;
-    const int64_t idx = (int64_t)(m0 + r) * N + n0 + c;
-    const bool ok = (m0 + r) < mvalid && (n0 + c) < nvalid;
-    const float d = ok ? y[idx] - t[idx] : 0.f;
-    sq += (double)d * (double)d;
-    const float g = gscale * d;
-    const uint16_t hb = f2bf(g);
-    dz[idx] = hb;
-    tile[c][r] = hb;
-    colsum += g;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = rg + 16 * i, m = m0 + r, n = n0 + c;
+    const float s = (q[i][0] + q[i][1]) + (q[i][2] + q[i][3]);
+    if constexpr (MODE == EPI_GELU) {
+      const float z = s + bias;
+      a.zout[idx[i]] = z;
+      const uint16_t hb = f2bf(gelu(z));
+      a.h[idx[i]] = hb;
+      tile[c][r] = hb;
+    } else if constexpr (MODE == EPI_OUT) {
+      const float y = s + bias;
+      if (m < a.mvalid && n < a.nvalid) a.q[(int64_t)m * a.ld + n] = a.scale * (double)y;
+    } else {
+      float dz;
+      if constexpr (MODE == EPI_LOSS) {
+        const float y = s + bias;
+        const float d = (m < a.mvalid && n < a.nvalid) ? y - other[i] : 0.f;
+        sq += (double)d * (double)d;
+        dz = a.gscale * d;
+      } else {
+        dz = s * gelu_d(other[i]);
+      }
+      const uint16_t hb = f2bf(dz);
+      a.h[idx[i]] = hb;
+      tile[c][r] = hb;
+      dzs[r][c] = dz;
+    }
   }
-  cs[rg][c] = colsum;
-  red[threadIdx.x] = sq;
+  if constexpr (MODE == EPI_OUT) return;
+  if constexpr (MODE == EPI_LOSS) red[threadIdx.x] = sq;
   __syncthreads();
-  for (int i = 0; i < 16; ++i) {
-    const int rr = rg + 4 * i;
-    dzt[(int64_t)(n0 + rr) * M + m0 + c] = tile[rr][c];
-  }
-  if (rg == 0) dbpart[(int64_t)blockIdx.y * N + n0 + c] = ((cs[0][c] + cs[1][c]) + cs[2][c]) + cs[3][c];
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+  *reinterpret_cast<uint2*>(a.ht + (int64_t)(n0 + rg) * a.M + m0 + 4 * c) = *reinterpret_cast<const uint2*>(&tile[rg][4 * c]);
+  if constexpr (DZ) {
+    if (rg < 4) {
+      float colsum = dzs[rg][c];
+      for (int i = 1; i < 16; ++i) colsum += dzs[rg + 4 * i][c];
+      cs[rg][c] = colsum;
+    }
     __syncthreads();
+    if (rg == 0) a.dbpart[(int64_t)blockIdx.y * a.N + n0 + c] = ((cs[0][c] + cs[1][c]) + cs[2][c]) + cs[3][c];
   }
-  if (threadIdx.x == 0) losspart[(int64_t)blockIdx.y * gridDim.x + blockIdx.x] = red[0];
+  if constexpr (MODE == EPI_LOSS) {
+    for (int w = 128; w > 0; w >>= 1) {
+      if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) a.losspart[(int64_t)blockIdx.y * gridDim.x + blockIdx.x] = red[0];
+  }
 }
 
-// out[n] = sum_t part[t][n], t in order
-__global__ void k_colsum(const float* __restrict__ part, int T, int N, float* __restrict__ out) {
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= N) return;
-  float s = 0.f;
-  for (int t = 0; t < T; ++t) s += part[(int64_t)t * N + n];
-  out[n] = s;
-}
-
-// one block: out[0] = sum of part[0..n) in a fixed order, times scale
-__global__ __launch_bounds__(256) void k_sum_fixed(const double* __restrict__ part, int n, double scale,
-                                                   double* __restrict__ out) {
-  __shared__ double red[256];
+// out[0] = sum of part[0..n) in a fixed order, times scale, by one workgroup of 256
+__device__ __forceinline__ void sum_fixed(const double* __restrict__ part, int n, double scale, double* red, double* out) {
   double s = 0.0;
   for (int i = threadIdx.x; i < n; i += 256) s += part[i];
   red[threadIdx.x] = s;
@@ -263,30 +287,33 @@ struct AdamArgs {
   float lr, b1, b2, eps, c1, c2;  // c1 = 1 / (1 - b1^t), c2 = 1 / (1 - b2^t)
 };
 
+// The moments' products are contracted explicitly, weights and biases each their way, so
+// that a step's bits do not depend on what the compiler fuses around them.
+template <bool BIAS = false>
 __device__ __forceinline__ float adam_update(float g, float& w, float& m, float& v, const AdamArgs& h) {
-  m = h.b1 * m + (1.f - h.b1) * g;
-  v = h.b2 * v + (1.f - h.b2) * g * g;
+  m = BIAS ? fmaf(h.b1, m, (1.f - h.b1) * g) : fmaf(1.f - h.b1, g, h.b1 * m);
+  v = BIAS ? fmaf(h.b2, v, (1.f - h.b2) * g * g) : fmaf((1.f - h.b2) * g, g, h.b2 * v);
   w = w - h.lr * (m * h.c1) / (sqrtf(v * h.c2) + h.eps);
   return w;
 }
 
-// Adam on a weight matrix [O][I] (64 x 64 tiles; O and I are multiples of 64);
-// writes the master weights, the moments and the BF16 copies Wf [O][I] and
+constexpr int kGradPitch = 68;   // floats per row of a gradient tile in LDS: 16-byte reads aligned, banks spread
+
+// Adam on a 64 x 64 tile of a weight matrix [O][I], its gradient in LDS (and written
+// to G): the master weights, the moments and the BF16 copies Wf [O][I] and
 // Wb [I][O].  A thread owns four consecutive columns of four rows: 16-byte
-// loads and stores, and all sixteen loads in flight before the first update.
-__global__ __launch_bounds__(256) void k_adam_w(int O, int I, const float* __restrict__ G, float* __restrict__ W,
-                                                float* __restrict__ m, float* __restrict__ v,
-                                                uint16_t* __restrict__ Wf, uint16_t* __restrict__ Wb, AdamArgs h) {
-  // [column][row] of the tile's BF16 weights; rows of 68 halves (136 bytes)
-  // keep the 8-byte reads of the transposed write aligned
-  __shared__ alignas(8) uint16_t tile[64][68];
-  const int i0 = blockIdx.x * 64, o0 = blockIdx.y * 64;
+// loads and stores, and all twelve loads in flight before the first update.
+// tile: [column][row] of the tile's BF16 weights; rows of 68 halves (136 bytes)
+// keep the 8-byte reads of the transposed write aligned.
+__device__ __forceinline__ void adam_tile(int i0, int o0, int O, int I, const float* sg, float* __restrict__ G,
+                                          float* __restrict__ W, float* __restrict__ m, float* __restrict__ v,
+                                          uint16_t* __restrict__ Wf, uint16_t* __restrict__ Wb, const AdamArgs& h,
+                                          uint16_t (*tile)[68]) {
   const int c4 = threadIdx.x & 15, rg = threadIdx.x >> 4;   // columns 4 c4 .. 4 c4 + 3, rows rg + 16 k
   float4 g[4], w[4], mm[4], vv[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     const int64_t idx = (int64_t)(o0 + rg + 16 * k) * I + i0 + 4 * c4;
-    g[k] = *reinterpret_cast<const float4*>(G + idx);
     w[k] = *reinterpret_cast<const float4*>(W + idx);
     mm[k] = *reinterpret_cast<const float4*>(m + idx);
     vv[k] = *reinterpret_cast<const float4*>(v + idx);
@@ -295,6 +322,8 @@ __global__ __launch_bounds__(256) void k_adam_w(int O, int I, const float* __res
   for (int k = 0; k < 4; ++k) {
     const int r = rg + 16 * k;
     const int64_t idx = (int64_t)(o0 + r) * I + i0 + 4 * c4;
+    g[k] = *reinterpret_cast<const float4*>(sg + r * kGradPitch + 4 * c4);
+    *reinterpret_cast<float4*>(G + idx) = g[k];
     adam_update(g[k].x, w[k].x, mm[k].x, vv[k].x, h);
     adam_update(g[k].y, w[k].y, mm[k].y, vv[k].y, h);
     adam_update(g[k].z, w[k].z, mm[k].z, vv[k].z, h);
@@ -318,15 +347,77 @@ __global__ __launch_bounds__(256) void k_adam_w(int O, int I, const float* __res
   }
 }
 
-__global__ void k_adam_vec(int n, const float* __restrict__ g, float* __restrict__ w, float* __restrict__ m,
-                           float* __restrict__ v, AdamArgs h) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  float ww = w[i], mm = m[i], vv = v[i];
-  adam_update(g[i], ww, mm, vv, h);
-  w[i] = ww;
-  m[i] = mm;
-  v[i] = vv;
+// A layer's gradient and update, one launch: the workgroups [0, ntile) take 64 x 64
+// tiles of the weights -- the gradient dW = dz^T h over the batch on the matrix cores,
+// kept in G, then Adam -- the next (O + 255) / 256 the bias -- its gradient, the
+// column sums dbpart[t][O] over t in order, then Adam -- and, with losspart, one more
+// adds the loss.  update = 0: gradients only.  Bound by the weights' 32 bytes (weights
+// and moments read and written, gradient and BF16 copies written; 3456 x 1024: 113 MB).
+// (As separate launches the product and Adam took 8 + 18 us at 3456 x 1024 and a gap,
+// the bias sums, bias updates and loss sum 3-4 us each and their gaps, seven times a step
+// of a network with two hidden layers.)
+struct BiasArgs {
+  const float* dbpart;
+  int T;
+  float *g, *w, *m, *v;
+  const double* losspart;
+  int nloss;
+  double loss_scale;
+  double* loss;
+};
+
+__global__ __launch_bounds__(256) void k_grad_update(int O, int I, int K, const uint16_t* __restrict__ dZt,
+                                                     const uint16_t* __restrict__ Ht, float* __restrict__ G,
+                                                     float* __restrict__ W, float* __restrict__ m,
+                                                     float* __restrict__ v, uint16_t* __restrict__ Wf,
+                                                     uint16_t* __restrict__ Wb, int update, AdamArgs h, BiasArgs a) {
+  constexpr int GT = 64, TI = gt_tiles<GT>();
+  __shared__ __attribute__((aligned(16))) uint16_t sm[kGradRing][2 * GT * GT_K];
+  static_assert(sizeof(sm) >= 64 * kGradPitch * sizeof(float) + 64 * 68 * sizeof(uint16_t), "the gradient and weight tiles take the K steps' place");
+  const int ntile = (O / GT) * (I / GT), nb = (O + 255) / 256;
+  const int t = blockIdx.x;
+  if (t < ntile) {
+    const int i0 = t % (I / GT) * GT, o0 = t / (I / GT) * GT;
+    f4_t acc[TI][TI];
+    gemm_tile<GT, kGradRing>(o0, i0, 0, K / GT_K, dZt, K, Ht, K, sm, acc);
+    __syncthreads();   // every wave is done with the K steps
+    float* sg = reinterpret_cast<float*>(&sm[0][0]);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int wm = (wave >> 1) * (GT / 2), wn = (wave & 1) * (GT / 2);
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int j = 0; j < TI; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sg[(wm + 16 * i + 4 * (lane >> 4) + e) * kGradPitch + wn + 16 * j + (lane & 15)] = acc[i][j][e];
+    __syncthreads();
+    if (update) {
+      adam_tile(i0, o0, O, I, sg, G, W, m, v, Wf, Wb, h, reinterpret_cast<uint16_t(*)[68]>(sg + 64 * kGradPitch));
+    } else {
+      const int c4 = threadIdx.x & 15, rg = threadIdx.x >> 4;
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        *reinterpret_cast<float4*>(G + (int64_t)(o0 + rg + 16 * k) * I + i0 + 4 * c4) =
+            *reinterpret_cast<const float4*>(sg + (rg + 16 * k) * kGradPitch + 4 * c4);
+    }
+    return;
+  }
+  if (t < ntile + nb) {
+    const int n = (t - ntile) * 256 + threadIdx.x;
+    if (n >= O) return;
+    float s = 0.f;
+    for (int k = 0; k < a.T; ++k) s += a.dbpart[(int64_t)k * O + n];
+    a.g[n] = s;
+    if (update) {
+      float ww = a.w[n], mm = a.m[n], vv = a.v[n];
+      adam_update<true>(s, ww, mm, vv, h);
+      a.w[n] = ww;
+      a.m[n] = mm;
+      a.v[n] = vv;
+    }
+    return;
+  }
+  sum_fixed(a.losspart, a.nloss, a.loss_scale, reinterpret_cast<double*>(&sm[0][0]), a.loss);
 }
 
 // BF16 copies of master weights [O][I]: Wf [O][I] and Wb [I][O]
@@ -350,44 +441,30 @@ __global__ __launch_bounds__(256) void k_weights_bf16(int O, int I, const float*
 }
 
 // Rows of f (FP64, [nrows][ld]) -> x = f / f_scale as BF16 [Mp][Kp] and [Kp][Mp],
-// zero outside nrows x N.
+// zero outside nrows x N.  Tiles of 64 rows x 16 columns, as the epilogues.
 __global__ __launch_bounds__(256) void k_rows_in(const double* __restrict__ F, int64_t ld, int nrows, int N,
                                                  double inv_scale, int Mp, int Kp, uint16_t* __restrict__ X,
                                                  uint16_t* __restrict__ Xt) {
-  __shared__ uint16_t tile[64][66];
-  const int k0 = blockIdx.x * 64, m0 = blockIdx.y * 64;
-  const int c = threadIdx.x & 63, rg = threadIdx.x >> 6;
-  for (int i = 0; i < 16; ++i) {
-    const int r = rg + 4 * i;
-    const int m = m0 + r, k = k0 + c;
+  __shared__ alignas(8) uint16_t tile[16][68];
+  const int k0 = xcd_column() * 16, m0 = blockIdx.y * 64;
+  const int c = threadIdx.x & 15, rg = threadIdx.x >> 4;
+  const int k = k0 + c;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = rg + 16 * i, m = m0 + r;
     const float x = (m < nrows && k < N) ? (float)(F[(int64_t)m * ld + k] * inv_scale) : 0.f;
     const uint16_t hb = f2bf(x);
     X[(int64_t)m * Kp + k] = hb;
     tile[c][r] = hb;
   }
   __syncthreads();
-  for (int i = 0; i < 16; ++i) {
-    const int rr = rg + 4 * i;
-    Xt[(int64_t)(k0 + rr) * Mp + m0 + c] = tile[rr][c];
-  }
+  *reinterpret_cast<uint2*>(Xt + (int64_t)(k0 + rg) * Mp + m0 + 4 * c) = *reinterpret_cast<const uint2*>(&tile[rg][4 * c]);
 }
 
-// Rows of Q (FP64) -> targets q / q_scale in FP32 [Mp][Np], zero outside
-__global__ void k_rows_target(const double* __restrict__ Q, int64_t ld, int nrows, int N, double inv_scale, int Np,
-                              int64_t total, float* __restrict__ T) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= total) return;
-  const int m = (int)(i / Np), n = (int)(i % Np);
-  T[i] = (m < nrows && n < N) ? (float)(Q[(int64_t)m * ld + n] * inv_scale) : 0.f;
-}
-
-// Output rows: q = q_scale * y in FP64
-__global__ void k_rows_out(const float* __restrict__ Y, int Np, int nrows, int N, double scale,
-                           double* __restrict__ q, int64_t ld) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (int64_t)nrows * N) return;
-  const int m = (int)(i / N), n = (int)(i % N);
-  q[(int64_t)m * ld + n] = scale * (double)Y[(int64_t)m * Np + n];
+// The valid [nrows][n] part of a padded matrix, dense
+__global__ void k_rows_dense(const float* __restrict__ P, int64_t pitch, int64_t n, int64_t total, float* __restrict__ out) {
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x)
+    out[i] = P[i / n * pitch + i % n];
 }
 
 // One block per row: D[m][n] = F[m][n] - fm[n] (D dense, N per row) and
@@ -558,15 +635,13 @@ struct Gemm {
 // Split-K: about 512 workgroups, but at least 8 K steps per workgroup, so that
 // the FP32 partials (S x M x N, summed by the epilogue) stay a small multiple of
 // the output.
-Gemm plan_gemm(int M, int N, int K, bool allow_split) {
+Gemm plan_gemm(int M, int N, int K) {
   Gemm g{M, N, K, 1, K};
-  if (allow_split) {
-    const int tiles = (M / GT_M) * (N / GT_N);
-    const int kt = K / GT_K;
-    int S = std::max(1, std::min(kt / 8, (512 + tiles - 1) / tiles));
-    g.kchunk = ((kt + S - 1) / S) * GT_K;
-    g.S = (K + g.kchunk - 1) / g.kchunk;
-  }
+  const int tiles = (M / GT_PAD) * (N / GT_PAD);
+  const int kt = K / GT_K;
+  const int S = std::max(1, std::min(kt / 8, (512 + tiles - 1) / tiles));
+  g.kchunk = ((kt + S - 1) / S) * GT_K;
+  g.S = (K + g.kchunk - 1) / g.kchunk;
   return g;
 }
 
@@ -579,15 +654,13 @@ struct dgv_surrogate {
   std::vector<SurLayer> layers;
   std::vector<uint16_t*> H, Ht;  // H[l]: input of layer l, BF16 [Bp][inp_l] and [inp_l][Bp]
   std::vector<float*> Z;         // Z[l], l < L-1: pre-activation [Bp][outp_l]
-  float* Y = nullptr;            // [Bp][outp_{L-1}]
-  float* T = nullptr;
   uint16_t* dZ[2] = {nullptr, nullptr};
   uint16_t* dZt[2] = {nullptr, nullptr};
   float* part = nullptr;
   int64_t part_elems = 0;
-  float* dbpart = nullptr;
+  float* dbpart[2] = {nullptr, nullptr};   // column sums of dz, of the layer and of the one before it
   double* losspart = nullptr;
-  double* d_loss = nullptr;
+  double* h_loss = nullptr;                // pinned: the kernel that adds the loss writes it there
   int64_t step = 0;
   double f_scale = 1.0, q_scale = 1.0;
   Chol5 chol{};
@@ -619,36 +692,50 @@ int serr(dgv_surrogate* s, int code, const std::string& m) {
     if (e_ != hipSuccess) return serr((s), DGV_ERR_HIP, std::string(#call) + ": " + hipGetErrorString(e_)); \
   } while (0)
 
+constexpr int64_t kSmallTiles = 512;
+
 int launch_gemm(dgv_surrogate* s, const Gemm& g, const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb,
                 float* C) {
-  if (g.M % GT_M || g.N % GT_N || g.K % GT_K || g.kchunk % GT_K || lda % 8 || ldb % 8 || lda < g.K || ldb < g.K)
+  if (g.M % GT_PAD || g.N % GT_PAD || g.K % GT_K || g.kchunk % GT_K || lda % 8 || ldb % 8 || lda < g.K || ldb < g.K)
     return serr(s, DGV_ERR_ARG, "matrix product shape does not fit the tiling");
-  hipLaunchKernelGGL(k_gemm_nt, dim3(g.N / GT_N, g.M / GT_M, g.S), dim3(256), 0, s->ctx->stream, g.M, g.N, g.K,
-                     g.kchunk, A, lda, B, ldb, C);
+  // tiles of 64 while they fit two to a CU at once, else the 128 that read half as much
+  // (forward pass of 64 rows, 729-300-300-729: 0.029 ms with 64, 0.038 with 128; 256 rows,
+  // 3375-1024-1024-3375: 0.052 and 0.057; 1024 rows, 19683-2048-2048-19683: 0.643 and 0.530.
+  // With tiles of 128, one K step in flight and the older epilogues: 0.071, 0.108, 0.576)
+  const int64_t n64 = (int64_t)(g.N / 64) * (g.M / 64) * g.S;
+  if (n64 <= kSmallTiles)
+    hipLaunchKernelGGL((k_gemm_nt<64, 4>), dim3(g.N / 64, g.M / 64, g.S), dim3(256), 0, s->ctx->stream, g.M, g.N, g.K,
+                       g.kchunk, A, lda, B, ldb, C);
+  else
+    hipLaunchKernelGGL((k_gemm_nt<128, 4>), dim3(g.N / 128, g.M / 128, g.S), dim3(256), 0, s->ctx->stream, g.M, g.N,
+                       g.K, g.kchunk, A, lda, B, ldb, C);
   return DGV_OK;
 }
 
-int forward(dgv_surrogate* s) {
+// the network on the loaded rows; the last layer's epilogue is out's (LOSS or OUT)
+int forward(dgv_surrogate* s, EpiArgs out, int out_mode) {
   hipStream_t st = s->ctx->stream;
   for (int l = 0; l < s->L; ++l) {
     const SurLayer& ly = s->layers[l];
-    const Gemm g = plan_gemm(s->Bp, ly.outp, ly.inp, true);
+    const Gemm g = plan_gemm(s->Bp, ly.outp, ly.inp);
     int rc = launch_gemm(s, g, s->H[l], ly.inp, ly.Wf, ly.inp, s->part);
     if (rc) return rc;
-    EpiArgs a{};
+    EpiArgs a = l + 1 < s->L ? EpiArgs{} : out;
     a.part = s->part;
     a.S = g.S;
     a.M = s->Bp;
     a.N = ly.outp;
     a.bias = ly.b;
+    const dim3 grid(ly.outp / 16, s->Bp / 64);
     if (l + 1 < s->L) {
       a.zout = s->Z[l];
       a.h = s->H[l + 1];
       a.ht = s->Ht[l + 1];
-      hipLaunchKernelGGL(k_epilogue, dim3(ly.outp / 64, s->Bp / 64), dim3(256), 0, st, a, (int)EPI_GELU);
+      hipLaunchKernelGGL(k_epilogue<EPI_GELU>, grid, dim3(256), 0, st, a);
+    } else if (out_mode == EPI_LOSS) {
+      hipLaunchKernelGGL(k_epilogue<EPI_LOSS>, grid, dim3(256), 0, st, a);
     } else {
-      a.zout = s->Y;
-      hipLaunchKernelGGL(k_epilogue, dim3(ly.outp / 64, s->Bp / 64), dim3(256), 0, st, a, (int)EPI_LINEAR);
+      hipLaunchKernelGGL(k_epilogue<EPI_OUT>, grid, dim3(256), 0, st, a);
     }
   }
   SHIP(s, hipGetLastError());
@@ -657,7 +744,7 @@ int forward(dgv_surrogate* s) {
 
 int load_rows(dgv_surrogate* s, const double* d_f, int64_t ld, int nrows) {
   const SurLayer& l0 = s->layers[0];
-  hipLaunchKernelGGL(k_rows_in, dim3(l0.inp / 64, s->Bp / 64), dim3(256), 0, s->ctx->stream, d_f, ld, nrows, l0.in,
+  hipLaunchKernelGGL(k_rows_in, dim3(l0.inp / 16, s->Bp / 64), dim3(256), 0, s->ctx->stream, d_f, ld, nrows, l0.in,
                      1.0 / s->f_scale, s->Bp, l0.inp, s->H[0], s->Ht[0]);
   SHIP(s, hipGetLastError());
   return DGV_OK;
@@ -668,11 +755,13 @@ int load_rows(dgv_surrogate* s, const double* d_f, int64_t ld, int nrows) {
 int predict_chunk(dgv_surrogate* s, const double* d_f, int64_t ld, int nrows, double* d_q, int project) {
   int rc = load_rows(s, d_f, ld, nrows);
   if (rc) return rc;
-  if ((rc = forward(s))) return rc;
-  const SurLayer& lo = s->layers[s->L - 1];
-  const int64_t n = (int64_t)nrows * lo.out;
-  hipLaunchKernelGGL(k_rows_out, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s->ctx->stream, s->Y, lo.outp,
-                     nrows, lo.out, s->q_scale, d_q, ld);
+  EpiArgs a{};
+  a.q = d_q;
+  a.ld = ld;
+  a.mvalid = nrows;
+  a.nvalid = s->layers[s->L - 1].out;
+  a.scale = s->q_scale;
+  if ((rc = forward(s, a, EPI_OUT))) return rc;
   if (project) {
     const dgv_ctx* c = s->ctx;
     hipLaunchKernelGGL(k_project_rows, dim3(nrows), dim3(256), 0, c->stream, d_q, ld, (int)c->g.N, c->d_u, c->d_v,
@@ -727,9 +816,8 @@ void free_surrogate(dgv_surrogate* s) {
   for (auto p : s->H) hipFree(p);
   for (auto p : s->Ht) hipFree(p);
   for (auto p : s->Z) hipFree(p);
-  hipFree(s->Y); hipFree(s->T);
   for (int i = 0; i < 2; ++i) { hipFree(s->dZ[i]); hipFree(s->dZt[i]); }
-  hipFree(s->part); hipFree(s->dbpart); hipFree(s->losspart); hipFree(s->d_loss);
+  hipFree(s->part); hipFree(s->dbpart[0]); hipFree(s->dbpart[1]); hipFree(s->losspart); hipHostFree(s->h_loss);
   hipFree(s->d_probe_nodes); hipFree(s->d_res);
   hipFree(s->d_df); hipFree(s->d_lin); hipFree(s->d_qfm); hipFree(s->d_rs);
   if (s->judge) dgv_batch_destroy(s->judge);
@@ -791,8 +879,8 @@ int dgv_sur_create(dgv_ctx* ctx, const int32_t* widths, int32_t nlayers, int32_t
       return fail(DGV_ERR_HIP, "surrogate initialisation failed");
     hipLaunchKernelGGL(k_weights_bf16, dim3(ly.inp / 64, ly.outp / 64), dim3(256), 0, ctx->stream, ly.outp, ly.inp,
                        ly.W, ly.Wf, ly.Wb);
-    const Gemm f = plan_gemm(s->Bp, ly.outp, ly.inp, true);
-    const Gemm d = plan_gemm(s->Bp, ly.inp, ly.outp, true);
+    const Gemm f = plan_gemm(s->Bp, ly.outp, ly.inp);
+    const Gemm d = plan_gemm(s->Bp, ly.inp, ly.outp);
     s->part_elems = std::max({s->part_elems, (int64_t)f.S * f.M * f.N, (int64_t)d.S * d.M * d.N});
   }
   s->H.assign(nlayers, nullptr);
@@ -805,13 +893,14 @@ int dgv_sur_create(dgv_ctx* ctx, const int32_t* widths, int32_t nlayers, int32_t
     if (l + 1 < nlayers && !dalloc((void**)&s->Z[l], 4 * (size_t)s->Bp * s->layers[l].outp))
       return fail(DGV_ERR_NOMEM, "hipMalloc(activations) failed");
   }
-  const size_t nout = (size_t)s->Bp * s->layers[nlayers - 1].outp;
   const size_t nmax = (size_t)s->Bp * maxw;
-  bool ok = dalloc((void**)&s->Y, 4 * nout) && dalloc((void**)&s->T, 4 * nout) && dalloc((void**)&s->dZ[0], 2 * nmax) &&
+  bool ok = dalloc((void**)&s->dZ[0], 2 * nmax) &&
             dalloc((void**)&s->dZ[1], 2 * nmax) && dalloc((void**)&s->dZt[0], 2 * nmax) &&
             dalloc((void**)&s->dZt[1], 2 * nmax) && dalloc((void**)&s->part, 4 * (size_t)s->part_elems) &&
-            dalloc((void**)&s->dbpart, 4 * (size_t)(s->Bp / 64) * maxw) &&
-            dalloc((void**)&s->losspart, 8 * (size_t)(s->Bp / 64) * (maxw / 64)) && dalloc((void**)&s->d_loss, 8) &&
+            dalloc((void**)&s->dbpart[0], 4 * (size_t)(s->Bp / 64) * maxw) &&
+            dalloc((void**)&s->dbpart[1], 4 * (size_t)(s->Bp / 64) * maxw) &&
+            dalloc((void**)&s->losspart, 8 * (size_t)(s->Bp / 64) * (maxw / 16)) &&
+            hipHostMalloc((void**)&s->h_loss, sizeof(double), 0) == hipSuccess &&
             dalloc((void**)&s->d_res, 8 * (size_t)s->Bp);
   if (!ok) return fail(DGV_ERR_NOMEM, "hipMalloc(surrogate buffers) failed");
   if (hipGetLastError() != hipSuccess || hipStreamSynchronize(ctx->stream) != hipSuccess)
@@ -857,7 +946,21 @@ static int layer_copy(dgv_surrogate* s, int32_t layer, float* W, float* b, const
     if (W) SHIP(s, hipMemcpy2DAsync(const_cast<float*>(Wd), pitch, W, rowb, rowb, ly.out, hipMemcpyHostToDevice, st));
     if (b) SHIP(s, hipMemcpyAsync(const_cast<float*>(bd), b, sizeof(float) * ly.out, hipMemcpyHostToDevice, st));
   } else {
-    if (W) SHIP(s, hipMemcpy2DAsync(W, rowb, Wd, pitch, rowb, ly.out, hipMemcpyDeviceToHost, st));
+    // rows without padding are one copy; padded ones are made dense on the device first,
+    // as many at a time as the partial sums' buffer holds (a pitched copy of 1024 x 3375
+    // weights took 38 ms)
+    const int64_t rows = pitch == rowb ? ly.out : std::min<int64_t>(ly.out, s->part_elems / ly.in);
+    for (int64_t r = 0; W && r < ly.out; r += rows) {
+      const int64_t n = std::min<int64_t>(rows, ly.out - r) * ly.in;
+      const float* src = Wd + r * ly.inp;
+      if (pitch != rowb) {
+        hipLaunchKernelGGL(k_rows_dense, dim3(stride_blocks(n, 256)), dim3(256), 0, st, src, (int64_t)ly.inp,
+                           (int64_t)ly.in, n, s->part);
+        SHIP(s, hipGetLastError());
+        src = s->part;
+      }
+      SHIP(s, hipMemcpyAsync(W + r * ly.in, src, sizeof(float) * n, hipMemcpyDeviceToHost, st));
+    }
     if (b) SHIP(s, hipMemcpyAsync(b, bd, sizeof(float) * ly.out, hipMemcpyDeviceToHost, st));
   }
   SHIP(s, hipStreamSynchronize(st));
@@ -897,16 +1000,20 @@ int dgv_sur_train_step(dgv_surrogate* s, const double* d_f, const double* d_q, i
   int rc = load_rows(s, d_f, ld, nrows);
   if (rc) return rc;
   const SurLayer& lo = s->layers[s->L - 1];
-  const int64_t nt = (int64_t)s->Bp * lo.outp;
-  hipLaunchKernelGGL(k_rows_target, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, st, d_q, ld, nrows, lo.out,
-                     1.0 / s->q_scale, lo.outp, nt, s->T);
-  if ((rc = forward(s))) return rc;
   const double inv_count = 1.0 / ((double)nrows * lo.out);
-  const int nlp = (lo.outp / 64) * (s->Bp / 64);
   int cur = 0;
-  hipLaunchKernelGGL(k_loss, dim3(lo.outp / 64, s->Bp / 64), dim3(256), 0, st, s->Y, s->T, s->Bp, lo.outp, nrows,
-                     lo.out, (float)(2.0 * inv_count), s->dZ[cur], s->dZt[cur], s->dbpart, s->losspart);
-  hipLaunchKernelGGL(k_sum_fixed, dim3(1), dim3(256), 0, st, s->losspart, nlp, inv_count, s->d_loss);
+  EpiArgs e{};
+  e.q = const_cast<double*>(d_q);
+  e.ld = ld;
+  e.mvalid = nrows;
+  e.nvalid = lo.out;
+  e.scale = 1.0 / s->q_scale;
+  e.gscale = (float)(2.0 * inv_count);
+  e.h = s->dZ[cur];
+  e.ht = s->dZt[cur];
+  e.dbpart = s->dbpart[cur];
+  e.losspart = s->losspart;
+  if ((rc = forward(s, e, EPI_LOSS))) return rc;
   ++s->step;
   AdamArgs h;
   h.lr = (float)lr;
@@ -917,9 +1024,8 @@ int dgv_sur_train_step(dgv_surrogate* s, const double* d_f, const double* d_q, i
   h.c2 = (float)(1.0 / (1.0 - std::pow(0.999, (double)s->step)));
   for (int l = s->L - 1; l >= 0; --l) {
     SurLayer& ly = s->layers[l];
-    hipLaunchKernelGGL(k_colsum, dim3((ly.outp + 255) / 256), dim3(256), 0, st, s->dbpart, s->Bp / 64, ly.outp, ly.gb);
     if (l > 0) {  // gradient of the layer's input, through GELU of the previous layer
-      const Gemm g = plan_gemm(s->Bp, ly.inp, ly.outp, true);
+      const Gemm g = plan_gemm(s->Bp, ly.inp, ly.outp);
       if ((rc = launch_gemm(s, g, s->dZ[cur], ly.outp, ly.Wb, ly.outp, s->part))) return rc;
       EpiArgs a{};
       a.part = s->part;
@@ -929,23 +1035,21 @@ int dgv_sur_train_step(dgv_surrogate* s, const double* d_f, const double* d_q, i
       a.zin = s->Z[l - 1];
       a.h = s->dZ[cur ^ 1];
       a.ht = s->dZt[cur ^ 1];
-      a.dbpart = s->dbpart;
-      hipLaunchKernelGGL(k_epilogue, dim3(ly.inp / 64, s->Bp / 64), dim3(256), 0, st, a, (int)EPI_BWD_GELU);
+      a.dbpart = s->dbpart[cur ^ 1];
+      hipLaunchKernelGGL(k_epilogue<EPI_BWD_GELU>, dim3(ly.inp / 16, s->Bp / 64), dim3(256), 0, st, a);
     }
-    const Gemm gw = plan_gemm(ly.outp, ly.inp, s->Bp, false);
-    if ((rc = launch_gemm(s, gw, s->dZt[cur], s->Bp, s->Ht[l], s->Bp, ly.G))) return rc;
-    if (lr > 0) {
-      hipLaunchKernelGGL(k_adam_w, dim3(ly.inp / 64, ly.outp / 64), dim3(256), 0, st, ly.outp, ly.inp, ly.G, ly.W,
-                         ly.mW, ly.vW, ly.Wf, ly.Wb, h);
-      hipLaunchKernelGGL(k_adam_vec, dim3((ly.outp + 255) / 256), dim3(256), 0, st, ly.outp, ly.gb, ly.b, ly.mb,
-                         ly.vb, h);
-    }
+    const bool last = l + 1 == s->L;   // its launch adds the loss too
+    const BiasArgs ba{s->dbpart[cur], s->Bp / 64, ly.gb, ly.b, ly.mb, ly.vb, s->losspart,
+                      (lo.outp / 16) * (s->Bp / 64), inv_count, s->h_loss};
+    const int nwg = (ly.inp / 64) * (ly.outp / 64) + (ly.outp + 255) / 256 + (last ? 1 : 0);
+    hipLaunchKernelGGL(k_grad_update, dim3((unsigned)nwg), dim3(256), 0, st, ly.outp, ly.inp, s->Bp, s->dZt[cur],
+                       s->Ht[l], ly.G, ly.W, ly.mW, ly.vW, ly.Wf, ly.Wb, lr > 0 ? 1 : 0, h, ba);
     cur ^= 1;
   }
   SHIP(s, hipGetLastError());
   if (loss) {
-    SHIP(s, hipMemcpyAsync(loss, s->d_loss, sizeof(double), hipMemcpyDeviceToHost, st));
     SHIP(s, hipStreamSynchronize(st));
+    *loss = *(volatile double*)s->h_loss;
   }
   return DGV_OK;
 }
