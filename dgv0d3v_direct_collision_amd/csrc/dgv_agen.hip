@@ -14,7 +14,8 @@
 //                  (p, q) and each cp's table (p, q) -> pair
 //   3. k_integrate: one thread per main diagonal, S_l (dgv_agen_math.h), then for
 //                  each pair of the box the D values of A: min_sens test, weights
-//                  and |g|/8                                             -> pairs
+//                  and |g|/8                                             -> pairs;
+//                  k_integrate_marked the few spheres whose records hang on rounding
 //   4. k_kept + host scan + k_compact: drop pairs whose D values are all zero and
 //                  emit per-cp segment tables (the block headers)
 #include <algorithm>
@@ -63,16 +64,23 @@ static int make_consts(const Grid& g, const dgv_agen_params& p, AgenConsts& C, s
   for (int d = 0; d < 3; ++d) {
     for (int i = 0; i < s[d]; ++i) C.kap[d][i] = g.gn[d][i];
     lagrange_monomials(C.kap[d], s[d], C.mono[d]);
+    if (d < 2) std::memcpy(C.monol[d], C.mono[d], sizeof(C.mono[d]));
+    const double h = 0.5 * (d == 0 ? C.u1 - C.u0 : d == 1 ? C.v1 - C.v0 : C.w1 - C.w0);
+    for (int i = 0; i < s[d]; ++i)
+      for (int m = 1; m < s[d]; ++m) C.mono[d][i][m] /= std::pow(h, m);
   }
   int nq = p.nquad > 0 ? p.nquad : 24;
   if (nq > kAgenMaxQ) { err = "nquad too large (max 48)"; return DGV_ERR_ARG; }
   C.nq = nq;
   std::vector<double> x(nq), w(nq);
   if (gauss_legendre(nq, x.data(), w.data())) { err = "Gauss-Legendre failed"; return DGV_ERR_ARG; }
-  const double pi = 3.141592653589793238462643383279502884;
+  const long double pi = 3.141592653589793238462643383279502884L;
   for (int i = 0; i < nq; ++i) {
-    C.qs[i] = 0.5 * pi * (x[i] + 1.0);
-    C.qw[i] = 0.5 * pi * w[i];
+    C.qs[i] = 0.5 * (double)pi * (x[i] + 1.0);
+    C.qv[i] = 0.5 * (double)pi * w[i];
+    const long double a = 0.5L * pi * (1.0L + x[i]);
+    C.qx[i] = (double)(1.0L - std::cos(a));
+    C.qw[i] = (double)(0.5L * pi * w[i] * std::sin(a));
   }
   C.Trad = p.Trad > 0 ? p.Trad : 100.0;
   C.moment_mode = p.moment_mode;
@@ -172,30 +180,49 @@ __global__ __launch_bounds__(64) void k_list(AgenConsts C, CellDims dims, const 
   }
 }
 
-// One thread per main diagonal.  FP64 transcendental arithmetic bounds it (up to 19
-// smooth pieces of 24 points, each with up to eight arc ends): 85 ms at 15^3 nodes
-// (3.2 M pairs) with one integration per pair, 26 ms with one per box.
+// The spheres' inputs: main diagonal k of the list
+// (kPointwise set in the entry: integrate it point by point)
+constexpr uint64_t kPointwise = (uint64_t)1 << 63;
+struct Mains {
+  const int2* cps;
+  uint64_t* list;
+};
+struct Main {
+  int2 XY;
+  int p, q;
+  double cen[3], dsph;
+};
 template <int SU, int SV, int SW>
-__global__ __launch_bounds__(128) void k_integrate(AgenConsts C, CellDims dims, int64_t nmain,
-                                                   const int2* __restrict__ cps, NodeGeo G,
-                                                   const uint64_t* __restrict__ mains,
-                                                   const int64_t* __restrict__ off, const int16_t* __restrict__ rank,
-                                                   double min_sens, double* __restrict__ pairs,
-                                                   uint8_t* __restrict__ keep) {
+__device__ __forceinline__ Main main_of(const AgenConsts& C, const Mains& M, const NodeGeo& G, int64_t k) {
   constexpr int D = SU * SV * SW;
-  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= nmain) return;
-  const uint64_t e = mains[k];
-  const int p = (int)((e >> 8) & 255), q = (int)(e & 255);
-  const int2 XY = cps[e >> 16];
-  const int64_t i0 = (int64_t)XY.x * D + p, j0 = (int64_t)XY.y * D + q;
+  Main m;
+  const uint64_t e = M.list[k] & ~kPointwise;
+  m.p = (int)((e >> 8) & 255);
+  m.q = (int)(e & 255);
+  m.XY = M.cps[e >> 16];
+  const int64_t i0 = (int64_t)m.XY.x * D + m.p, j0 = (int64_t)m.XY.y * D + m.q;
   const double lo[3] = {G.u[i0], G.v[i0], G.w[i0]}, hi[3] = {G.u[j0], G.v[j0], G.w[j0]};
-  const double dsph = pair_distance(C, lo, hi);
-  double S[D];
-  if (C.moment_mode == 0) {
-    const double cen[3] = {0.5 * (lo[0] + hi[0]), 0.5 * (lo[1] + hi[1]), 0.5 * (lo[2] + hi[2])};
-    sphere_integrals<SU, SV, SW>(C, cen, 0.5 * dsph, S);
-  }
+  m.dsph = pair_distance(C, lo, hi);
+  for (int d = 0; d < 3; ++d) m.cen[d] = 0.5 * (lo[d] + hi[d]);
+  return m;
+}
+
+// Diagonal z of a main diagonal's box, if it is one: the pair's D values of A.  Returns
+// whether one of them is too close to the cutoff for its side of it to be certain.
+struct PairsOut {
+  const int64_t* off;
+  const int16_t* rank;
+  double min_sens;
+  double* pairs;
+  uint8_t* keep;
+};
+template <int SU, int SV, int SW>
+__device__ __forceinline__ bool write_diagonal(const AgenConsts& C, const CellDims& dims, const NodeGeo& G, const PairsOut& O,
+                                               const Main& m, const double* S, int z) {
+  constexpr int D = SU * SV * SW;
+  const int2 XY = m.XY;
+  const int p = m.p, q = m.q;
+  const double dsph = m.dsph;
   // the box's corners: cell and local coordinates of the low and the high one
   const int lc[3] = {XY.x / (dims.Mv * dims.Mw), XY.x / dims.Mw % dims.Mv, XY.x % dims.Mw};
   const int hc[3] = {XY.y / (dims.Mv * dims.Mw), XY.y / dims.Mw % dims.Mv, XY.y % dims.Mw};
@@ -203,47 +230,112 @@ __global__ __launch_bounds__(128) void k_integrate(AgenConsts C, CellDims dims, 
   int differ = 0;
   for (int d = 0; d < 3; ++d) differ |= (lc[d] != hc[d] || ll[d] != hl[d]) << d;
   const int flips = differ & (differ - 1);   // the first dimension that differs stays: each diagonal once
-  for (int z = 0; z < 8; ++z) {
-    if (z & ~flips) continue;
-    int ac[3], al[3], bc[3], bl[3];   // the diagonal's ends: `a` takes the high corner where bit d of z is set
-    for (int d = 0; d < 3; ++d) {
-      const bool f = (z >> d) & 1;
-      ac[d] = f ? hc[d] : lc[d]; al[d] = f ? hl[d] : ll[d];
-      bc[d] = f ? lc[d] : hc[d]; bl[d] = f ? ll[d] : hl[d];
+  if (z & ~flips) return false;
+  int ac[3], al[3], bc[3], bl[3];   // the diagonal's ends: `a` takes the high corner where bit d of z is set
+  for (int d = 0; d < 3; ++d) {
+    const bool f = (z >> d) & 1;
+    ac[d] = f ? hc[d] : lc[d]; al[d] = f ? hl[d] : ll[d];
+    bc[d] = f ? lc[d] : hc[d]; bl[d] = f ? ll[d] : hl[d];
+  }
+  int X = (ac[0] * dims.Mv + ac[1]) * dims.Mw + ac[2], Y = (bc[0] * dims.Mv + bc[1]) * dims.Mw + bc[2];
+  int P = (al[0] * SV + al[1]) * SW + al[2], Q = (bl[0] * SV + bl[1]) * SW + bl[2];
+  if (X > Y || (X == Y && P > Q)) {   // xi < xi1 in node order
+    const int t = X, u = P;
+    X = Y; Y = t;
+    P = Q; Q = u;
+  }
+  const int64_t cp = (int64_t)X * dims.nc - (int64_t)X * (X - 1) / 2 + (Y - X);
+  const int64_t at = O.off[cp] + O.rank[cp * (D * D) + P * D + Q];
+  const int64_t i = (int64_t)X * D + P, j = (int64_t)Y * D + Q;
+  const double x[3] = {G.u[i], G.v[i], G.w[i]}, y[3] = {G.u[j], G.v[j], G.w[j]};
+  double raw[D];
+  if (C.moment_mode == 0) {
+    raw_from_sphere<SU, SV, SW>(C, x, y, S, raw);
+  } else {
+    const double v = raw_moment(C.moment_mode, x, y, 0.5 * dsph);
+    for (int l = 0; l < D; ++l) raw[l] = v;
+  }
+  const double wi = G.gwts[i], wj = G.gwts[j];
+  double* out = O.pairs + at * (D + 1);
+  bool any = false, near = false;
+  for (int l = 0; l < D; ++l) {
+    near = near || near_cutoff(raw[l], O.min_sens);
+    double a = 0.0;
+    if (fabs(raw[l]) > O.min_sens) {  // line 641, then lines 654-659
+      a = raw[l] * wj;
+      a = a * wi;
+      a = a * (dsph / 8.0);
+      any = true;
     }
-    int X = (ac[0] * dims.Mv + ac[1]) * dims.Mw + ac[2], Y = (bc[0] * dims.Mv + bc[1]) * dims.Mw + bc[2];
-    int P = (al[0] * SV + al[1]) * SW + al[2], Q = (bl[0] * SV + bl[1]) * SW + bl[2];
-    if (X > Y || (X == Y && P > Q)) {   // xi < xi1 in node order
-      const int t = X, u = P;
-      X = Y; Y = t;
-      P = Q; Q = u;
+    out[l] = a;
+  }
+  out[D] = __longlong_as_double((long long)pair_code_bits(P, Q));
+  O.keep[at] = any ? 1 : 0;
+  return near;
+}
+
+// One thread per main diagonal.  FP64 arithmetic bounds it: up to 19 smooth pieces of 24
+// points, each with up to four crossed lines (an inverse sine, a square root and the
+// antiderivatives each).  26 ms at 15^3 nodes (0.86 M spheres, 3.2 M pairs) with the arcs
+// searched, and their ends' sines and cosines taken, at every point; 3.7 ms (and 0.7 for
+// the marked ones) with the arcs' ends known per piece.
+// Spheres that have to be integrated point by point are marked for k_integrate_marked.
+template <int SU, int SV, int SW>
+__global__ __launch_bounds__(128) void k_integrate(AgenConsts C, CellDims dims, int64_t nmain, Mains M, NodeGeo G,
+                                                   PairsOut O) {
+  constexpr int D = SU * SV * SW;
+  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= nmain) return;
+  const Main m = main_of<SU, SV, SW>(C, M, G, k);
+  double S[D];
+  bool hit = false;
+  if (C.moment_mode == 0) {
+    if (grazing(C, m.cen, 0.5 * m.dsph)) {
+      M.list[k] |= kPointwise;
+      return;
     }
-    const int64_t cp = (int64_t)X * dims.nc - (int64_t)X * (X - 1) / 2 + (Y - X);
-    const int64_t at = off[cp] + rank[cp * (D * D) + P * D + Q];
-    const int64_t i = (int64_t)X * D + P, j = (int64_t)Y * D + Q;
-    const double x[3] = {G.u[i], G.v[i], G.w[i]}, y[3] = {G.u[j], G.v[j], G.w[j]};
-    double raw[D];
-    if (C.moment_mode == 0) {
-      raw_from_sphere<SU, SV, SW>(C, x, y, S, raw);
-    } else {
-      const double v = raw_moment(C.moment_mode, x, y, 0.5 * dsph);
-      for (int l = 0; l < D; ++l) raw[l] = v;
-    }
-    const double wi = G.gwts[i], wj = G.gwts[j];
-    double* out = pairs + at * (D + 1);
-    bool any = false;
-    for (int l = 0; l < D; ++l) {
-      double a = 0.0;
-      if (fabs(raw[l]) > min_sens) {  // line 641, then lines 654-659
-        a = raw[l] * wj;
-        a = a * wi;
-        a = a * (dsph / 8.0);
-        any = true;
+    sphere_integrals<SU, SV, SW>(C, m.cen, 0.5 * m.dsph, S);
+#pragma unroll
+    for (int l = 0; l < D; ++l) hit = hit || S[l] != 0.0;
+  }
+  bool near = false;
+  for (int z = 0; z < 8; ++z) near = write_diagonal<SU, SV, SW>(C, dims, G, O, m, S, z) || near;
+  if (hit && near) M.list[k] |= kPointwise;
+}
+
+// The marked ones: a wave looks through kMarkedRun main diagonals and takes the marked
+// ones among them one after the other, its lanes the points of all pieces (a lane per
+// sphere would wait 4 ms for the slowest); each basis function's sum then runs over the
+// points in order, in one lane.
+constexpr int kMarkedRun = 256;
+template <int SU, int SV, int SW>
+__global__ __launch_bounds__(64) void k_integrate_marked(AgenConsts C, CellDims dims, int64_t nmain, Mains M, NodeGeo G,
+                                                          PairsOut O) {
+  constexpr int D = SU * SV * SW, F = SU * SV + SW;
+  static_assert(D <= 64, "a lane per basis function");
+  __shared__ double pt[F][64 + 1];
+  const int lane = threadIdx.x;
+  for (int64_t k0 = (int64_t)blockIdx.x * kMarkedRun; k0 < min(nmain, ((int64_t)blockIdx.x + 1) * kMarkedRun); k0 += 64) {
+    const bool mine = k0 + lane < nmain && (M.list[k0 + lane] & kPointwise) != 0;
+    for (uint64_t todo = __ballot(mine); todo != 0; todo &= todo - 1) {
+      const Main m = main_of<SU, SV, SW>(C, M, G, k0 + __builtin_ctzll(todo));
+      const double r = 0.5 * m.dsph;
+      double bp[20], sum = 0.0, S[D];
+      const int nb = sphere_pieces(C, m.cen, r, bp), npt = nb > 1 ? (nb - 1) * C.nq : 0;
+      for (int t0 = 0; t0 < npt; t0 += 64) {
+        const int t = t0 + lane, p = min(t / C.nq, max(nb - 2, 0));
+        double f[F];
+        if (!(t < npt && bp[p + 1] > bp[p] && grazing_point<SU, SV, SW>(C, m.cen, r, bp[p], bp[p + 1], t - p * C.nq, f)))
+          for (int i = 0; i < F; ++i) f[i] = 0.0;
+        for (int i = 0; i < F; ++i) pt[i][lane] = f[i];
+        __syncthreads();
+        if (lane < D)
+          for (int i = 0; i < 64; ++i) sum += pt[SU * SV + lane % SW][i] * pt[lane / SW][i];
+        __syncthreads();
       }
-      out[l] = a;
+      for (int l = 0; l < D; ++l) S[l] = __shfl(sum, l);
+      if (lane < 8) write_diagonal<SU, SV, SW>(C, dims, G, O, m, S, lane);
     }
-    out[D] = __longlong_as_double((long long)pair_code_bits(P, Q));
-    keep[at] = any ? 1 : 0;
   }
 }
 
@@ -381,12 +473,16 @@ static int generate_t(dgv_ctx* ctx, const AgenConsts& C, double min_sens) {
   AG_HIP(hipGetLastError());
   AG_HIP(hipMalloc(&d_raw, sizeof(double) * (D + 1) * std::max<int64_t>(np, 1)));
   AG_HIP(hipMalloc(&d_keep, std::max<int64_t>(np, 1)));
+  const PairsOut O{d_off, d_rank, min_sens, d_raw, d_keep};
   // integrate in slices so that each launch stays short
   const int64_t slice = 1 << 22;
   for (int64_t b = 0; b < nmain; b += slice) {
     const int64_t n = std::min(slice, nmain - b);
-    k_integrate<SU, SV, SW><<<dim3((unsigned)((n + 127) / 128)), dim3(128), 0, st>>>(
-        C, dims, n, d_cps, G, d_mains + b, d_off, d_rank, min_sens, d_raw, d_keep);
+    const Mains M{d_cps, d_mains + b};
+    hipLaunchKernelGGL((k_integrate<SU, SV, SW>), dim3((unsigned)((n + 127) / 128)), dim3(128), 0, st, C, dims, n, M, G, O);
+    if (C.moment_mode == 0)
+      hipLaunchKernelGGL((k_integrate_marked<SU, SV, SW>), dim3((unsigned)((n + kMarkedRun - 1) / kMarkedRun)), dim3(64), 0,
+                         st, C, dims, n, M, G, O);
     AG_HIP(hipGetLastError());
   }
   // compaction
