@@ -336,8 +336,10 @@ __global__ __launch_bounds__(64 * kPbWaves) void k_pb_mfma(const WorkItem* __res
 // Final FP64 reduction, one workgroup per output cell: W lanes read a partial
 // row (contiguous), kRedThreads / W rows side by side in list order, then a fixed
 // tree over the row groups; Q = (2 * sum) / w, times `scale` (the spatial
-// operator's (d/L)^2 N dt, spat_oper_mod.f90:65-66).
-constexpr int kRedThreads = 512;
+// operator's (d/L)^2 N dt, spat_oper_mod.f90:65-66).  Bound by the latency of its row
+// loads where there are few cells: 1024 threads against 512 take 107 and 150 us at
+// 27^3 nodes (729 cells), 7.8 and 9.4 us at 15^3 (125), 4.1 and 4.9 us at 9^3 (27).
+constexpr int kRedThreads = 1024;
 template <int D>
 __global__ __launch_bounds__(kRedThreads) void k_pb_reduce(int64_t ncells, const int64_t* __restrict__ cell_ptr,
                                                            const int32_t* __restrict__ cell_rows,
