@@ -253,6 +253,7 @@ struct dgv_ctx {
   double* d_f = nullptr;
   double* d_q = nullptr;
   double* d_ft = nullptr;         // two VDFs transposed, for the merged evaluator
+  double* h_io = nullptr;         // pinned: one VDF in, one Q out (host-array calls)
   double* d_tmp[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
   double* d_red = nullptr;        // moment reduction scratch
   double* d_hi = nullptr;         // high-moment reduction scratch (on first use)
