@@ -277,7 +277,7 @@ __device__ __forceinline__ bool write_diagonal(const AgenConsts& C, const CellDi
 // One thread per main diagonal.  FP64 arithmetic bounds it: up to 19 smooth pieces of 24
 // points, each with up to four crossed lines (an inverse sine, a square root and the
 // antiderivatives each).  26 ms at 15^3 nodes (0.86 M spheres, 3.2 M pairs) with the arcs
-// searched, and their ends' sines and cosines taken, at every point; 3.7 ms (and 0.7 for
+// searched, and their ends' sines and cosines taken, at every point; 3.6 ms (and 1.2 for
 // the marked ones) with the arcs' ends known per piece.
 // Spheres that have to be integrated point by point are marked for k_integrate_marked.
 template <int SU, int SV, int SW>
@@ -290,11 +290,10 @@ __global__ __launch_bounds__(128) void k_integrate(AgenConsts C, CellDims dims, 
   double S[D];
   bool hit = false;
   if (C.moment_mode == 0) {
-    if (grazing(C, m.cen, 0.5 * m.dsph)) {
+    if (grazing(C, m.cen, 0.5 * m.dsph) || !sphere_integrals<SU, SV, SW>(C, m.cen, 0.5 * m.dsph, S)) {
       M.list[k] |= kPointwise;
       return;
     }
-    sphere_integrals<SU, SV, SW>(C, m.cen, 0.5 * m.dsph, S);
 #pragma unroll
     for (int l = 0; l < D; ++l) hit = hit || S[l] != 0.0;
   }

@@ -280,16 +280,21 @@ DGV_HD inline bool grazing(const AgenConsts& C, const double cen[3], double r) {
 }
 
 // S[l] = int_{S^2} phi_l(c + r k) dk for the su*sv*sw canonical basis functions; the sphere
-// is not a grazing one.
+// is not a grazing one.  False, and no S, if a piece is a sliver: where the radius equals the
+// distance of a face line or a corner to rounding, two breakpoints lie about 2e-8 apart and
+// which of the sliver's arcs are inside is a matter of the last bits.  Left to the search at
+// every point too, so that the values stay what that search gives (1e-8 of a raw value).
 template <int su, int sv, int sw>
-DGV_HD inline void sphere_integrals(const AgenConsts& C, const double cen[3], double r, double* S) {
+DGV_HD inline bool sphere_integrals(const AgenConsts& C, const double cen[3], double r, double* S) {
   constexpr int D = su * sv * sw;
 #pragma unroll
   for (int l = 0; l < D; ++l) S[l] = 0.0;
   const double pi = 3.141592653589793238462643383279502884;
   double bp[20];
   const int nb = sphere_pieces(C, cen, r, bp);
-  if (nb == 0) return;
+  if (nb == 0) return true;
+  for (int p = 0; p + 1 < nb; ++p)
+    if (bp[p + 1] - bp[p] > 1e-11 && bp[p + 1] - bp[p] < 1e-6) return false;
   const double du[2] = {C.u0 - cen[0], C.u1 - cen[0]}, dv[2] = {C.v0 - cen[1], C.v1 - cen[1]};
   const double mu = 0.5 * (C.u1 + C.u0), mv = 0.5 * (C.v1 + C.v0), mw = 0.5 * (C.w1 + C.w0);
   const double au = cen[0] - mu, av = cen[1] - mv, aw = cen[2] - mw;
@@ -362,6 +367,7 @@ DGV_HD inline void sphere_integrals(const AgenConsts& C, const double cen[3], do
         }
         S[(i * sv + j) * sw + l] = E;
       }
+  return true;
 }
 
 // ---- Grazing spheres -------------------------------------------------------------------
@@ -369,10 +375,11 @@ DGV_HD inline void sphere_integrals(const AgenConsts& C, const double cen[3], do
 // A record exists where a value exceeds min_sens, which may be 0.  For a sphere that
 // touches the cell to rounding that is decided by single points whose arcs are a few
 // units in the last place long; for one within the cell, or with a value that is zero but
-// for rounding (near_cutoff), by how the last bits fall.  These spheres keep the search
+// for rounding (near_cutoff), by how the last bits fall; and slivers (sphere_integrals) by
+// them too.  These spheres keep the search
 // for the arcs at every point, with the basis functions expanded there, so that the
 // set of records does not depend on how the others are integrated.  They are few (1 in
-// 1000, up to 3 in 100 where cells and nodes are alike in all dimensions) and eight
+// 500, up to 4 in 100 where cells and nodes are alike in all dimensions) and eight
 // times as costly per point.
 DGV_HD inline bool near_cutoff(double raw, double min_sens) { return fabs(fabs(raw) - min_sens) <= 1e-12; }
 
@@ -588,8 +595,8 @@ DGV_HD inline int pair_raw(const AgenConsts& C, const double x[3], const double 
   double S[D];
   const double r = 0.5 * dsph;
   bool pointwise = grazing(C, cen, r);
+  if (!pointwise) pointwise = !sphere_integrals<SU, SV, SW>(C, cen, r, S);
   if (!pointwise) {
-    sphere_integrals<SU, SV, SW>(C, cen, r, S);
     raw_from_sphere<SU, SV, SW>(C, x, y, S, raw);
     bool hit = false, near = false;
     for (int l = 0; l < D; ++l) {
