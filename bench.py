@@ -34,24 +34,45 @@ INT8_MFMA_PEAK_TOPS = 5000.0   # MI355X dense int8 matrix
 
 # per batched precision mode: rocprof kernel name, ops per in-grid record visit
 # and VDF, the matrix-core peak and its unit, and the algorithmic coefficient
-# bytes per launch as a function of (records, pairs)
+# bytes per launch as a function of (records, pairs).  FP64 runs on the merged
+# layout: the up to four diagonals of a box of nodes share one coefficient row, so
+# its operations and bytes are those of boxes (box_shares), not of records.
 MODE_ROOFLINE = {
     "INT8_SPLIT": ("k_batch_i8<27>", 28.0, INT8_MFMA_PEAK_TOPS, "TOP/s", lambda R, P: 260.0 * P),
     "FP32_COMP": ("k_batch_mfma<27,1>", 2.0, FP32_MFMA_PEAK_TFLOPS, "TFLOP/s", lambda R, P: 12.0 * R),
     "FP32_F64ACC": ("k_batch_mfma<27,2>", 2.0, FP32_MFMA_PEAK_TFLOPS, "TFLOP/s", lambda R, P: 12.0 * R),
-    "FP64": ("k_batch_mfma<27,0>", 2.0, FP64_PEAK_TFLOPS, "TFLOP/s", lambda R, P: 16.0 * R),
+    "FP64": ("k_quad_batch<27>", 2.0, FP64_PEAK_TFLOPS, "TFLOP/s", lambda R, P: 16.0 * R),
 }
 MODE_OPS_DEF = {
     "INT8_SPLIT": "2 x 14 int8 digit multiply-adds per in-grid record visit and VDF (five-digit coefficient x "
                   "four-digit product, digit products down to 256^-4 of the leading one)",
     "FP32_COMP": "2 flop per in-grid record visit and VDF", "FP32_F64ACC": "2 flop per in-grid record visit and VDF",
-    "FP64": "2 flop per in-grid record visit and VDF"}
+    "FP64": "2 flop per in-grid visit of a coefficient row and VDF, one row per box of nodes (box_shares of the "
+            "record visits)"}
 MODE_DTYPE = {"INT8_SPLIT": "i8 digits, i32 exact sums, f64 scaling", "FP32_COMP": "f32+twosum/f64",
               "FP32_F64ACC": "f32/f64 sums", "FP64": "f64"}
 
 
 def log(msg: str) -> None:
     print(f"[bench] {msg}", file=sys.stderr, flush=True)
+
+
+def box_shares(d, u, v, w, M, s, rng, nsample=400000):
+    """(share of the in-grid record visits, share of the records) that remain with
+    one coefficient row per box of nodes: a pair whose nodes differ in k dimensions is
+    one of its box's 2^(k - 1) diagonals, which all reach the same output cells.  From a
+    sample of one basis function's records."""
+    _, xi, xi1 = d.get_aarray_basis(s ** 3 // 2)
+    k = rng.integers(0, len(xi), min(nsample, len(xi)))
+    x, y = np.asarray(xi)[k].astype(np.int64) - 1, np.asarray(xi1)[k].astype(np.int64) - 1
+    diag = 2.0 ** (sum((np.abs(c[x] - c[y]) > 1e-12).astype(int) for c in (u, v, w)) - 1)
+    cc = d.ccell - 1
+    visits = np.ones(len(k))
+    for div in (M * M, M, 1):
+        a, b, c0 = x // s ** 3 // div % M, y // s ** 3 // div % M, cc // div % M
+        lo, hi = np.maximum(0, np.maximum(c0 - a, c0 - b)), np.minimum(M, np.minimum(M + c0 - a, M + c0 - b))
+        visits *= np.maximum(hi - lo, 0)
+    return float((visits / diag).sum() / visits.sum()), float((1 / diag).mean())
 
 
 def config_vdf(u, v, w, gwts, M, rng):
@@ -97,7 +118,7 @@ def main():
     ap.add_argument("--sur-rows", type=int, default=8192, help="(f, Q) pairs generated for the surrogate")
     ap.add_argument("--sur-steps", type=int, default=4000)
     ap.add_argument("--profile", action="store_true", help="evaluator loops only (for rocprofv3)")
-    ap.add_argument("--headline-mode", default="INT8_SPLIT", help="batched mode timed by --profile")
+    ap.add_argument("--headline-mode", default="FP64", help="batched mode timed by --profile")
     ap.add_argument("--copy-probe", action="store_true",
                     help="only a plain device copy of 1 GiB, 5 times (calibrates rocprofv3 byte counters)")
     ap.add_argument("--profile-surrogate", action="store_true",
@@ -139,7 +160,7 @@ def main():
     kernels = {}
     names = {"record": dgv.DGV_KERNEL_RECORD, "pairblock_valu": dgv.DGV_KERNEL_PAIRBLOCK,
              "pairblock_mfma": dgv.DGV_KERNEL_MFMA}
-    knames = {"record": "k_rec_eval", "pairblock_valu": "k_pb_eval<27>", "pairblock_mfma": "k_pb_mfma<27>"}
+    knames = {"record": "k_rec_eval", "pairblock_valu": "k_pb_eval<27>", "pairblock_mfma": "k_quad_eval<27>"}
     cand = ["pairblock_mfma"] if args.profile else [k for k in names if not (k == "record" and M > 5)]
     for name in cand:
         d.set_kernel(names[name])
@@ -284,16 +305,21 @@ def main():
     rh = results[head]
     value = rh["vdf_q_per_s"]
     kname, ops_per_visit, peak, punit, coef_bytes = MODE_ROOFLINE[head]
-    ops = ops_per_visit * V * B   # per launch: multiply-adds per in-grid record visit and VDF, x2
+    visit_share, record_share = box_shares(d, u, v, w, M, 3, np.random.default_rng(seed))
+    # FP64 modes: coefficient rows per box of nodes
+    V1 = V * visit_share if knames[best] == "k_quad_eval<27>" else V
+    R1 = R * record_share if knames[best] == "k_quad_eval<27>" else R
+    Vh, Rh = (V * visit_share, R * record_share) if head == "FP64" else (V, R)
+    ops = ops_per_visit * Vh * B   # per launch: multiply-adds per in-grid record visit and VDF, x2
     achieved = ops / (rh["kernel_ms"] * 1e-3) / 1e12
     single_qps = 1e3 / ms_single
     # the HBM roofline: algorithmic bytes per launch (coefficient records streamed
     # once per launch, f read and Q written once) against 8 TB/s, and the
     # counter-measured traffic
-    bytes_b = coef_bytes(R, wl["pairs"]) + 16.0 * N * B
-    bytes_1 = 16.0 * R + 16.0 * N
+    bytes_b = coef_bytes(Rh, wl["pairs"]) + 16.0 * N * B
+    bytes_1 = 16.0 * R1 + 16.0 * N
     tr_b = measured_traffic(kname, f"batch{B}_M{M}")
-    tr_1 = measured_traffic("k_pb_mfma<27,false>", f"single_M{M}")
+    tr_1 = measured_traffic(knames[best], f"single_M{M}")
 
     def hbm(bytes_alg, traffic, kernel_ms, rate, per_unit):
         t = kernel_ms * 1e-3
@@ -310,7 +336,7 @@ def main():
         hbm_1["rk3_frac_of_hbm_roofline"] = rk["projected"]["steps_per_sec"] / hbm_1["rk3_steps_per_s_bound_at_hbm_peak"]
     for prec in modes:   # every mode against its own matrix-core peak
         kn, opv, pk, pu, _ = MODE_ROOFLINE[prec]
-        a = opv * V * B / (results[prec]["kernel_ms"] * 1e-3) / 1e12
+        a = opv * (V * visit_share if prec == "FP64" else V) * B / (results[prec]["kernel_ms"] * 1e-3) / 1e12
         results[prec]["roofline"] = {"kernel": kn, "achieved": a, "peak": pk, "unit": pu, "frac": a / pk,
                                      "speedup_vs_fp64_plain": results[prec]["vdf_q_per_s"] / single_qps}
     out = {
@@ -340,11 +366,12 @@ def main():
                      "ops_per_launch": ops, "ops_definition": MODE_OPS_DEF[head],
                      "hbm_bytes_per_launch_algorithmic": bytes_b, "hbm": hbm_b,
                      "fp64_plain": {"kernel": knames[best], "kernel_ms": ms_single_main, "hbm": hbm_1,
-                                    "tflops": 2.0 * V / (ms_single_main * 1e-3) / 1e12,
-                                    "frac_fp64_peak": 2.0 * V / (ms_single_main * 1e-3) / 1e12 / FP64_PEAK_TFLOPS,
-                                    "hbm_gbs_algorithmic": (16.0 * R + 16.0 * N) / (ms_single_main * 1e-3) / 1e9,
+                                    "tflops": 2.0 * V1 / (ms_single_main * 1e-3) / 1e12,
+                                    "frac_fp64_peak": 2.0 * V1 / (ms_single_main * 1e-3) / 1e12 / FP64_PEAK_TFLOPS,
+                                    "hbm_gbs_algorithmic": (16.0 * R1 + 16.0 * N) / (ms_single_main * 1e-3) / 1e9,
                                     "traffic": tr_1,
-                                    "l2": measured_l2("k_pb_mfma<27,false>", f"single_M{M}")}},
+                                    "l2": measured_l2(knames[best], f"single_M{M}")},
+                     "box_visit_share": visit_share, "box_record_share": record_share},
         "cpu_baseline": cpu,
         "conservation": {"sum_w_psi_Q": [float(x) for x in mom], "sum_abs_w_psi_Q": absmom,
                          "after_projection_rel_max": proj_rel},
@@ -539,7 +566,7 @@ def mixed_grid_leg(dgv, d27, rng, args, tiles=None):
         b.rk_run(0.005, 2, rkmts=2, use_graph=True)
         rk_el = (time.perf_counter() - t) / 2
         out[prec] = {"seconds_per_batch": el, "vdf_q_per_s": len(which) / el,
-                     "tflops": 2.0 * visits / el / 1e12, "rk2_graph_step_seconds": rk_el}
+                     "record_visit_tflops": 2.0 * visits / el / 1e12, "rk2_graph_step_seconds": rk_el}
         log(f"mixed grids {prec}: {el:.2f} s per 512 VDFs = {len(which) / el:.1f} VDF-Q/s; RK2 step {rk_el:.2f} s")
         b.close()
     for prec in ("INT8_SPLIT", "FP32_COMP", "FP32_F64ACC"):
