@@ -453,18 +453,16 @@ __global__ __launch_bounds__(256) void k_quad_transpose(int64_t ncells, int D, c
 // = (column, parity of the node).  f element (cell, p) is at cell * sc + p * sp
 // bytes: with f transposed the columns of one row are runs of cells along w.
 template <int D, bool MIX, int NW>
-__global__ __launch_bounds__(64 * NW, NW == 6 ? 3 : 2) void k_quad_eval(const QuadItem* __restrict__ items,
+__global__ __launch_bounds__(64 * NW, 2) void k_quad_eval(const QuadItem* __restrict__ items,
                                                           const QuadBlk* __restrict__ blocks,
                                                           const double* __restrict__ steps,
                                                           const double* __restrict__ f, const double* __restrict__ gm,
                                                           uint32_t sc, uint32_t sp, double* __restrict__ partial,
                                                           int Mv, int Mw) {
   constexpr int ROWS = quad_rows<D>();
-  constexpr int HALVES = NW == 6 ? 2 : 1;         // a wave stages whole slots, or halves of their rows
-  constexpr int NA = (D + 1) / 2;                 // loads per lane and slot
-  constexpr int NI = (NA + HALVES - 1) / HALVES;  // and unit
-  constexpr int NU = (MIX ? 16 : 8) * HALVES;     // units
-  constexpr int SL = (NU + NW - 1) / NW;          // per wave
+  constexpr int NI = (D + 1) / 2;                 // loads per lane and slot
+  constexpr int SL = (MIX ? 16 : 8) / NW;         // slot copies per wave
+  static_assert(SL * NW == (MIX ? 16 : 8), "the slots divide over the waves");
   __shared__ __attribute__((aligned(16))) double lf[ROWS * kQuadRow];
   __shared__ __attribute__((aligned(16))) double lg[MIX ? ROWS * kQuadRow : 2];
   const QuadItem& it = items[blockIdx.x];
@@ -495,25 +493,25 @@ __global__ __launch_bounds__(64 * NW, NW == 6 ? 3 : 2) void k_quad_eval(const Qu
   auto fetch = [&](const QuadBlk& B) {
 #pragma unroll
     for (int k = 0; k < SL; ++k) {
-      const int un = wave + NW * k, sl = un / HALVES, h = un % HALVES, slot = sl & 7;
-      if (un >= NU || (slot & B.same)) continue;   // the cell of a lower slot: its rows are used
+      const int sl = wave + NW * k, slot = sl & 7;
+      if (slot & B.same) continue;   // the cell of a lower slot: its rows are used
       const int du = slot & 1 ? B.b[0] : B.a[0], dv = slot & 2 ? B.b[1] : B.a[1], dw = slot & 4 ? B.b[2] : B.a[2];
       const double* src = MIX && sl >= 8 ? gm : f;
       const __amdgpu_buffer_rsrc_t F =
-          ring_rsrc(reinterpret_cast<const char*>(src) + (int64_t)((du * Mv + dv) * Mw + dw) * sc + (int64_t)(2 * NI * h) * sp);
+          ring_rsrc(reinterpret_cast<const char*>(src) + (int64_t)((du * Mv + dv) * Mw + dw) * sc);
 #pragma unroll
-      for (int i = 0; i < NI; ++i) v[k][i] = ring_f64(F, h == HALVES - 1 && i + 1 == NI ? glast : goff, (uint32_t)(2 * i) * sp);
+      for (int i = 0; i < NI; ++i) v[k][i] = ring_f64(F, i + 1 < NI ? goff : glast, (uint32_t)(2 * i) * sp);
     }
   };
   auto store = [&](const QuadBlk& B) {
 #pragma unroll
     for (int k = 0; k < SL; ++k) {
-      const int un = wave + NW * k, sl = un / HALVES, h = un % HALVES, slot = sl & 7;
-      if (un >= NU || (slot & B.same)) continue;
-      char* dst = reinterpret_cast<char*>(MIX && sl >= 8 ? lg : lf) + (slot * D + 2 * NI * h) * kQuadRow * 8;
+      const int sl = wave + NW * k, slot = sl & 7;
+      if (slot & B.same) continue;
+      char* dst = reinterpret_cast<char*>(MIX && sl >= 8 ? lg : lf) + slot * D * kQuadRow * 8;
 #pragma unroll
       for (int i = 0; i < NI; ++i)
-        *reinterpret_cast<double*>(dst + (h == HALVES - 1 && i + 1 == NI ? llast : loff) + 2 * i * kQuadRow * 8) = v[k][i];
+        *reinterpret_cast<double*>(dst + (i + 1 < NI ? loff : llast) + 2 * i * kQuadRow * 8) = v[k][i];
     }
   };
   const int ncols = min(kQuadCols, ncells - chunk * kQuadCols);
@@ -561,7 +559,7 @@ int launch_main_quad(dgv_ctx* ctx, const double* d_f, const double* d_g, double*
                      Q.d_blocks, Q.d_steps, F, G, sc, sp, part, g.Mv, g.Mw)
   if (g.D == 27) {
     if (d_g) DGV_QUAD(27, true, 8);
-    else DGV_QUAD(27, false, 6);
+    else DGV_QUAD(27, false, 4);
   } else {
     if (d_g) DGV_QUAD(8, true, 8);
     else DGV_QUAD(8, false, 4);
