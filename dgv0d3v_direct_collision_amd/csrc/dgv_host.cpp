@@ -143,6 +143,7 @@ void bump_aarray_generation(dgv_ctx* ctx) {
 
 void free_pairblock(dgv_ctx* ctx) {
   bump_aarray_generation(ctx);
+  free_plan(ctx);   // its items refer to this array's blocks
   free_linear(ctx);
   free_quads(ctx);
   PairBlock& pb = ctx->pb;
@@ -498,6 +499,7 @@ int plan_cell_rows(dgv_ctx* ctx, const std::vector<int64_t>& row0, const std::ve
   DGV_HIP(ctx, hipMemcpy(P.d_cell_ptr, cnt.data(), sizeof(int64_t) * (g.ncells + 1), hipMemcpyHostToDevice));
   DGV_HIP(ctx, hipMalloc(&P.d_cell_rows, sizeof(int32_t) * std::max<size_t>(rows.size(), 1)));
   DGV_HIP(ctx, hipMemcpy(P.d_cell_rows, rows.data(), sizeof(int32_t) * rows.size(), hipMemcpyHostToDevice));
+  P.ready = true;
   return DGV_OK;
 }
 

@@ -178,6 +178,7 @@ struct alignas(16) QuadItem {
 // Work decomposition of one evaluation (depends on tile size).
 struct Plan {
   int32_t pairs_per_item = 0;
+  bool ready = false;                 // every part is built: evaluations may use it
   bool quad = false;                  // items of the merged layout
   bool transpose = false;             // ... which read f transposed
   std::vector<WorkItem> items;

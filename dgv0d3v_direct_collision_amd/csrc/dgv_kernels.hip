@@ -429,6 +429,9 @@ static int launch_main_pairblock(dgv_ctx* ctx, const double* d_f, bool mfma, con
   const PairBlock& pb = ctx->pb;
   const Plan& P = ctx->plan;
   double* const part = partial ? partial : P.d_partial;
+  // a call that failed while it changed the A-array or the plan leaves none
+  if (!P.ready)
+    return set_error(ctx, DGV_ERR_STATE, "no work plan: the call that last changed the A-array or the plan failed");
   if (P.quad) return launch_main_quad(ctx, d_f, d_g, part);
   const int nitems = (int)P.items.size();
   if (nitems == 0) return DGV_OK;

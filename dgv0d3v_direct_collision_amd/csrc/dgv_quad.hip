@@ -203,6 +203,7 @@ __global__ __launch_bounds__(256) void k_quad_write(QuadDims<D> g, const QuadBlk
 }
 
 void free_quads(dgv_ctx* ctx) {
+  if (ctx->plan.quad) free_plan(ctx);   // its items walk these blocks
   QuadLayout& Q = ctx->quad;
   hipFree(Q.d_steps); hipFree(Q.d_blocks);
   Q = QuadLayout();
@@ -299,7 +300,12 @@ static int build_quads_t(dgv_ctx* ctx) {
   hipError_t e = hipMemcpyAsync(d_src, src2.data(), sizeof(QuadSrc) * nq, hipMemcpyHostToDevice, st);
   if (e == hipSuccess)
     e = hipMemcpyAsync(Q.d_blocks, Q.blocks.data(), sizeof(QuadBlk) * nq, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess && launch_pair_index(ctx, d_pidx) == DGV_OK) {
+  if (e == hipSuccess) {
+    if (int rc = launch_pair_index(ctx, d_pidx)) {
+      drop();
+      free_quads(ctx);
+      return rc;
+    }
     hipLaunchKernelGGL(k_quad_assign<D>, dim3((unsigned)nq), dim3(256), 0, st, dims, Q.d_blocks, d_src, pb.d_blocks,
                        d_pidx, pb.d_pairs, kQuadTol, d_assign, d_count);
     e = hipGetLastError();

@@ -88,6 +88,7 @@ static int truncate_aarray(dgv_ctx* ctx, const TruncArgs& ta) {
   const int64_t np = pb.npairs;
   uint8_t* d_keep = nullptr;
   DGV_HIP(ctx, hipMalloc(&d_keep, std::max<int64_t>(np, 1)));
+  free_quads(ctx);   // rows of the array as it was
   if (!pb.blocks.empty())
     hipLaunchKernelGGL(k_truncate, dim3((unsigned)pb.blocks.size()), dim3(256), 0, ctx->stream, pb.d_blocks,
                        pb.d_pairs, ctx->d_u, ctx->d_v, ctx->d_w, d_keep, ta);
@@ -195,6 +196,7 @@ int dgv_ctx_aarray_abs(dgv_ctx* ctx) {
   if (!ctx->has_a) return set_error(ctx, DGV_ERR_STATE, "no A-array");
   DGV_HIP(ctx, hipSetDevice(ctx->device));
   bump_aarray_generation(ctx);
+  free_quads(ctx);   // rows of the array as it was
   const int64_t tot = ctx->pb.npairs * (ctx->g.D + 1);
   if (tot > 0)
     hipLaunchKernelGGL(k_abs_coeff, dim3(stride_blocks(tot, 256)), dim3(256), 0, ctx->stream, ctx->pb.npairs,

@@ -1,0 +1,83 @@
+// A stand-in for the HIP runtime, for host-side tests of what the library does when a
+// call of it fails: device memory is zeroed host memory, copies are memcpy, kernels are not run.  Linked into a
+// copy of libdgv_amd.so (tests/fake_device.py).  fake_fail_kernel / fake_fail_malloc choose
+// the call that fails; the launches so far, and the widest, can be read back.
+#include <cstdint>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <string>
+
+typedef int hipError_t;   // hipSuccess 0, hipErrorOutOfMemory 2, hipErrorInvalidConfiguration 9
+struct dim3_t { uint32_t x, y, z; };
+
+static std::map<const void*, std::string> names;
+static std::string fail_kernel, launched;
+static int64_t fail_malloc_above = INT64_MAX;
+static uint64_t widest = 0;
+static hipError_t last = 0;
+static struct { dim3_t g, b; size_t shm; void* st; } conf;
+
+extern "C" {
+void fake_fail_kernel(const char* part) { fail_kernel = part; }
+void fake_fail_malloc_above(int64_t bytes) { fail_malloc_above = bytes; }
+void fake_reset() { launched.clear(); widest = 0; }
+const char* fake_launched() { return launched.c_str(); }
+uint64_t fake_widest_launch() { return widest; }
+
+void** __hipRegisterFatBinary(const void*) { static void* h = nullptr; return &h; }
+void __hipUnregisterFatBinary(void**) {}
+void __hipRegisterFunction(void**, const void* host, char*, const char* device, unsigned, void*, void*, dim3_t*, dim3_t*, int*) {
+  names[host] = device;
+}
+void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
+hipError_t __hipPushCallConfiguration(dim3_t g, dim3_t b, size_t shm, void* st) { conf = {g, b, shm, st}; return 0; }
+hipError_t __hipPopCallConfiguration(dim3_t* g, dim3_t* b, size_t* shm, void** st) {
+  *g = conf.g; *b = conf.b; *shm = conf.shm; *st = conf.st;
+  return 0;
+}
+hipError_t hipLaunchKernel(const void* f, dim3_t g, dim3_t b, void**, size_t, void*) {
+  const std::string& n = names[f];
+  launched += n + "\n";
+  const uint64_t items = (uint64_t)g.x * b.x;
+  if (items > widest) widest = items;
+  if (items >> 32) return last = 9;   // a grid dimension holds fewer than 2^32 work-items
+  if (!fail_kernel.empty() && n.find(fail_kernel) != std::string::npos) return last = 9;
+  return 0;
+}
+hipError_t hipGetLastError() { const hipError_t e = last; last = 0; return e; }
+const char* hipGetErrorString(hipError_t e) { return e ? "fake error" : "no error"; }
+hipError_t hipMalloc(void** p, size_t n) {
+  if ((int64_t)n > fail_malloc_above || !(*p = calloc(n ? n : 1, 1))) return 2;   // reported here alone
+  return 0;
+}
+hipError_t hipFree(void* p) { free(p); return 0; }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return hipMalloc(p, n); }
+hipError_t hipHostFree(void* p) { free(p); return 0; }
+hipError_t hipMemcpy(void* d, const void* s, size_t n, int) { memcpy(d, s, n); return 0; }
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, int, void*) { memcpy(d, s, n); return 0; }
+hipError_t hipMemcpy2DAsync(void* d, size_t dp, const void* s, size_t sp, size_t w, size_t h, int, void*) {
+  for (size_t i = 0; i < h; ++i) memcpy((char*)d + i * dp, (const char*)s + i * sp, w);
+  return 0;
+}
+hipError_t hipMemsetAsync(void* d, int v, size_t n, void*) { memset(d, v, n); return 0; }
+hipError_t hipGetSymbolAddress(void** p, const void* s) { *p = const_cast<void*>(s); return 0; }
+hipError_t hipGetDeviceCount(int* n) { *n = 1; return 0; }
+hipError_t hipGetDevicePropertiesR0600(void*, int) { return 0; }
+hipError_t hipSetDevice(int) { return 0; }
+hipError_t hipDeviceSynchronize() { return 0; }
+hipError_t hipStreamCreateWithFlags(void** s, unsigned) { *s = nullptr; return 0; }
+hipError_t hipStreamDestroy(void*) { return 0; }
+hipError_t hipStreamSynchronize(void*) { return 0; }
+hipError_t hipStreamBeginCapture(void*, int) { return 0; }
+hipError_t hipStreamEndCapture(void*, void** g) { *g = nullptr; return 0; }
+hipError_t hipEventCreate(void** e) { *e = nullptr; return 0; }
+hipError_t hipEventDestroy(void*) { return 0; }
+hipError_t hipEventRecord(void*, void*) { return 0; }
+hipError_t hipEventSynchronize(void*) { return 0; }
+hipError_t hipEventElapsedTime(float* ms, void*, void*) { *ms = 1.f; return 0; }
+hipError_t hipGraphInstantiate(void** x, void*, void*, char*, size_t) { *x = nullptr; return 0; }
+hipError_t hipGraphLaunch(void*, void*) { return 0; }
+hipError_t hipGraphDestroy(void*) { return 0; }
+hipError_t hipGraphExecDestroy(void*) { return 0; }
+}
