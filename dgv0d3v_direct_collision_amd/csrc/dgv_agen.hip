@@ -133,50 +133,52 @@ __device__ __forceinline__ bool candidate(const AgenConsts& C, int2 XY, int c, c
   return pair_distance(C, x, y) >= 0.0;
 }
 
-// One wave per cp: cnt = its pairs and its main diagonals
+// One wave per cp in turn: cnt = its pairs and its main diagonals
 template <int SU, int SV, int SW>
-__global__ __launch_bounds__(64) void k_count(AgenConsts C, CellDims dims, const int2* __restrict__ cps, NodeGeo G,
-                                              uint2* __restrict__ cnt) {
+__global__ __launch_bounds__(64) void k_count(AgenConsts C, CellDims dims, int64_t ncp, const int2* __restrict__ cps,
+                                              NodeGeo G, uint2* __restrict__ cnt) {
   constexpr int D = SU * SV * SW;
-  const int64_t cp = blockIdx.x;
-  const int2 XY = cps[cp];
-  uint32_t n = 0, m = 0;
-  for (int c0 = 0; c0 < D * D; c0 += 64) {
-    const int c = c0 + (int)threadIdx.x;
-    const bool ok = candidate<D>(C, XY, c, G);
-    const bool main = ok && main_diagonal<SU, SV, SW>(dims, XY, c / D, c % D);
-    n += __popcll(__ballot(ok));
-    m += __popcll(__ballot(main));
+  for (int64_t cp = blockIdx.x; cp < ncp; cp += gridDim.x) {
+    const int2 XY = cps[cp];
+    uint32_t n = 0, m = 0;
+    for (int c0 = 0; c0 < D * D; c0 += 64) {
+      const int c = c0 + (int)threadIdx.x;
+      const bool ok = candidate<D>(C, XY, c, G);
+      const bool main = ok && main_diagonal<SU, SV, SW>(dims, XY, c / D, c % D);
+      n += __popcll(__ballot(ok));
+      m += __popcll(__ballot(main));
+    }
+    if (threadIdx.x == 0) cnt[cp] = make_uint2(n, m);
   }
-  if (threadIdx.x == 0) cnt[cp] = make_uint2(n, m);
 }
 
 // ... the pairs' codes p << 8 | q in (p, q) order, each candidate's rank among them
 // (-1: no pair) and the main diagonals
 template <int SU, int SV, int SW>
-__global__ __launch_bounds__(64) void k_list(AgenConsts C, CellDims dims, const int2* __restrict__ cps, NodeGeo G,
-                                             const int64_t* __restrict__ off, const int64_t* __restrict__ moff,
-                                             uint16_t* __restrict__ code, int16_t* __restrict__ rank,
-                                             uint64_t* __restrict__ mains) {
+__global__ __launch_bounds__(64) void k_list(AgenConsts C, CellDims dims, int64_t ncp, const int2* __restrict__ cps,
+                                             NodeGeo G, const int64_t* __restrict__ off,
+                                             const int64_t* __restrict__ moff, uint16_t* __restrict__ code,
+                                             int16_t* __restrict__ rank, uint64_t* __restrict__ mains) {
   constexpr int D = SU * SV * SW;
-  const int64_t cp = blockIdx.x;
-  const int2 XY = cps[cp];
   const int lane = threadIdx.x;
   const uint64_t below = ((uint64_t)1 << lane) - 1;
-  int n = 0;
-  int64_t m = moff[cp];
-  const int64_t o = off[cp];
-  for (int c0 = 0; c0 < D * D; c0 += 64) {
-    const int c = c0 + lane;
-    const bool ok = candidate<D>(C, XY, c, G);
-    const bool main = ok && main_diagonal<SU, SV, SW>(dims, XY, c / D, c % D);
-    const uint64_t bo = __ballot(ok), bm = __ballot(main);
-    const int r = n + __popcll(bo & below);
-    if (c < D * D) rank[cp * (D * D) + c] = ok ? (int16_t)r : (int16_t)-1;
-    if (ok) code[o + r] = (uint16_t)((c / D) << 8 | c % D);
-    if (main) mains[m + __popcll(bm & below)] = ((uint64_t)cp << 16) | ((uint64_t)(c / D) << 8) | (uint64_t)(c % D);
-    n += __popcll(bo);
-    m += __popcll(bm);
+  for (int64_t cp = blockIdx.x; cp < ncp; cp += gridDim.x) {
+    const int2 XY = cps[cp];
+    int n = 0;
+    int64_t m = moff[cp];
+    const int64_t o = off[cp];
+    for (int c0 = 0; c0 < D * D; c0 += 64) {
+      const int c = c0 + lane;
+      const bool ok = candidate<D>(C, XY, c, G);
+      const bool main = ok && main_diagonal<SU, SV, SW>(dims, XY, c / D, c % D);
+      const uint64_t bo = __ballot(ok), bm = __ballot(main);
+      const int r = n + __popcll(bo & below);
+      if (c < D * D) rank[cp * (D * D) + c] = ok ? (int16_t)r : (int16_t)-1;
+      if (ok) code[o + r] = (uint16_t)((c / D) << 8 | c % D);
+      if (main) mains[m + __popcll(bm & below)] = ((uint64_t)cp << 16) | ((uint64_t)(c / D) << 8) | (uint64_t)(c % D);
+      n += __popcll(bo);
+      m += __popcll(bm);
+    }
   }
 }
 
@@ -338,28 +340,30 @@ __global__ __launch_bounds__(64) void k_integrate_marked(AgenConsts C, CellDims 
   }
 }
 
-// One wave per cp: its kept pairs and, for each p, the first kept pair with local
-// index of xi >= p
+// One wave per cp in turn: its kept pairs and, for each p, the first kept pair with
+// local index of xi >= p
 template <int D>
-__global__ __launch_bounds__(64) void k_kept(const int64_t* __restrict__ off, const uint16_t* __restrict__ code,
-                                             const uint8_t* __restrict__ keep, int32_t* __restrict__ kcnt,
-                                             uint16_t* __restrict__ seg) {
+__global__ __launch_bounds__(64) void k_kept(int64_t ncp, const int64_t* __restrict__ off,
+                                             const uint16_t* __restrict__ code, const uint8_t* __restrict__ keep,
+                                             int32_t* __restrict__ kcnt, uint16_t* __restrict__ seg) {
   __shared__ int per[D];
-  const int64_t cp = blockIdx.x;
-  if (threadIdx.x < D) per[threadIdx.x] = 0;
-  __syncthreads();
-  for (int64_t k = off[cp] + threadIdx.x; k < off[cp + 1]; k += 64)
-    if (keep[k]) atomicAdd(&per[code[k] >> 8], 1);
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint16_t* s = seg + cp * (D + 1);
-    int n = 0;
-    for (int p = 0; p < D; ++p) {
-      s[p] = (uint16_t)n;
-      n += per[p];
+  for (int64_t cp = blockIdx.x; cp < ncp; cp += gridDim.x) {
+    if (threadIdx.x < D) per[threadIdx.x] = 0;
+    __syncthreads();
+    for (int64_t k = off[cp] + threadIdx.x; k < off[cp + 1]; k += 64)
+      if (keep[k]) atomicAdd(&per[code[k] >> 8], 1);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      uint16_t* s = seg + cp * (D + 1);
+      int n = 0;
+      for (int p = 0; p < D; ++p) {
+        s[p] = (uint16_t)n;
+        n += per[p];
+      }
+      s[D] = (uint16_t)n;
+      kcnt[cp] = n;
     }
-    s[D] = (uint16_t)n;
-    kcnt[cp] = n;
+    __syncthreads();   // `per` is read
   }
 }
 
@@ -445,11 +449,10 @@ static int generate_t(dgv_ctx* ctx, const AgenConsts& C, double min_sens) {
   const NodeGeo G{ctx->d_u, ctx->d_v, ctx->d_w, ctx->d_gwts};
   const CellDims dims{g.Mv, g.Mw, nc};
   hipStream_t st = ctx->stream;
-  if (ncp >= (int64_t)1 << 31) return set_error(ctx, DGV_ERR_UNSUPPORTED, "A-array generator: too many cell pairs");
   AG_HIP(hipMalloc(&d_cps, sizeof(int2) * ncp));
   AG_HIP(hipMemcpyAsync(d_cps, cps.data(), sizeof(int2) * ncp, hipMemcpyHostToDevice, st));
   AG_HIP(hipMalloc(&d_cnt, sizeof(uint2) * ncp));
-  hipLaunchKernelGGL((k_count<SU, SV, SW>), dim3((unsigned)ncp), dim3(64), 0, st, C, dims, d_cps, G, d_cnt);
+  hipLaunchKernelGGL((k_count<SU, SV, SW>), dim3(loop_blocks(ncp)), dim3(64), 0, st, C, dims, ncp, d_cps, G, d_cnt);
   AG_HIP(hipGetLastError());
   std::vector<uint2> cnt(ncp);
   AG_HIP(hipMemcpyAsync(cnt.data(), d_cnt, sizeof(uint2) * ncp, hipMemcpyDeviceToHost, st));
@@ -467,7 +470,7 @@ static int generate_t(dgv_ctx* ctx, const AgenConsts& C, double min_sens) {
   AG_HIP(hipMalloc(&d_code, sizeof(uint16_t) * std::max<int64_t>(np, 1)));
   AG_HIP(hipMalloc(&d_rank, sizeof(int16_t) * D * D * ncp));
   AG_HIP(hipMalloc(&d_mains, sizeof(uint64_t) * std::max<int64_t>(nmain, 1)));
-  hipLaunchKernelGGL((k_list<SU, SV, SW>), dim3((unsigned)ncp), dim3(64), 0, st, C, dims, d_cps, G, d_off, d_moff,
+  hipLaunchKernelGGL((k_list<SU, SV, SW>), dim3(loop_blocks(ncp)), dim3(64), 0, st, C, dims, ncp, d_cps, G, d_off, d_moff,
                      d_code, d_rank, d_mains);
   AG_HIP(hipGetLastError());
   AG_HIP(hipMalloc(&d_raw, sizeof(double) * (D + 1) * std::max<int64_t>(np, 1)));
@@ -488,7 +491,7 @@ static int generate_t(dgv_ctx* ctx, const AgenConsts& C, double min_sens) {
   AG_HIP(hipMalloc(&d_kcnt, sizeof(int32_t) * ncp));
   AG_HIP(hipMalloc(&d_seg, sizeof(uint16_t) * (D + 1) * ncp));
   AG_HIP(hipMalloc(&d_bcnt, sizeof(unsigned long long) * D));
-  hipLaunchKernelGGL(k_kept<D>, dim3((unsigned)ncp), dim3(64), 0, st, d_off, d_code, d_keep, d_kcnt, d_seg);
+  hipLaunchKernelGGL(k_kept<D>, dim3(loop_blocks(ncp)), dim3(64), 0, st, ncp, d_off, d_code, d_keep, d_kcnt, d_seg);
   AG_HIP(hipGetLastError());
   std::vector<int32_t> kcnt(ncp);
   std::vector<uint16_t> seg((size_t)ncp * (D + 1));

@@ -24,6 +24,7 @@
 // sharing the product f*f of a pair between its D basis functions.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <array>
 #include <cstdint>
 #include <string>
@@ -103,6 +104,10 @@ inline unsigned stride_blocks(int64_t n, int block) {
   if (b > (1 << 20)) b = 1 << 20;
   return (unsigned)(b < 1 ? 1 : b);
 }
+
+// Workgroups for a loop over n items that takes a whole workgroup each: the same limit
+// would hold 2^24 of 256 threads, and there are more cell pairs than that on 19^3 cells.
+inline unsigned loop_blocks(int64_t n) { return (unsigned)std::max<int64_t>(1, std::min<int64_t>(n, 1 << 16)); }
 
 struct Grid {
   int Mu = 0, Mv = 0, Mw = 0, su = 0, sv = 0, sw = 0, D = 0;
