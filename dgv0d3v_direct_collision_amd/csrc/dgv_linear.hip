@@ -51,28 +51,32 @@ struct FmaDims {
   __host__ __device__ int64_t ncext() const { return (int64_t)eu() * ev() * ew(); }
 };
 
-__global__ void k_pair_index(int D, const BlockHdr* __restrict__ blocks, const double* __restrict__ pairs,
-                             int16_t* __restrict__ idx) {
+// One workgroup per block in turn: idx[(block) D D + p D + q] = the pair (p, q) of the block, or -1
+__global__ __launch_bounds__(256) void k_pair_index(int D, int64_t nblocks, const BlockHdr* __restrict__ blocks,
+                                                    const double* __restrict__ pairs, int16_t* __restrict__ idx) {
   __shared__ int16_t t[64 * 64];
-  const BlockHdr* B = blocks + blockIdx.x;
   const int DD = D * D;
-  for (int i = threadIdx.x; i < DD; i += blockDim.x) t[i] = -1;
-  __syncthreads();
-  const int n = B->seg[D];
-  const double* P = pairs + B->pbeg * (D + 1);
-  for (int k = threadIdx.x; k < n; k += blockDim.x) {
-    const int code = (int)(__double_as_longlong(P[(int64_t)k * (D + 1) + D]) & 0xffff);
-    t[(code >> 8) * D + (code & 255)] = (int16_t)k;
+  for (int64_t b = blockIdx.x; b < nblocks; b += gridDim.x) {
+    const BlockHdr* B = blocks + b;
+    for (int i = threadIdx.x; i < DD; i += blockDim.x) t[i] = -1;
+    __syncthreads();
+    const int n = B->seg[D];
+    const double* P = pairs + B->pbeg * (D + 1);
+    for (int k = threadIdx.x; k < n; k += blockDim.x) {
+      const int code = (int)(__double_as_longlong(P[(int64_t)k * (D + 1) + D]) & 0xffff);
+      t[(code >> 8) * D + (code & 255)] = (int16_t)k;
+    }
+    __syncthreads();
+    int16_t* out = idx + b * DD;
+    for (int i = threadIdx.x; i < DD; i += blockDim.x) out[i] = t[i];
+    __syncthreads();   // the table is read
   }
-  __syncthreads();
-  int16_t* out = idx + (int64_t)blockIdx.x * DD;
-  for (int i = threadIdx.x; i < DD; i += blockDim.x) out[i] = t[i];
 }
 
 int launch_pair_index(dgv_ctx* ctx, int16_t* d_idx) {
   const int64_t nb = (int64_t)ctx->pb.blocks.size();
   if (nb > 0)
-    hipLaunchKernelGGL(k_pair_index, dim3((unsigned)nb), dim3(256), 0, ctx->stream, ctx->g.D, ctx->pb.d_blocks,
+    hipLaunchKernelGGL(k_pair_index, dim3(loop_blocks(nb)), dim3(256), 0, ctx->stream, ctx->g.D, nb, ctx->pb.d_blocks,
                        ctx->pb.d_pairs, d_idx);
   DGV_HIP(ctx, hipGetLastError());
   return DGV_OK;

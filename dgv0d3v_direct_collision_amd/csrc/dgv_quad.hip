@@ -89,58 +89,59 @@ __device__ __forceinline__ int block_scan(int v, int& before) {
   return total;
 }
 
-// One workgroup per quad block: which records of each candidate box merge.
+// One workgroup per quad block in turn: which records of each candidate box merge.
 // assign[(block) D D + c]: 4 bits per entry, 0 = absent, else 1 + its cluster.
 template <int D>
-__global__ __launch_bounds__(256) void k_quad_assign(QuadDims<D> g, const QuadBlk* __restrict__ qb,
+__global__ __launch_bounds__(256) void k_quad_assign(QuadDims<D> g, int64_t nq, const QuadBlk* __restrict__ qb,
                                                      const QuadSrc* __restrict__ src,
                                                      const BlockHdr* __restrict__ blocks,
                                                      const int16_t* __restrict__ pidx,
                                                      const double* __restrict__ pairs, double tol,
                                                      uint32_t* __restrict__ assign, int32_t* __restrict__ count) {
-  const int64_t b = blockIdx.x;
-  const QuadSrc S = src[b];
-  const int same = qb[b].same;
-  int mine = 0;
-  for (int c = threadIdx.x; c < D * D; c += 256) {
-    uint32_t a = 0;
-    int ncl = 0;
-    int64_t lead[8];
-    int size[8];
-    quad_entries<D>(g, c / D, c % D, same, S, blocks, pidx, [&](int e, int64_t pair, uint32_t, uint32_t) {
-      const double* T = pairs + pair * (D + 1);
-      int k = 0;
-      for (; k < ncl; ++k) {
-        if (size[k] == 4) continue;
-        const double* L = pairs + lead[k] * (D + 1);
-        bool eq = true;
-        for (int l = 0; l < D && eq; ++l) {
-          const double x = T[l], y = L[l];
-          eq = fabs(x - y) <= tol * fmax(fabs(x), fabs(y));   // false for a NaN: never merged
+  for (int64_t b = blockIdx.x; b < nq; b += gridDim.x) {
+    const QuadSrc S = src[b];
+    const int same = qb[b].same;
+    int mine = 0;
+    for (int c = threadIdx.x; c < D * D; c += 256) {
+      uint32_t a = 0;
+      int ncl = 0;
+      int64_t lead[8];
+      int size[8];
+      quad_entries<D>(g, c / D, c % D, same, S, blocks, pidx, [&](int e, int64_t pair, uint32_t, uint32_t) {
+        const double* T = pairs + pair * (D + 1);
+        int k = 0;
+        for (; k < ncl; ++k) {
+          if (size[k] == 4) continue;
+          const double* L = pairs + lead[k] * (D + 1);
+          bool eq = true;
+          for (int l = 0; l < D && eq; ++l) {
+            const double x = T[l], y = L[l];
+            eq = fabs(x - y) <= tol * fmax(fabs(x), fabs(y));   // false for a NaN: never merged
+          }
+          if (eq) break;
         }
-        if (eq) break;
-      }
-      if (k == ncl) {
-        lead[ncl] = pair;
-        size[ncl++] = 0;
-      }
-      ++size[k];
-      a |= (uint32_t)(k + 1) << (4 * e);
-    });
-    assign[b * D * D + c] = a;
-    mine += ncl;
+        if (k == ncl) {
+          lead[ncl] = pair;
+          size[ncl++] = 0;
+        }
+        ++size[k];
+        a |= (uint32_t)(k + 1) << (4 * e);
+      });
+      assign[b * D * D + c] = a;
+      mine += ncl;
+    }
+    int before;
+    const int total = block_scan(mine, before);
+    if (threadIdx.x == 0) count[b] = total;
   }
-  int before;
-  const int total = block_scan(mine, before);
-  if (threadIdx.x == 0) count[b] = total;
 }
 
-// One workgroup per quad block: the steps, 256 candidates at a time.  Each thread
+// One workgroup per quad block in turn: the steps, 256 candidates at a time.  Each thread
 // lists its candidate's quads (their records, and the codes in place), then the
 // workgroup writes the coefficients, one element of a row per thread (a thread per
 // quad took 1.6 ms at 15^3 nodes, strided writes; this way 0.42 ms).
 template <int D>
-__global__ __launch_bounds__(256) void k_quad_write(QuadDims<D> g, const QuadBlk* __restrict__ qb,
+__global__ __launch_bounds__(256) void k_quad_write(QuadDims<D> g, int64_t nq, const QuadBlk* __restrict__ qb,
                                                     const QuadSrc* __restrict__ src,
                                                     const BlockHdr* __restrict__ blocks,
                                                     const int16_t* __restrict__ pidx,
@@ -148,57 +149,58 @@ __global__ __launch_bounds__(256) void k_quad_write(QuadDims<D> g, const QuadBlk
                                                     const uint32_t* __restrict__ assign, char* __restrict__ steps) {
   constexpr uint32_t kNone = 0xffffffffu;
   __shared__ uint32_t rec[256 * 8][4];   // the records of the quads of 256 candidates
-  const int64_t b = blockIdx.x;
-  const QuadSrc S = src[b];
-  const int same = qb[b].same;
-  const uint32_t* A = assign + b * D * D;
-  char* base = steps + qb[b].sbeg * (int64_t)quad_step_bytes<D>();
-  const uint32_t zero = quad_row_off(D, 8, 0);
-  auto slot_T = [&](int quad) { return reinterpret_cast<double*>(base + (int64_t)(quad >> 2) * quad_step_bytes<D>()) + (quad & 3); };
-  auto slot_code = [&](int quad) {
-    return reinterpret_cast<uint16_t*>(base + (int64_t)(quad >> 2) * quad_step_bytes<D>() + D * 32 + (quad & 3) * 16);
-  };
-  int done = 0;   // quads written before this round
-  for (int c0 = 0; c0 < D * D; c0 += 256) {
-    const int c = c0 + (int)threadIdx.x;
-    const uint32_t a = c < D * D ? A[c] : 0;
-    int n = 0;
-    for (int e = 0; e < 8; ++e) n = max(n, (int)((a >> (4 * e)) & 15));
-    int at;
-    const int total = block_scan(n, at);
-    for (int k = 1; k <= n; ++k, ++at) {
-      uint16_t* code = slot_code(done + at);
-      int m = 0;
-      quad_entries<D>(g, c / D, c % D, same, S, blocks, pidx, [&](int e, int64_t pair, uint32_t ox, uint32_t oy) {
-        if ((int)((a >> (4 * e)) & 15) != k) return;
-        rec[at][m] = (uint32_t)pair;
-        code[2 * m] = (uint16_t)ox;
-        code[2 * m + 1] = (uint16_t)oy;
-        ++m;
-      });
-      for (; m < 4; ++m) {
-        rec[at][m] = kNone;
-        code[2 * m] = code[2 * m + 1] = (uint16_t)zero;
+  for (int64_t b = blockIdx.x; b < nq; b += gridDim.x) {
+    const QuadSrc S = src[b];
+    const int same = qb[b].same;
+    const uint32_t* A = assign + b * D * D;
+    char* base = steps + qb[b].sbeg * (int64_t)quad_step_bytes<D>();
+    const uint32_t zero = quad_row_off(D, 8, 0);
+    auto slot_T = [&](int quad) { return reinterpret_cast<double*>(base + (int64_t)(quad >> 2) * quad_step_bytes<D>()) + (quad & 3); };
+    auto slot_code = [&](int quad) {
+      return reinterpret_cast<uint16_t*>(base + (int64_t)(quad >> 2) * quad_step_bytes<D>() + D * 32 + (quad & 3) * 16);
+    };
+    int done = 0;   // quads written before this round
+    for (int c0 = 0; c0 < D * D; c0 += 256) {
+      const int c = c0 + (int)threadIdx.x;
+      const uint32_t a = c < D * D ? A[c] : 0;
+      int n = 0;
+      for (int e = 0; e < 8; ++e) n = max(n, (int)((a >> (4 * e)) & 15));
+      int at;
+      const int total = block_scan(n, at);
+      for (int k = 1; k <= n; ++k, ++at) {
+        uint16_t* code = slot_code(done + at);
+        int m = 0;
+        quad_entries<D>(g, c / D, c % D, same, S, blocks, pidx, [&](int e, int64_t pair, uint32_t ox, uint32_t oy) {
+          if ((int)((a >> (4 * e)) & 15) != k) return;
+          rec[at][m] = (uint32_t)pair;
+          code[2 * m] = (uint16_t)ox;
+          code[2 * m + 1] = (uint16_t)oy;
+          ++m;
+        });
+        for (; m < 4; ++m) {
+          rec[at][m] = kNone;
+          code[2 * m] = code[2 * m + 1] = (uint16_t)zero;
+        }
       }
+      __syncthreads();
+      for (int i = threadIdx.x; i < total * D; i += 256) {
+        const int k = i / D, l = i - k * D;
+        double t = pairs[(int64_t)rec[k][0] * (D + 1) + l];
+        int m = 1;
+        for (; m < 4 && rec[k][m] != kNone; ++m) t += pairs[(int64_t)rec[k][m] * (D + 1) + l];
+        if (m > 1) t = m == 2 ? t * 0.5 : m == 4 ? t * 0.25 : t / 3.0;
+        slot_T(done + k)[4 * l] = t;
+      }
+      done += total;
+      __syncthreads();
     }
-    __syncthreads();
-    for (int i = threadIdx.x; i < total * D; i += 256) {
-      const int k = i / D, l = i - k * D;
-      double t = pairs[(int64_t)rec[k][0] * (D + 1) + l];
-      int m = 1;
-      for (; m < 4 && rec[k][m] != kNone; ++m) t += pairs[(int64_t)rec[k][m] * (D + 1) + l];
-      if (m > 1) t = m == 2 ? t * 0.5 : m == 4 ? t * 0.25 : t / 3.0;
-      slot_T(done + k)[4 * l] = t;
+    // the last step's missing quads: zero rows
+    for (int k = done + threadIdx.x; k < ((done + 3) & ~3); k += 256) {
+      double* T = slot_T(k);
+      uint16_t* code = slot_code(k);
+      for (int l = 0; l < D; ++l) T[4 * l] = 0.0;
+      for (int m = 0; m < 8; ++m) code[m] = (uint16_t)zero;
     }
-    done += total;
-    __syncthreads();
-  }
-  // the last step's missing quads: zero rows
-  for (int k = done + threadIdx.x; k < ((done + 3) & ~3); k += 256) {
-    double* T = slot_T(k);
-    uint16_t* code = slot_code(k);
-    for (int l = 0; l < D; ++l) T[4 * l] = 0.0;
-    for (int m = 0; m < 8; ++m) code[m] = (uint16_t)zero;
   }
 }
 
@@ -306,7 +308,7 @@ static int build_quads_t(dgv_ctx* ctx) {
       free_quads(ctx);
       return rc;
     }
-    hipLaunchKernelGGL(k_quad_assign<D>, dim3((unsigned)nq), dim3(256), 0, st, dims, Q.d_blocks, d_src, pb.d_blocks,
+    hipLaunchKernelGGL(k_quad_assign<D>, dim3(loop_blocks(nq)), dim3(256), 0, st, dims, nq, Q.d_blocks, d_src, pb.d_blocks,
                        d_pidx, pb.d_pairs, kQuadTol, d_assign, d_count);
     e = hipGetLastError();
   }
@@ -330,7 +332,7 @@ static int build_quads_t(dgv_ctx* ctx) {
   if (e == hipSuccess)
     e = hipMemcpyAsync(Q.d_blocks, Q.blocks.data(), sizeof(QuadBlk) * nq, hipMemcpyHostToDevice, st);
   if (e == hipSuccess) {
-    hipLaunchKernelGGL(k_quad_write<D>, dim3((unsigned)nq), dim3(256), 0, st, dims, Q.d_blocks, d_src, pb.d_blocks,
+    hipLaunchKernelGGL(k_quad_write<D>, dim3(loop_blocks(nq)), dim3(256), 0, st, dims, nq, Q.d_blocks, d_src, pb.d_blocks,
                        d_pidx, pb.d_pairs, d_assign, (char*)Q.d_steps);
     e = hipGetLastError();
   }
@@ -560,9 +562,12 @@ int launch_main_quad(dgv_ctx* ctx, const double* d_f, const double* d_g, double*
     sc = 8;
     sp = (uint32_t)g.ncells * 8;
   }
+  // 2^22 items of up to 512 threads a launch (a multiple of the XCDs, so the order holds)
+  constexpr unsigned kItems = 1u << 22;
 #define DGV_QUAD(DD, MM, NW)                                                                            \
-  hipLaunchKernelGGL((k_quad_eval<DD, MM, NW>), dim3(n), dim3(64 * NW), 0, ctx->stream, P.d_qitems,     \
-                     Q.d_blocks, Q.d_steps, F, G, sc, sp, part, g.Mv, g.Mw)
+  for (unsigned i = 0; i < n; i += kItems)                                                              \
+  hipLaunchKernelGGL((k_quad_eval<DD, MM, NW>), dim3(std::min(kItems, n - i)), dim3(64 * NW), 0,        \
+                     ctx->stream, P.d_qitems + i, Q.d_blocks, Q.d_steps, F, G, sc, sp, part, g.Mv, g.Mw)
   if (g.D == 27) {
     if (d_g) DGV_QUAD(27, true, 8);
     else DGV_QUAD(27, false, 4);

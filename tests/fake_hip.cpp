@@ -2,8 +2,9 @@
 // call of it fails: device memory is zeroed host memory, copies are memcpy, kernels are not run.  Linked into a
 // copy of libdgv_amd.so (tests/fake_device.py).  fake_fail_kernel / fake_fail_malloc choose
 // the call that fails; the launches so far, and the widest, can be read back.
+#include <sys/mman.h>
+
 #include <cstdint>
-#include <cstdlib>
 #include <cstring>
 #include <map>
 #include <string>
@@ -12,6 +13,7 @@ typedef int hipError_t;   // hipSuccess 0, hipErrorOutOfMemory 2, hipErrorInvali
 struct dim3_t { uint32_t x, y, z; };
 
 static std::map<const void*, std::string> names;
+static std::map<void*, size_t> sizes;
 static std::string fail_kernel, launched;
 static int64_t fail_malloc_above = INT64_MAX;
 static uint64_t widest = 0;
@@ -47,13 +49,23 @@ hipError_t hipLaunchKernel(const void* f, dim3_t g, dim3_t b, void**, size_t, vo
 }
 hipError_t hipGetLastError() { const hipError_t e = last; last = 0; return e; }
 const char* hipGetErrorString(hipError_t e) { return e ? "fake error" : "no error"; }
+// zeroed pages that take memory only where they are written: a device's memory is larger than the host's
 hipError_t hipMalloc(void** p, size_t n) {
-  if ((int64_t)n > fail_malloc_above || !(*p = calloc(n ? n : 1, 1))) return 2;   // reported here alone
+  if ((int64_t)n > fail_malloc_above) return 2;   // reported here alone
+  *p = mmap(nullptr, n ? n : 1, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
+  if (*p == MAP_FAILED) return 2;
+  sizes[*p] = n ? n : 1;
   return 0;
 }
-hipError_t hipFree(void* p) { free(p); return 0; }
+hipError_t hipFree(void* p) {
+  const auto it = sizes.find(p);
+  if (it == sizes.end()) return p ? 1 : 0;
+  munmap(p, it->second);
+  sizes.erase(it);
+  return 0;
+}
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return hipMalloc(p, n); }
-hipError_t hipHostFree(void* p) { free(p); return 0; }
+hipError_t hipHostFree(void* p) { return hipFree(p); }
 hipError_t hipMemcpy(void* d, const void* s, size_t n, int) { memcpy(d, s, n); return 0; }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, int, void*) { memcpy(d, s, n); return 0; }
 hipError_t hipMemcpy2DAsync(void* d, size_t dp, const void* s, size_t sp, size_t w, size_t h, int, void*) {
