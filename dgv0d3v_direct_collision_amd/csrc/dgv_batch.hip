@@ -1121,7 +1121,14 @@ __global__ __launch_bounds__(64) void k_batch_reduce(int64_t ntask, const int32_
 
 // FP64 on the merged layout: persistent workgroups of four waves, an item = one
 // cell's quad blocks of one run for 32 instances.  The columns of quad_walk are
-// instances: a staged row is 256 contiguous bytes of the packed f.
+// instances: a staged row is 256 contiguous bytes of the packed f.  An item is walked
+// kQuadWalk blocks (up to about 3072 steps) at a time and the walks' sums are added, as the pair-block
+// kernel adds block sums: in one chain of matrix-core sums the error grows with the run.  15^3 nodes, error
+// against extended precision by pairs per run 16 K / 256 K / 1 M: one chain 6e-16 / 3.8e-15 / 2e-14,
+// walks of 4 blocks 5 / 4 / 8e-16, of 16 5 / 6 / 6e-16; the pair-block kernel 7e-16 / 1.1e-15 / 1.6e-15.
+// A walk's start and its sums cost 1 % (256 VDFs on 27^3 nodes 1154 -> 1165 ms).
+template <int D>
+constexpr int kQuadWalk = 3072 / (D * D / 4);
 template <int D>
 __global__ __launch_bounds__(256, 2) void k_quad_batch(const BatchItem* __restrict__ items, const QueueBounds QB,
                                                        const BatchGridDev* __restrict__ grids,
@@ -1153,7 +1160,6 @@ __global__ __launch_bounds__(256, 2) void k_quad_batch(const BatchItem* __restri
     const uint32_t goff = (uint32_t)odd * sp + (uint32_t)col * 8, glast = D % 2 ? (uint32_t)col * 8 : goff;
     const uint32_t loff = (uint32_t)(odd * kQuadRow + col) * 8, llast = D % 2 ? (uint32_t)col * 8 : loff;
     double v[SL][NI];
-    auto header = [&](int i) { return blocks[list[i]]; };
     auto fetch = [&](const QuadBlk& B) {
 #pragma unroll
       for (int k = 0; k < SL; ++k) {
@@ -1179,13 +1185,17 @@ __global__ __launch_bounds__(256, 2) void k_quad_batch(const BatchItem* __restri
     const int n = it.b1 - it.b0;
     auto walk = [&](auto ct) {
       constexpr int CT = decltype(ct)::value;
-      qd4 acc[RT][CT];
+      for (int i0 = 0; i0 < n; i0 += kQuadWalk<D>) {
+        auto header = [&](int i) { return blocks[list[i0 + i]]; };
+        qd4 acc[RT][CT];
 #pragma unroll
-      for (int rt = 0; rt < RT; ++rt)
+        for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-        for (int c = 0; c < CT; ++c) acc[rt][c] = qd4{0.0, 0.0, 0.0, 0.0};
-      quad_walk<D, false, NW, CT>(n, header(0), 0, INT_MAX, G.qsteps, lf, lf, header, fetch, store, acc);
-      quad_flush<D, NW, CT>(lf, acc, ncols, partial + it.prow * D);
+          for (int c = 0; c < CT; ++c) acc[rt][c] = qd4{0.0, 0.0, 0.0, 0.0};
+        quad_walk<D, false, NW, CT>(min(kQuadWalk<D>, n - i0), header(0), 0, INT_MAX, G.qsteps, lf, lf, header, fetch,
+                                    store, acc);
+        quad_flush<D, NW, CT>(lf, acc, ncols, partial + it.prow * D, i0 > 0);
+      }
     };
     if (ncols > 16) walk(std::integral_constant<int, 2>{});
     else walk(std::integral_constant<int, 1>{});

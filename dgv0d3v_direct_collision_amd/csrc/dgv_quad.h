@@ -182,11 +182,12 @@ __device__ __forceinline__ void quad_walk(int n, QuadBlk cur, int s0, int s1, co
   }
 }
 
-// The waves' sums of an item, added in wave order: element (l, col) to
-// out[col * D + l] for col < ncols.  `red` overlays the staged rows (the zero row
-// behind them stays).
+// The waves' sums of a walk, added in wave order: element (l, col) to
+// out[col * D + l] for col < ncols, `more`: on top of what an earlier walk left there.
+// `red` overlays the staged rows (the zero row behind them stays).
 template <int D, int NW, int CT>
-__device__ __forceinline__ void quad_flush(double* red, const qd4 (&acc)[(D + 15) / 16][CT], int ncols, double* out) {
+__device__ __forceinline__ void quad_flush(double* red, const qd4 (&acc)[(D + 15) / 16][CT], int ncols, double* out,
+                                           bool more = false) {
   constexpr int RT = (D + 15) / 16;
   constexpr int S = NW <= 4 ? kQuadCols + 2 : kQuadCols;   // padded where there is room: the column sums read across rows
   static_assert(NW * D * S <= 8 * D * kQuadRow, "the sums fit the staged rows");
@@ -209,7 +210,7 @@ __device__ __forceinline__ void quad_flush(double* red, const qd4 (&acc)[(D + 15
     double s = red[l * S + col];
 #pragma unroll
     for (int w = 1; w < NW; ++w) s += red[(w * D + l) * S + col];
-    out[i] = s;
+    out[i] = more ? out[i] + s : s;
   }
 }
 

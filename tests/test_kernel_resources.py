@@ -25,7 +25,7 @@ def resources(source):
     return out
 
 
-@pytest.mark.parametrize("source,kernel,count", [("dgv_quad.hip", "k_quad_eval", 4)])
+@pytest.mark.parametrize("source,kernel,count", [("dgv_quad.hip", "k_quad_eval", 4), ("dgv_batch.hip", "k_quad_batchI", 2)])
 def test_no_scratch(source, kernel, count):
     try:
         build.hipcc()
