@@ -105,6 +105,7 @@ __device__ __forceinline__ int take_item(int* __restrict__ counter, const QueueB
 // of their partial rows.  A batch keeps the plan over all cells and, on
 // request, a probe plan over a chosen set of cells.
 struct BatchPlan {
+  bool ready = false;              // every part is built
   int32_t tile = 0;
   QueueBounds queues{};            // queue q holds items queues.beg[q] .. queues.beg[q + 1] - 1
   std::vector<BatchItem> items;
@@ -1369,6 +1370,7 @@ static void destroy_plan(dgv_batch* b, BatchPlan& P) {
   hipFree(P.d_items); hipFree(P.d_partial); hipFree(P.d_red_rows); hipFree(P.d_red_ptr); hipFree(P.d_red_key);
   P.d_items = nullptr; P.d_partial = nullptr; P.d_red_rows = nullptr; P.d_red_ptr = nullptr; P.d_red_key = nullptr;
   P.items.clear();
+  P.ready = false;
   P.nrows = 0;
   P.nred = 0;
   if (&P == &b->plan && b->graph) { hipGraphExecDestroy(b->graph); b->graph = nullptr; }
@@ -1382,9 +1384,50 @@ static int shares_of_item(const dgv_batch* b, int nvc) {   // shares of an item 
   return b->quad || b->precision == DGV_FP64 ? 1 : chunks_of_item(b) / nvc;
 }
 
+// The run of each of a grid's quad blocks, in their own order, cut at about `tile` pairs
+static std::vector<int32_t> quad_runs(const dgv_ctx* ctx, int32_t tile) {
+  const QuadLayout& L = ctx->quad;
+  const double per_step = (double)ctx->pb.npairs / (double)std::max<int64_t>(L.nsteps, 1);
+  std::vector<int32_t> run(L.blocks.size());
+  double acc = 0;
+  int32_t r = 0;
+  for (size_t k = 0; k < L.blocks.size(); ++k) {
+    run[k] = r;
+    acc += L.blocks[k].nst * per_step;
+    if (acc >= tile) { ++r; acc = 0; }
+  }
+  return run;
+}
+
+// A merged batch's partial rows with such runs
+static int64_t quad_nrows(const dgv_batch* b, int32_t tile, const std::vector<int32_t>* cells) {
+  int64_t rows = 0;
+  for (size_t g = 0; g < b->grids.size(); ++g) {
+    if (b->nin[g] == 0) continue;
+    const std::vector<int32_t> run = quad_runs(b->grids[g], tile);
+    const std::vector<int64_t>& cp = b->cell_ptr[g];
+    const std::vector<int32_t>& bl = b->h_blist[g];
+    int64_t segs = 0;
+    auto add = [&](int64_t c) {
+      for (int64_t k = cp[c]; k < cp[c + 1]; ++k) segs += k + 1 == cp[c + 1] || run[bl[k + 1]] != run[bl[k]];
+    };
+    if (cells) {
+      for (int32_t c : *cells)
+        if (c >= 0 && c < b->grids[g]->g.ncells) add(c);
+    } else {
+      for (int64_t c = 0; c < b->grids[g]->g.ncells; ++c) add(c);
+    }
+    rows += segs * ((b->nin[g] + kQuadCols - 1) / kQuadCols) * kQuadCols;
+  }
+  return rows;
+}
+
 // Pairs per run.  Merged batch: about 2048 steps (2 MB of coefficients, shared
 // through one XCD's 4 MB L2 by the cells running on it), less where a small batch
-// would not give each of the 512 workgroups four items.
+// would not give each of the 512 workgroups four items; but, up to 1 M pairs, as many as
+// keep the partial sums within a quarter of the coefficients' bytes, pair blocks and
+// merged rows, or 1 GB (256 VDFs on 27^3 nodes: 1165 ms and 25 GB with 2048 steps, 1160 ms
+// with 64 K to 256 K pairs, there 4 GB, 1164 with 512 K, 1176 with 1 M).
 // Otherwise: 4096 pairs for each wave of an item, which keeps the runs of the
 // cells on one XCD close enough together to meet in L2 (27^3 nodes, 64 instances
 // INT8_SPLIT: 479 ms with 1 M pairs a run, 375 with 64 K; 256 instances FP32: 1478
@@ -1440,8 +1483,15 @@ static int32_t auto_tile(const dgv_batch* b, const std::vector<int32_t>* cells) 
   }
   const double per_walk = steps / std::max<double>(1, (double)b->grids.size());
   const double runs = std::max(per_walk / 2048.0, 4.0 * 512.0 / std::max(items, 1.0));
-  const double tile = pairs / std::max<double>(1, (double)b->grids.size()) / std::max(runs, 1.0);
-  return (int32_t)std::min(1e9, std::max(256.0, tile));
+  double tile = std::min(1e9, std::max(256.0, pairs / std::max<double>(1, (double)b->grids.size()) / std::max(runs, 1.0)));
+  const int D = b->grids[0]->g.D;
+  const double most = std::max(1e9, (pairs * (D + 1) * 8 + steps * (D * 32 + 64)) / 4);
+  while (tile < (1 << 20)) {   // the rows fall about as the runs grow
+    const double over = (double)quad_nrows(b, (int32_t)tile, cells) * D * 8 / most;
+    if (over <= 1) break;
+    tile = std::min(1048576.0, tile * std::max(1.1, over));
+  }
+  return (int32_t)tile;
 }
 
 // Per cell and grid: blocks whose box contains the cell, cut into segments;
@@ -1472,17 +1522,8 @@ static int build_batch_plan(dgv_batch* b, BatchPlan& P, int32_t tile, const std:
     const std::vector<int64_t>& cp = b->cell_ptr[gi];
     const std::vector<int32_t>& blist = b->h_blist[gi];
     const int nchunk = b->quad ? (b->nin[gi] + kQuadCols - 1) / kQuadCols : b->Bpad[gi] / 64;
-    if (b->quad) {   // the quad blocks' own order
-      const QuadLayout& L = ctx->quad;
-      const double per_step = (double)pb.npairs / (double)std::max<int64_t>(L.nsteps, 1);
-      run_of[gi].assign(L.blocks.size(), 0);
-      double acc = 0;
-      int32_t run = 0;
-      for (size_t k = 0; k < L.blocks.size(); ++k) {
-        run_of[gi][k] = run;
-        acc += L.blocks[k].nst * per_step;
-        if (acc >= tile) { ++run; acc = 0; }
-      }
+    if (b->quad) {
+      run_of[gi] = quad_runs(ctx, tile);
     } else {
       std::vector<int32_t> order(pb.blocks.size());
       std::iota(order.begin(), order.end(), 0);
@@ -1608,7 +1649,7 @@ static int build_batch_plan(dgv_batch* b, BatchPlan& P, int32_t tile, const std:
   if (hipMalloc(&P.d_partial, sizeof(double) * std::max<int64_t>(P.nrows * D, 1)) != hipSuccess) {
     P.d_partial = nullptr;
     (void)hipGetLastError();
-    if (automatic && !b->quad && tile < (1 << 20)) return build_batch_plan(b, P, 1 << 20, cells);   // the fewest rows
+    if (automatic && tile < (1 << 20)) return build_batch_plan(b, P, 1 << 20, cells);   // the fewest rows
   }
   if (!P.d_partial)
     return berr(b, DGV_ERR_NOMEM, "hipMalloc(batch partial sums) failed");
@@ -1618,12 +1659,14 @@ static int build_batch_plan(dgv_batch* b, BatchPlan& P, int32_t tile, const std:
   BHIP(b, hipMemcpy(P.d_red_ptr, rptr.data(), sizeof(int64_t) * rptr.size(), hipMemcpyHostToDevice));
   BHIP(b, hipMalloc(&P.d_red_key, sizeof(int32_t) * std::max<size_t>(key.size(), 1)));
   BHIP(b, hipMemcpy(P.d_red_key, key.data(), sizeof(int32_t) * key.size(), hipMemcpyHostToDevice));
+  P.ready = true;
   return DGV_OK;
 }
 
 static int batch_eval_dev(dgv_batch* b, const BatchPlan& P, const double* d_f, double* d_q, double scale,
                           bool reduce = true) {
   if (int rc = batch_check_grids(b)) return rc;
+  if (!P.ready) return berr(b, DGV_ERR_STATE, "no work plan: the call that last changed it failed");
   const int D = b->grids[0]->g.D;
   const int nitems = (int)P.items.size();
   hipStream_t st = b->stream;

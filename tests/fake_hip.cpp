@@ -1,5 +1,5 @@
 // A stand-in for the HIP runtime, for host-side tests of what the library does when a
-// call of it fails: device memory is zeroed host memory, copies are memcpy, kernels are not run.  Linked into a
+// call of it fails: device memory is zeroed host memory, copies are memcpy, kernels are not run (but one).  Linked into a
 // copy of libdgv_amd.so (tests/fake_device.py).  fake_fail_kernel / fake_fail_malloc choose
 // the call that fails; the launches so far, and the widest, can be read back.
 #include <sys/mman.h>
@@ -15,7 +15,7 @@ struct dim3_t { uint32_t x, y, z; };
 static std::map<const void*, std::string> names;
 static std::map<void*, size_t> sizes;
 static std::string fail_kernel, launched;
-static int64_t fail_malloc_above = INT64_MAX;
+static int64_t fail_malloc_above = INT64_MAX, largest = 0;
 static uint64_t widest = 0;
 static hipError_t last = 0;
 static struct { dim3_t g, b; size_t shm; void* st; } conf;
@@ -23,9 +23,10 @@ static struct { dim3_t g, b; size_t shm; void* st; } conf;
 extern "C" {
 void fake_fail_kernel(const char* part) { fail_kernel = part; }
 void fake_fail_malloc_above(int64_t bytes) { fail_malloc_above = bytes; }
-void fake_reset() { launched.clear(); widest = 0; }
+void fake_reset() { launched.clear(); widest = 0; largest = 0; }
 const char* fake_launched() { return launched.c_str(); }
 uint64_t fake_widest_launch() { return widest; }
+int64_t fake_largest_malloc() { return largest; }
 
 void** __hipRegisterFatBinary(const void*) { static void* h = nullptr; return &h; }
 void __hipUnregisterFatBinary(void**) {}
@@ -38,13 +39,22 @@ hipError_t __hipPopCallConfiguration(dim3_t* g, dim3_t* b, size_t* shm, void** s
   *g = conf.g; *b = conf.b; *shm = conf.shm; *st = conf.st;
   return 0;
 }
-hipError_t hipLaunchKernel(const void* f, dim3_t g, dim3_t b, void**, size_t, void*) {
+// The one kernel whose result sizes what is built: quads per block, a third of its pairs
+struct alignas(16) QuadBlk { int64_t sbeg; int32_t nst; int8_t a[3], b[3]; uint8_t same, pad; int32_t npairs; };
+static void assign(void** arg) {
+  const int64_t nq = *(const int64_t*)arg[1];
+  const QuadBlk* qb = *(const QuadBlk* const*)arg[2];
+  int32_t* count = *(int32_t* const*)arg[9];
+  for (int64_t k = 0; k < nq; ++k) count[k] = qb[k].npairs / 3;
+}
+hipError_t hipLaunchKernel(const void* f, dim3_t g, dim3_t b, void** arg, size_t, void*) {
   const std::string& n = names[f];
   launched += n + "\n";
   const uint64_t items = (uint64_t)g.x * b.x;
   if (items > widest) widest = items;
   if (items >> 32) return last = 9;   // a grid dimension holds fewer than 2^32 work-items
   if (!fail_kernel.empty() && n.find(fail_kernel) != std::string::npos) return last = 9;
+  if (n.find("k_quad_assign") != std::string::npos) assign(arg);
   return 0;
 }
 hipError_t hipGetLastError() { const hipError_t e = last; last = 0; return e; }
@@ -55,6 +65,7 @@ hipError_t hipMalloc(void** p, size_t n) {
   *p = mmap(nullptr, n ? n : 1, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
   if (*p == MAP_FAILED) return 2;
   sizes[*p] = n ? n : 1;
+  if ((int64_t)n > largest) largest = n;
   return 0;
 }
 hipError_t hipFree(void* p) {
