@@ -217,7 +217,8 @@ struct LinearState {
   int64_t* d_beg = nullptr;       // per (row offset, node): its entries in d_desc
   uint2* d_desc = nullptr;        // (pair, byte offset of the partner in d_halo)
   double* d_halo = nullptr;       // fm with a halo of zeros
-  double* d_part = nullptr;       // partial products of eval_linear_dev
+  double* d_part = nullptr;       // partial products of eval_linear_dev, for passes of up to part_vec vectors
+  int part_vec = 0;
   int64_t nitems = 0;
   bool fma_valid = false;
   double* d_vec[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};  // fm, new Maxwellian, Df, scratch, reduction

@@ -499,6 +499,7 @@ void free_linear(dgv_ctx* ctx) {
   hipFree(L.d_part);
   L.d_fma = nullptr; L.d_items = nullptr; L.d_beg = nullptr; L.d_desc = nullptr; L.d_halo = nullptr;
   L.d_part = nullptr;
+  L.part_vec = 0;
   L.nitems = 0;
   L.fma_valid = false;
   L.run_mode = 0;
@@ -692,20 +693,48 @@ int prepare_fma_dev(dgv_ctx* ctx, const double* d_fm) {
   return DGV_OK;
 }
 
+// The buffer of the chunks' sums, for passes of at least kLinVecMin vectors and of all nvec
+// (up to kLinVec, 0.5 GB at 27^3 nodes) where there is memory for them.  It does not grow
+// while the stream is captured: more passes over fmA give the same results to the last bit.
+constexpr int kLinVecMin = 8;
+static int ensure_partials(dgv_ctx* ctx, int nvec) {
+  LinearState& L = ctx->lin;
+  const int want = std::min(std::max(nvec, kLinVecMin), kLinVec);
+  if (L.part_vec >= want) return DGV_OK;
+  if (L.d_part) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return DGV_OK;
+    DGV_HIP(ctx, hipStreamSynchronize(ctx->stream));   // earlier passes are done with it
+  }
+  const int64_t N = ctx->g.N;
+  // the chunks depend on N alone
+  auto alloc = [&](int nv, double** p) {
+    return hipMalloc(p, sizeof(double) * (size_t)std::max<int64_t>((int64_t)lin_plan(N, nv).nchunk * nv * N, 1)) == hipSuccess;
+  };
+  double* p = nullptr;
+  int got = want;
+  if (!alloc(want, &p)) {
+    (void)hipGetLastError();
+    if (L.d_part) return DGV_OK;
+    got = kLinVecMin;
+    if (want == got || !alloc(got, &p)) {
+      (void)hipGetLastError();
+      return set_error(ctx, DGV_ERR_NOMEM, "hipMalloc(partial products) failed");
+    }
+  }
+  hipFree(L.d_part);
+  L.d_part = p;
+  L.part_vec = got;
+  return DGV_OK;
+}
+
 int eval_linear_dev(dgv_ctx* ctx, const double* d_f, int64_t ldf, double* d_fc, int64_t ldq, int nvec) {
   LinearState& L = ctx->lin;
   if (!L.fma_valid) return set_error(ctx, DGV_ERR_STATE, "EvalCollisionLinear: no linearised operator (PrepareFMA)");
   const int64_t N = ctx->g.N;
-  if (!L.d_part) {   // sums of the chunks, for the largest pass
-    int64_t most = 1;
-    for (int nv = 1; nv <= kLinVec; ++nv) most = std::max<int64_t>(most, (int64_t)lin_plan(N, nv).nchunk * nv * N);
-    if (hipMalloc(&L.d_part, sizeof(double) * (size_t)most) != hipSuccess) {
-      L.d_part = nullptr;
-      return set_error(ctx, DGV_ERR_NOMEM, "hipMalloc(partial products) failed");
-    }
-  }
-  for (int v0 = 0; v0 < nvec; v0 += kLinVec) {
-    const int nv = std::min(kLinVec, nvec - v0);
+  if (int rc = ensure_partials(ctx, nvec)) return rc;
+  for (int v0 = 0; v0 < nvec; v0 += L.part_vec) {
+    const int nv = std::min(L.part_vec, nvec - v0);
     const double* f = d_f + v0 * ldf;
     const LinPlan p = lin_plan(N, nv);
     const unsigned nwg = (unsigned)(((int64_t)p.colblocks * p.nchunk + 7) / 8 * 8 * p.vblocks);

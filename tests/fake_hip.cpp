@@ -17,12 +17,14 @@ static std::map<void*, size_t> sizes;
 static std::string fail_kernel, launched;
 static int64_t fail_malloc_above = INT64_MAX, largest = 0;
 static uint64_t widest = 0;
+static int capturing = 0;
 static hipError_t last = 0;
 static struct { dim3_t g, b; size_t shm; void* st; } conf;
 
 extern "C" {
 void fake_fail_kernel(const char* part) { fail_kernel = part; }
 void fake_fail_malloc_above(int64_t bytes) { fail_malloc_above = bytes; }
+void fake_capturing(int on) { capturing = on; }
 void fake_reset() { launched.clear(); widest = 0; largest = 0; }
 const char* fake_launched() { return launched.c_str(); }
 uint64_t fake_widest_launch() { return widest; }
@@ -92,6 +94,7 @@ hipError_t hipDeviceSynchronize() { return 0; }
 hipError_t hipStreamCreateWithFlags(void** s, unsigned) { *s = nullptr; return 0; }
 hipError_t hipStreamDestroy(void*) { return 0; }
 hipError_t hipStreamSynchronize(void*) { return 0; }
+hipError_t hipStreamIsCapturing(void*, int* s) { *s = capturing; return 0; }
 hipError_t hipStreamBeginCapture(void*, int) { return 0; }
 hipError_t hipStreamEndCapture(void*, void** g) { *g = nullptr; return 0; }
 hipError_t hipEventCreate(void** e) { *e = nullptr; return 0; }
