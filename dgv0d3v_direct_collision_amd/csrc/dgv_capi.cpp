@@ -382,7 +382,11 @@ int dgv_ctx_autotune(dgv_ctx* ctx, int32_t* best_pairs_per_item, double* best_ms
   // f = 1 everywhere is a valid input for timing
   std::vector<double> ones(ctx->g.N, 1.0);
   DGV_HIP(ctx, hipMemcpy(ctx->d_f, ones.data(), sizeof(double) * ones.size(), hipMemcpyHostToDevice));
-  const int32_t cand[] = {512, 1024, 2048, 4096, 8192, 16384};
+  // The merged plan's own rule (0) takes up to 2048 steps an item, about 30 K pairs where boxes
+  // merge well.  Q by pairs per item: 27^3 nodes 8 K 4.79 ms, 16 K 4.66, 32 K and the rule 4.64;
+  // 9^3 nodes 1 K 13.4 us, the rule 12.9.  64 K and 128 K are no better than 32 K on any of six grids.
+  std::vector<int32_t> cand = {512, 1024, 2048, 4096, 8192, 16384};
+  if (ctx->plan.quad) cand.insert(cand.begin(), {0, 1 << 15});
   int32_t best = 0;
   double bms = 1e300;
   for (int32_t t : cand) {
@@ -404,7 +408,7 @@ int dgv_ctx_autotune(dgv_ctx* ctx, int32_t* best_pairs_per_item, double* best_ms
   ctx->tile = best;
   int rc = build_plan(ctx, best);
   if (rc) return rc;
-  if (best_pairs_per_item) *best_pairs_per_item = best;
+  if (best_pairs_per_item) *best_pairs_per_item = best > 0 ? best : ctx->plan.pairs_per_item;
   if (best_ms) *best_ms = bms;
   return DGV_OK;
 }

@@ -3,6 +3,7 @@
 #include <algorithm>
 #include <array>
 #include <climits>
+#include <cmath>
 #include <cstring>
 #include <map>
 #include <vector>
@@ -378,6 +379,9 @@ int build_quad_plan(dgv_ctx* ctx, int32_t ppi) {
   // 94 us with, 102 without; 9^3 nodes (22 K steps) 17.4 with, 15.2 without
   P.transpose = total >= (1 << 16);
   const int64_t target = std::max<int64_t>(1, (int64_t)steps);
+  if (ppi <= 0)   // the pairs that make the same items
+    P.pairs_per_item =
+        (int32_t)std::min(1e9, std::ceil(steps * (double)ctx->pb.npairs / (double)std::max<int64_t>(Q.nsteps, 1)));
   struct Run { int32_t group, b0, b1, s0, s1; int64_t work; };
   std::vector<Run> runs;
   for (size_t gi = 0; gi < Q.groups.size(); ++gi) {

@@ -198,7 +198,8 @@ int dgv_eval_mixed(dgv_ctx* ctx, const double* f, const double* fm, double* fc, 
 int dgv_eval_mixed_dev(dgv_ctx* ctx, const double* d_f, const double* d_fm, double* d_fc, int64_t n);
 /* selects the kernel used by dgv_eval_q* (DGV_KERNEL_*) */
 int dgv_ctx_set_kernel(dgv_ctx* ctx, int kernel);
-/* tunables of the pair-block kernel (pairs per work item); 0 = keep */
+/* tunables of the evaluators (pairs per work item); 0 = keep.  Without a call the size
+ * follows the grid; dgv_ctx_autotune goes back to that where it is the fastest */
 int dgv_ctx_set_tile(dgv_ctx* ctx, int32_t pairs_per_item);
 /* on != 0: every Q of the context (evaluations, spatial operator, RK/AB stages,
  * graph replays) is projected in FP64 onto the complement of the collision

@@ -17,13 +17,14 @@ static std::map<void*, size_t> sizes;
 static std::string fail_kernel, launched;
 static int64_t fail_malloc_above = INT64_MAX, largest = 0;
 static uint64_t widest = 0;
-static int capturing = 0;
+static int capturing = 0, fastest = -1, timed = 0;
 static hipError_t last = 0;
 static struct { dim3_t g, b; size_t shm; void* st; } conf;
 
 extern "C" {
 void fake_fail_kernel(const char* part) { fail_kernel = part; }
 void fake_fail_malloc_above(int64_t bytes) { fail_malloc_above = bytes; }
+void fake_fastest(int k) { fastest = k; timed = 0; }   // the k-th time read from now on is the shortest
 void fake_capturing(int on) { capturing = on; }
 void fake_reset() { launched.clear(); widest = 0; largest = 0; }
 const char* fake_launched() { return launched.c_str(); }
@@ -101,7 +102,7 @@ hipError_t hipEventCreate(void** e) { *e = nullptr; return 0; }
 hipError_t hipEventDestroy(void*) { return 0; }
 hipError_t hipEventRecord(void*, void*) { return 0; }
 hipError_t hipEventSynchronize(void*) { return 0; }
-hipError_t hipEventElapsedTime(float* ms, void*, void*) { *ms = 1.f; return 0; }
+hipError_t hipEventElapsedTime(float* ms, void*, void*) { *ms = timed++ == fastest ? 1.f : 2.f; return 0; }
 hipError_t hipGraphInstantiate(void** x, void*, void*, char*, size_t) { *x = nullptr; return 0; }
 hipError_t hipGraphLaunch(void*, void*) { return 0; }
 hipError_t hipGraphDestroy(void*) { return 0; }
