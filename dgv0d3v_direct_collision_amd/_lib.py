@@ -68,6 +68,7 @@ SIGNATURES = {
     "dgv_agen_pair": (C.c_int, [C.POINTER(GridDesc), _i64, _i64, C.POINTER(AgenParams), _dp, _dp]),
     "dgv_ctx_aarray_size": (C.c_int, [_vp, _lp, _lp]),
     "dgv_ctx_workload": (C.c_int, [_vp, _lp]),
+    "dgv_ctx_merged_rows": (C.c_int, [_vp, _lp]),
     "dgv_ctx_get_aarray_basis": (C.c_int, [_vp, _i32, _dp, _ip, _ip, _i64, _lp, C.c_int]),
     "dgv_ctx_get_aarray_bases": (C.c_int, [_vp, _ip, _i32, _dp, _ip, _ip, _i64, _lp, C.c_int]),
     "dgv_aarray_write_file": (C.c_int, [_vp, C.c_char_p]),
@@ -134,6 +135,7 @@ SIGNATURES = {
     "dgv_batch_get_f_rows_dev": (C.c_int, [_vp, _vp, _i64, _i32, _i32]),
     "dgv_batch_eval_q": (C.c_int, [_vp]),
     "dgv_batch_rk_run": (C.c_int, [_vp, _dbl, _dbl, _i32, _i64, C.c_int]),
+    "dgv_batch_merged": (C.c_int, [_vp, _ip]),
     "dgv_batch_autotune": (C.c_int, [_vp, _ip, _dp]),
     "dgv_batch_set_tile": (C.c_int, [_vp, _i32, _i32]),
     "dgv_batch_set_projection": (C.c_int, [_vp, _i32]),

@@ -300,6 +300,12 @@ class DGV:
         return dict(records=int(out[0]), pairs=int(out[1]), visits=int(out[2]),
                     pair_visits=int(out[3]))
 
+    def merged_rows(self):
+        """dict(rows, pairs, used): the merged layout of the A-array, and whether the selected kernel reads it."""
+        out = np.zeros(3, np.int64)
+        self._chk(self._L.dgv_ctx_merged_rows(self._ctx, out.ctypes.data_as(C.POINTER(C.c_int64))))
+        return dict(rows=int(out[0]), pairs=int(out[1]), used=bool(out[2]))
+
     def get_aarray_basis(self, l: int, index_base: int = 1):
         n = C.c_int64()
         self._chk(self._L.dgv_ctx_get_aarray_basis(self._ctx, l, None, None, None, 0,
@@ -719,6 +725,13 @@ class DGVBatch:
     def eval_q_probe(self):
         """Q of every instance on the probe cells only."""
         self._chk(self._L.dgv_batch_eval_q_probe(self._b))
+
+    @property
+    def merged(self):
+        """Whether the batch is evaluated on its grids' merged layouts."""
+        m = C.c_int32()
+        check(self._L.dgv_batch_merged(self._b, C.byref(m)))
+        return bool(m.value)
 
     def autotune(self):
         best = C.c_int32()

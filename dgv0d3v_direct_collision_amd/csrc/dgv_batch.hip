@@ -2231,6 +2231,12 @@ int dgv_batch_time_eval(dgv_batch* b, int32_t niter, double* ms_per_call, double
   return DGV_OK;
 }
 
+int dgv_batch_merged(const dgv_batch* b, int32_t* merged) {
+  if (!b || !merged) { set_global_error("null argument"); return DGV_ERR_ARG; }
+  *merged = b->quad ? 1 : 0;
+  return DGV_OK;
+}
+
 int dgv_batch_autotune(dgv_batch* b, int32_t* best, double* best_ms) {
   if (!b) { set_global_error("null batch"); return DGV_ERR_ARG; }
   BHIP(b, hipSetDevice(b->grids[0]->device));

@@ -218,6 +218,18 @@ int dgv_ctx_workload(const dgv_ctx* ctx, int64_t out[4]) {
   return workload(c, out);
 }
 
+int dgv_ctx_merged_rows(const dgv_ctx* ctx, int64_t out[3]) {
+  CHECK_CTX(ctx);
+  dgv_ctx* c = const_cast<dgv_ctx*>(ctx);
+  if (!ctx->has_a) return set_error(c, DGV_ERR_STATE, "no A-array set");
+  if (!out) return set_error(c, DGV_ERR_ARG, "null output");
+  const bool kept = ctx->quad.use;
+  out[0] = kept ? ctx->quad.nquads : 0;
+  out[1] = kept ? ctx->pb.npairs : 0;
+  out[2] = ctx->plan.ready && ctx->plan.quad ? 1 : 0;
+  return DGV_OK;
+}
+
 int dgv_ctx_get_aarray_basis(const dgv_ctx* ctx, int32_t l, double* A, int32_t* A_xi, int32_t* A_xi1, int64_t cap,
                              int64_t* nrec, int index_base) {
   CHECK_CTX(ctx);

@@ -105,6 +105,10 @@ int dgv_ctx_aarray_size(const dgv_ctx* ctx, int64_t* nrec, int64_t* per_basis);
  * (the records that pass the bounds tests of collision_mod.f90:196-211, summed
  * over all nodes), out[3] = in-grid pair visits */
 int dgv_ctx_workload(const dgv_ctx* ctx, int64_t out[4]);
+/* the merged layout of the current A-array (one coefficient row for the pairs of a
+ * box of nodes that share it): out[0] = its rows, out[1] = the pairs in them, both 0
+ * where too few merge and none is kept; out[2] = 1 if the selected kernel reads it */
+int dgv_ctx_merged_rows(const dgv_ctx* ctx, int64_t out[3]);
 /* export the records of one canonical basis function (0-based local index l)
  * in the reference's serial order (xi ascending, then xi1); index_base 0/1 */
 int dgv_ctx_get_aarray_basis(const dgv_ctx* ctx, int32_t l, double* A, int32_t* A_xi,
@@ -350,6 +354,7 @@ int dgv_batch_rk_run(dgv_batch* b, double dt, double coef, int32_t rkmts, int64_
                      int use_graph);
 /* times segment sizes 2^14..2^21 pairs and 4 or 8 waves per CU, keeps the
  * fastest (best = its segment size, best_ms = its time per evaluation) */
+int dgv_batch_merged(const dgv_batch* b, int32_t* merged); /* 1: evaluated on the grids' merged layouts */
 int dgv_batch_autotune(dgv_batch* b, int32_t* best, double* best_ms);
 /* segment size (pairs; 0 = default) and persistent-grid size (waves per CU;
  * 0 = keep) of the batched evaluation */
