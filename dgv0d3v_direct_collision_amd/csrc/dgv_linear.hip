@@ -275,13 +275,18 @@ __global__ __launch_bounds__(256, 2) void k_fma_build(const FmaItem* __restrict_
 // 32 columns 256 contiguous bytes).  A workgroup of four waves takes 128 columns, 16
 // VT vectors and a chunk of rows; the chunks' sums are added in order by k_fma_sum.
 // One pass serves up to kLinVec vectors: up to about 50 the reading of fmA bounds it,
-// above them the matrix cores.  27^3 nodes (3.1 GB): 2 vectors 0.55 ms (5.6 TB/s), 32
-// 0.63, 64 0.94, 128 1.78, 256 3.46 ms (57 TFLOP/s); a pass over fmA per 8 vectors
-// on the vector units took 0.62, 3.1, 6.2, 12.4 and 24.7 ms.
+// above them the matrix cores.  27^3 nodes (3.1 GB): 2 vectors 0.53 ms (5.8 TB/s), 32
+// 0.63, 64 0.97, 128 1.86, 256 3.66 ms (54 TFLOP/s); a pass over fmA per 8 vectors
+// on the vector units took 0.61, 3.1, 6.2, 12.3 and 24.7 ms.  (Tiles of 128 vectors, 3.45 ms, leave
+// no registers for the running sums; with one wave per SIMD they take 4.16 ms.)
 // rows of fmA per LDS tile of f (32 and 64 rows for the smaller vector tiles: 1-3 %
 // slower at 27^3 nodes, no faster at 15^3)
 constexpr int kLinRows = 16;
 constexpr int kLinCols = 128;    // columns per workgroup
+// rows whose products are added in one chain before they join the running sum (a chunk in one chain, about
+// 1500 rows at 27^3 nodes, is 1.6 to 2 times as far from extended precision as chunks of 256; chains of
+// 256 / 128 / 64: 9.1 / 5.2 / 5.2e-16 there for one vector, 256 vectors 3.65 / 3.66 / 3.71 ms)
+constexpr int kLinSum = 128;
 constexpr int kLinVec = 256;     // vectors per pass
 
 template <int VT>
@@ -327,12 +332,11 @@ __global__ __launch_bounds__(256, 2) void k_fma_rows(int64_t N, int nv, int colb
       __builtin_memcpy(&bt[b][k], p, 16);
     }
   };
-  ld4 acc[VT][2];
+  ld4 sum[VT][2], acc[VT][2];
 #pragma unroll
-  for (int t = 0; t < VT; ++t) acc[t][0] = acc[t][1] = ld4{0.0, 0.0, 0.0, 0.0};
+  for (int t = 0; t < VT; ++t) sum[t][0] = sum[t][1] = ld4{0.0, 0.0, 0.0, 0.0};
   fload(r0);
   bload(0, r0);
-  int cur = 0;
   auto tile = [&](int b, int64_t r) {   // b: this tile's buffers (constant after unrolling)
     fstore(b);
     __syncthreads();
@@ -352,9 +356,18 @@ __global__ __launch_bounds__(256, 2) void k_fma_rows(int64_t N, int nv, int colb
       }
     }
   };
-  for (int64_t r = r0; r < r1; r += 2 * kLinRows) {
-    tile(0, r);
-    if (r + kLinRows < r1) tile(1, r + kLinRows);
+  for (int64_t rs = r0; rs < r1; rs += kLinSum) {
+#pragma unroll
+    for (int t = 0; t < VT; ++t) acc[t][0] = acc[t][1] = ld4{0.0, 0.0, 0.0, 0.0};
+    for (int64_t r = rs; r < min(r1, rs + kLinSum); r += 2 * kLinRows) {
+      tile(0, r);
+      if (r + kLinRows < r1) tile(1, r + kLinRows);
+    }
+#pragma unroll
+    for (int t = 0; t < VT; ++t) {
+      sum[t][0] += acc[t][0];
+      sum[t][1] += acc[t][1];
+    }
   }
   // output layout: element e of lane jj + 16 kk is row (vector) 4 e + kk, columns col, col + 1
   double* out = part + ck * nv * N;
@@ -364,8 +377,8 @@ __global__ __launch_bounds__(256, 2) void k_fma_rows(int64_t N, int nv, int colb
     for (int e = 0; e < 4; ++e) {
       const int v = v0 + 16 * t + 4 * e + kk;
       if (v >= nv) continue;
-      if (col < N) out[(int64_t)v * N + col] = cl == col ? acc[t][0][e] : acc[t][1][e];
-      if (col + 1 < N) out[(int64_t)v * N + col + 1] = acc[t][1][e];
+      if (col < N) out[(int64_t)v * N + col] = cl == col ? sum[t][0][e] : sum[t][1][e];
+      if (col + 1 < N) out[(int64_t)v * N + col + 1] = sum[t][1][e];
     }
 }
 
@@ -377,16 +390,18 @@ __global__ __launch_bounds__(256) void k_fma_gemv(int64_t N, int64_t chunk, cons
                                                   const double* __restrict__ f, double* __restrict__ part) {
   constexpr int kU = 16;     // row loads in flight per thread
   constexpr int kF = 256;    // rows of f in LDS
+  static_assert(kF % kLinSum == 0 && kLinSum % kU == 0, "chains end where the tiles do");
   __shared__ double fs[kF];
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int64_t r0 = (int64_t)blockIdx.y * chunk, r1 = min(N, r0 + chunk);
   const double* col = fma + (i < N ? i : N - 1);
-  double acc = 0.0;
+  double sum = 0.0;
   for (int64_t b = r0; b < r1; b += kF) {
     const int nr = (int)min((int64_t)kF, r1 - b);
     __syncthreads();
     fs[threadIdx.x] = (int)threadIdx.x < nr ? f[b + threadIdx.x] : 0.0;
     __syncthreads();
+    double acc = 0.0;
     int r = 0;
     for (; r + kU <= nr; r += kU) {
       double m[kU];
@@ -394,10 +409,15 @@ __global__ __launch_bounds__(256) void k_fma_gemv(int64_t N, int64_t chunk, cons
       for (int u = 0; u < kU; ++u) m[u] = col[(b + r + u) * N];
 #pragma unroll
       for (int u = 0; u < kU; ++u) acc = __fma_rn(fs[r + u], m[u], acc);
+      if ((r + kU) % kLinSum == 0) {
+        sum += acc;
+        acc = 0.0;
+      }
     }
     for (; r < nr; ++r) acc = __fma_rn(fs[r], col[(b + r) * N], acc);
+    sum += acc;
   }
-  if (i < N) part[(int64_t)blockIdx.y * N + i] = acc;
+  if (i < N) part[(int64_t)blockIdx.y * N + i] = sum;
 }
 
 __global__ void k_fma_sum(int64_t N, int nchunk, int nv, const double* __restrict__ part, double* __restrict__ fc,
@@ -429,7 +449,7 @@ struct LinPlan {
 };
 static LinPlan lin_plan(int64_t N, int nv) {
   LinPlan p;
-  p.vt = nv == 1 ? 0 : nv <= 16 ? 1 : nv <= 32 ? 2 : nv <= 64 ? 4 : 8;
+  p.vt = nv == 1 ? 0 : nv <= 16 ? 1 : nv <= 32 ? 2 : 4;
   p.vblocks = p.vt == 0 ? 1 : (nv + 16 * p.vt - 1) / (16 * p.vt);
   p.colblocks = (int)((N + kLinCols - 1) / kLinCols);
   const int64_t s = std::max<int64_t>(1, std::min<int64_t>(N / 256, 2048 / p.colblocks));
@@ -748,7 +768,7 @@ int eval_linear_dev(dgv_ctx* ctx, const double* d_f, int64_t ldf, double* d_fc, 
     hipLaunchKernelGGL(k_fma_rows<VT>, dim3(nwg), dim3(256), 0, ctx->stream, N, nv, p.colblocks, p.vblocks, p.chunk, \
                        L.d_fma, f, ldf, L.d_part);                                                              \
     break;
-      DGV_LIN_CASE(1) DGV_LIN_CASE(2) DGV_LIN_CASE(4) DGV_LIN_CASE(8)
+      DGV_LIN_CASE(1) DGV_LIN_CASE(2) DGV_LIN_CASE(4)
 #undef DGV_LIN_CASE
     }
     hipLaunchKernelGGL(k_fma_sum, dim3(stride_blocks(N * nv, 64)), dim3(64), 0, ctx->stream, N, p.nchunk, nv,
