@@ -328,8 +328,13 @@ __global__ __launch_bounds__(256, 2) void k_fma_rows(int64_t N, int nv, int colb
   auto bload = [&](int b, int64_t r) {
 #pragma unroll
     for (int k = 0; k < KS; ++k) {
-      const double* p = fma + min(r + 4 * k + kk, N - 1) * N + cl;   // rows past the chunk meet zeros of f
+      const double* p = fma + min(r + 4 * k + kk, N - 1) * N + cl;   // chunks but the last are whole tiles
       __builtin_memcpy(&bt[b][k], p, 16);
+    }
+    if (r + kLinRows > N) {   // no rows: zeros, as an infinite last row would not vanish against a zero of f
+#pragma unroll
+      for (int k = 0; k < KS; ++k)
+        if (r + 4 * k + kk >= N) bt[b][k] = ld2{0.0, 0.0};
     }
   };
   ld4 sum[VT][2], acc[VT][2];
