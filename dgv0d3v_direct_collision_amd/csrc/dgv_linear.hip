@@ -633,10 +633,13 @@ static int build_fma_plan(dgv_ctx* ctx) {
     for (int t = 0; t < 2; ++t) { hipFree(d_ptr[t]); hipFree(d_list[t]); }
     hipFree(d_cnt);
   };
-  auto nomem = [&]() {
+  auto release = [&]() {   // a call that fails leaves no part of the plan
     drop();
     hipFree(L.d_items); hipFree(L.d_beg); hipFree(L.d_desc); hipFree(L.d_halo);
     L.d_items = nullptr; L.d_beg = nullptr; L.d_desc = nullptr; L.d_halo = nullptr;
+  };
+  auto nomem = [&]() {
+    release();
     return set_error(ctx, DGV_ERR_NOMEM, "hipMalloc(fmA plan) failed");
   };
   bool ok = hipMalloc(&L.d_beg, sizeof(int64_t) * (ne * D + 1)) == hipSuccess &&
@@ -677,12 +680,11 @@ static int build_fma_plan(dgv_ctx* ctx) {
     if (e == hipSuccess) e = lists(L.d_desc);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
   }
-  drop();
   if (e != hipSuccess) {
-    hipFree(L.d_items);
-    L.d_items = nullptr;
+    release();
     return set_error(ctx, DGV_ERR_HIP, std::string("fmA plan: ") + hipGetErrorString(e));
   }
+  drop();
   return DGV_OK;
 }
 

@@ -16,6 +16,7 @@ L = dgv.load()
 L.fake_launched.restype = C.c_char_p
 L.fake_widest_launch.restype = C.c_uint64
 L.fake_largest_malloc.restype = C.c_int64
+L.fake_live_bytes.restype = C.c_int64
 L.fake_fail_malloc_above.argtypes = [C.c_int64]
 def launched(): return L.fake_launched().decode()
 def fail_kernel(part): L.fake_fail_kernel(part.encode())

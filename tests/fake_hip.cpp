@@ -30,6 +30,11 @@ void fake_reset() { launched.clear(); widest = 0; largest = 0; }
 const char* fake_launched() { return launched.c_str(); }
 uint64_t fake_widest_launch() { return widest; }
 int64_t fake_largest_malloc() { return largest; }
+int64_t fake_live_bytes() {
+  int64_t n = 0;
+  for (const auto& s : sizes) n += (int64_t)s.second;
+  return n;
+}
 
 void** __hipRegisterFatBinary(const void*) { static void* h = nullptr; return &h; }
 void __hipUnregisterFatBinary(void**) {}

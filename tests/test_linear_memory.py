@@ -51,3 +51,23 @@ assert passes(200) == (25, 0)
 L.fake_capturing(0)
 assert passes(200)[0] == 1
 """)
+
+
+@pytest.mark.parametrize("how", ['fail_kernel("k_fma_lists")', "L.fake_fail_malloc_above(300_000)"], ids=["launch", "memory"])
+def test_a_plan_that_fails_keeps_nothing(lib, how):
+    """However often PrepareFMA fails on the way to its plan, the next success finds the memory there."""
+    fake_device.run(lib, LINEAR.replace("g.PrepareFMA_DGV(np.ones(n))", "") + f"""
+def prepare():
+    try:
+        g.PrepareFMA_DGV(np.ones(n))
+    except dgv.DGVError:
+        return False
+    return True
+before = L.fake_live_bytes()
+{how}
+assert not prepare() and not prepare()
+assert L.fake_live_bytes() - before < 10 * 8 * n, L.fake_live_bytes() - before   # the regime's vectors at most
+fail_kernel("")
+L.fake_fail_malloc_above(1 << 40)
+assert prepare()
+""")
