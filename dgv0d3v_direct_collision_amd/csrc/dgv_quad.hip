@@ -373,7 +373,9 @@ int build_quad_plan(dgv_ctx* ctx, int32_t ppi) {
     for (int b = G.bbeg; b < G.bend; ++b) n += Q.blocks[b].nst;
     total += (double)n * ((G.ncells + kQuadCols - 1) / kQuadCols);
   }
-  const double steps = ppi > 0 ? (double)ppi * (double)Q.nsteps / (double)std::max<int64_t>(ctx->pb.npairs, 1)
+  // a caller's tile cuts no block finer than about its pair blocks, the least the pair-block
+  // plan takes: 48 of up to 183 steps (27 nodes per cell; those of 8 are never cut)
+  const double steps = ppi > 0 ? std::max(48.0, (double)ppi * (double)Q.nsteps / (double)std::max<int64_t>(ctx->pb.npairs, 1))
                                : std::min(2048.0, std::max(96.0, total / 512));
   // f is transposed first where that pays for its launch: 15^3 nodes (340 K steps)
   // 94 us with, 102 without; 9^3 nodes (22 K steps) 17.4 with, 15.2 without
