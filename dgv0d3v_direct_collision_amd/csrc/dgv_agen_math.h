@@ -29,7 +29,8 @@
 //    face lines, in the same order -- so which crossings bound an arc inside the cell
 //    is found once per piece.  A point of the outer integral then
 //    takes each crossing's angle (one inverse function), its cosine and sine (one of
-//    them the crossing's coordinate over rho, the other a square root), and adds its
+//    them the crossing's coordinate over rho, the other a square root; with up to two
+//    nodes per dimension those of the angle), and adds its
 //    antiderivatives with the sign of its end.
 //  * The basis functions enter at the end: a point adds to the moments
 //      W_kni = int w~^i sin(th) d th int_arcs u~^k v~^n d eps

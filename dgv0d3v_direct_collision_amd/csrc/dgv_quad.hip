@@ -14,7 +14,8 @@ namespace dgv {
 
 // Coefficients of a box's diagonals come from one sphere integral and from
 // products of the same node weights in different orders: at most a dozen
-// roundings apart (2^-49); the merged row is their mean.
+// roundings apart (2^-49); the merged row is their mean, which moves Q by 2e-18 to 3e-17
+// (relative L2, in extended precision, 2- and 3-node grids of up to 960 nodes).
 constexpr double kQuadTol = 3.6e-15;   // 2^-48
 // The merged evaluator is used when it leaves at most this share of the pairs as
 // quads.  One Q at 27^3 nodes: 4.7 ms with the generated A-array (0.29 of the
